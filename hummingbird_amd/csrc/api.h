@@ -21,7 +21,8 @@ inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
 // The dense workspace holds three equally sized (B, H, Lp, D) regions of prepared key-side rows, Lp = L rounded
 // up to kDenseQueryBlock and zero-filled past L: k' and k_diff' (normalised and rotated) and v' (V * mask).
-// Elements are bf16 for HB_BF16 and fp32 for HB_F32. The queries are prepared inside the attention kernel.
+// Elements are bf16 for HB_BF16 and HB_F16; for HB_F32 each value is a pair of halves (4 bytes) in key tiles (fp32.hip).
+// The queries are prepared inside the attention kernel.
 struct DenseLayout {
   int64_t Lp;
   int64_t region_elems;  // B * H * Lp * D
@@ -72,9 +73,9 @@ int launch_dense_attend_16bit(hipStream_t stream, int dtype, const void* q, int6
                               const float* lam, void* out, int B, int L, int Lk, int H, int D, const DenseLayout& lay,
                               const void* workspace);
 int launch_dense_prep_f32(hipStream_t stream, const void* qkv, int64_t rs, int sk, int skd, int sv, const float* kw,
-                          const float* cosT, const float* sinT, int half, const float* vmask, int B, int L, int H, int D,
-                          float eps, const DenseLayout& lay, void* ws);
-int launch_dense_attend_f32(hipStream_t stream, const void* qkv, int64_t rs, int sqd, const float* qw,
+                          const float* cosT, const float* sinT, int half, const float* vmask, int B, int L, int H,
+                          int D, float eps, const DenseLayout& lay, void* ws);
+int launch_dense_attend_f32(hipStream_t stream, const void* qkv, int64_t rs, int sqd, const float* qw, const float* kw,
                             const float* cosT, const float* sinT, int half, float eps, const void* ws, const float* lam,
                             void* out, int B, int L, int Lk, int H, int D, const DenseLayout& lay);
 // Streaming band kernel (band_ring.hip): bf16 or half, D = 64, half % 8 == 0, window <= 128. Arguments are

@@ -1,137 +1,320 @@
-// fp32 inputs: the dense and band differential attentions computed in fp32 throughout.
+// fp32 inputs: the dense and band differential attentions at fp32 accuracy.
 //
 // This is the parity path of the reference's FP32_PARITY preset (sa3jax/dtypes.py:41-49), under which every
 // cast of the XLA chain is a no-op: RMSNorm or DyT, RoPE, the logits, the softmax, P V and the subtraction all
 // stay fp32 (sa3jax/dit.py:45-57, 90-98, 113-119, 146; sa3jax/same_l.py:58-69, 92-100, 134-148, 168-169).
-// Nothing is rounded to bf16, so both products run on the fp32 matrix cores (v_mfma_f32_32x32x2_f32):
+// Norms, RoPE, softmax, row sums, accumulators and the subtraction are fp32. The two products run on the half
+// matrix cores (v_mfma_f32_32x32x16_f16, 16 times the rate of the fp32 ones) on operands split exactly enough not to
+// lose fp32 accuracy: x = hi + lo, hi = half(x), lo = half(x - hi), which leaves at most 2^-23 of x, and three products
+// lo hi + hi lo + hi hi (the lo lo one left out is below 2^-22 of the product at its largest, 2^-25 rms) accumulated in
+// fp32. An fp32 MFMA chain rounds its accumulator once per two dims; these round it three times per sixteen, so the
+// results are nearer to the 64-bit ones than the fp32 chain's were: relative error (2-norm) 6.4e-7 against 9.1e-7 on
+// dense B = 2, L = 1292, 8.4e-7 against 1.3e-6 at L = 2584, 7.0e-7 against 7.9e-7 on the band at w = 17 (24 heads, no
+// lambda), 1.2e-6 against 1.6e-6 at w = 100, 3.9e-7 against 5.4e-7 on the cross-attention. Times, whole calls against
+// the fp32 matrix cores fed through registers: dense (2, 1292, 24 heads) 534 -> 179 us, L = 2584 1565 -> 580, head_dim
+// 128 (2, 1292, 12 heads) 690 -> 180, cross (2, 2584 x 257) 205 -> 78, band S = 16384, w = 128 263 -> 138. Three bf16 terms
+// and six products, which need no scaling, were measured too: 290 us for the first of these. The matrix cores slow down
+// on such operands (about 27 ns per 32x32x16 product and SIMD), so the number of products sets the time.
 //
-//   S^T[key][query] = K Q^T   A = K rows from LDS, B = q held in registers; the reduction over d is split as
-//                             d = (D/2) * (lane / 32) + j, so each lane reads one contiguous half-row of K
-//   P = exp2(S^T c - m)       c = log2(e)/sqrt(D), m the running max of S^T c (online softmax), one FMA per
-//                             score; masked scores are -inf and give exactly 0
-//   O^T[d][query] += V^T P^T  A = V rows from LDS (lane reads V[key][d], consecutive d across lanes), B = P
-//                             straight from the S^T accumulators (their keys are the MFMA's k index)
+//   S^T[key][query] = K Q^T   A = K rows from LDS, B = q in registers
+//   P = exp2(S^T c - m)       m the running max of S^T c (online softmax), one FMA per score; masked scores are -inf
+//                             and give exactly 0
+//   O^T[d][query] += V^T P^T  A = V^T rows from LDS, B = P straight from the S^T accumulators
+//
+// Ranges. A half holds 2^-24 .. 65504, so every operand is scaled by powers of two (exact, undone in c and at the end):
+//   - dim d of the keys by 2^kx[d] and of the queries by 2^qx[d], chosen from the norm parameters alone, which bound a
+//     key's dim after RMSNorm, DyT and RoPE (see scale_table): each key dim fills the half range whatever its gain, and
+//     the query dim takes up the difference, so that the largest product bound over the dims fills it too. What falls
+//     below the range is below 2^-38 of the largest logit the parameters allow.
+//   - V by 2^-e per key tile, e from the tile's largest magnitude, stored with the tile; P by 2^(14 + e - E), E the
+//     largest e so far (O is rescaled when it grows, as for a growing maximum).
 //
 // Work split: a workgroup (4 waves) owns 64 queries of one (batch, head); waves 0-1 run branch 1 on 32 queries
 // each, waves 2-3 branch 2, and the branch-2 waves hand lam * O2 / l2 to the branch-1 waves through LDS. Keys
-// stream through LDS in 64-key tiles (K, K_diff, V). The dense kernel reads the fp32 workspace written by its
-// prep kernel. The band call prepares every key once into a workspace (band_keys_f32: DyT with tanh_f32 below,
-// RoPE) and streams the prepared tiles (band_attend_ws_f32, the next tile fetched into registers while the current
-// one is attended); without a workspace it prepares the K / K_diff tiles
-// of each query block's window itself (band_attend_f32).
+// stream through LDS in 32-key tiles, prepared once per call into the workspace as the bytes the tile has in LDS
+// (K, K_diff and V^T, each a plane of hi and a plane of lo halves: the 4 bytes per value of the fp32 rows) and copied
+// there by DMA. The band call without a workspace prepares the tiles of each query block's window itself.
 #include "api.h"
 #include "attn_tile.h"
 #include "common.h"
+#include "tiles.h"
 
 namespace hb {
-
-template <int D>
-struct F32Tile {
-  static constexpr int KP = D + 4;  // row pitch in floats: conflict-free 16-byte K reads down a column of rows
-  static constexpr int TILE = 64 * KP;
-  static constexpr int LDS_FLOATS = 3 * TILE;  // K, K_diff, V
-  static constexpr int XBUF = 2 * (D / 32) * 16 * 64;  // epilogue hand-over, aliases the tiles
-  static_assert(XBUF <= LDS_FLOATS, "epilogue buffer must fit in the tile area");
-};
 
 __device__ __forceinline__ f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 __device__ __forceinline__ void st4(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
 
-// The next 64-key tile of prepared K, K_diff and V (three workspace regions of D-float rows) held in registers:
-// fetched from global memory while the current tile is attended, stored into the LDS tile rows after the
-// barrier that retires it, so the loads' latency is hidden behind the tile's MFMAs.
+// One key tile, the same bytes in LDS and in the workspace: K, K_diff and V, each a hi and a lo plane of KT x D halves.
+// K planes are [key][d], V planes V^T [d][position] in v_tile_key order; the 16-byte chunks of a row are XOR-swizzled,
+// so that the 16 rows that a pass of the operand reads takes fall in distinct banks.
+// D = 64: two stages (48 KB), three workgroups per CU (124 VGPRs). D = 128: one (48 KB), two workgroups per CU by
+// registers (196 VGPRs).
 template <int D>
-struct TileRegs {
-  f32x4 v[3][D / 16];
-  __device__ __forceinline__ void fetch(const float* const (&src)[3], int k0) {
+struct SplitTile {
+  static constexpr int KT = 32;
+  static constexpr int PLANE = KT * D;       // halves per plane
+  static constexpr int TENSOR = 2 * PLANE;   // hi and lo
+  static constexpr int STAGE = 3 * TENSOR;   // K, K_diff, V
+  static constexpr int STAGES = D == 64 ? 2 : 1;
+  static constexpr int OCC = D == 64 ? 3 : 2;  // workgroups per CU
+  static constexpr int ELEMS = STAGES * STAGE;
+  static constexpr int VN = PLANE / 8 / 256;   // (dim, 8 positions) chunks of V per thread
+  static constexpr int XBUF_BYTES = 2 * (D / 32) * 16 * 64 * 4;  // epilogue hand-over, aliases the stages
+  static_assert(XBUF_BYTES <= 2 * ELEMS, "epilogue buffer must fit in the stages");
+  __device__ static __forceinline__ int k_at(int row, int chunk) { return swz<D>(row, chunk); }
+  __device__ static __forceinline__ int v_at(int d, int chunk) { return d * KT + 8 * (chunk ^ ((d >> 2) & 3)); }
+};
+
+// 8 values as hi + lo halves.
+__device__ __forceinline__ void split8(const float (&x)[8], u32x4& hi, u32x4& lo) {
 #pragma unroll
-    for (int s3 = 0; s3 < 3; ++s3)
-#pragma unroll
-      for (int i = 0; i < D / 16; ++i) {
-        const int ch = threadIdx.x + 256 * i, row = ch / (D / 4), col = (ch % (D / 4)) * 4;
-        v[s3][i] = ld4(src[s3] + static_cast<int64_t>(k0 + row) * D + col);
-      }
+  for (int i = 0; i < 4; ++i) {
+    f16x2 h, l;
+    h[0] = static_cast<_Float16>(x[2 * i]);
+    h[1] = static_cast<_Float16>(x[2 * i + 1]);
+    l[0] = static_cast<_Float16>(__fmaf_rn(static_cast<float>(h[0]), -1.f, x[2 * i]));
+    l[1] = static_cast<_Float16>(__fmaf_rn(static_cast<float>(h[1]), -1.f, x[2 * i + 1]));
+    hi[i] = __builtin_bit_cast(uint32_t, h);
+    lo[i] = __builtin_bit_cast(uint32_t, l);
   }
-  __device__ __forceinline__ void store(float* __restrict__ smem) const {
+}
+
+// Exponent of the leading bit of a bound, within [-100, 100] (zero, subnormal, infinite and NaN bounds included).
+__device__ __forceinline__ int bound_exp(float b) {
+  const int e = static_cast<int>((__float_as_uint(b) >> 23) & 255u) - 127;
+  return e < -100 ? -100 : e > 100 ? 100 : e;
+}
+
+// Powers of two for the operand dims: a key's dim d goes to the matrix cores times 2^k[d], a query's times 2^q[d], and
+// the logit is the product sum times 2^logit. `kb(d)`, `qb(d)`: bounds of dim d before RoPE, which mixes dims d and
+// d +- half (each stays below sqrt(2) times the larger bound). Key: below 2^14.5. Query: eq + ek <= emax, so below
+// 2^13.5.
+struct ScaleTable {
+  int k[128], q[128], logit;
+};
+template <int D, class KBound, class QBound>
+__device__ __forceinline__ void scale_table(ScaleTable& t, int half, KBound kb, QBound qb) {
+  const int lane = threadIdx.x & 63;
+  int ek[D / 64], emax = -1000;
 #pragma unroll
-    for (int s3 = 0; s3 < 3; ++s3)
+  for (int i = 0; i < D / 64; ++i) {
+    const int d = lane + 64 * i, p = d < half ? d + half : d < 2 * half ? d - half : d;
+    ek[i] = bound_exp(fmaxf(kb(d), kb(p)));
+    const int e = bound_exp(fmaxf(qb(d), qb(p))) + ek[i];
+    emax = e > emax ? e : emax;
+  }
 #pragma unroll
-      for (int i = 0; i < D / 16; ++i) {
-        const int ch = threadIdx.x + 256 * i, row = ch / (D / 4), col = (ch % (D / 4)) * 4;
-        st4(smem + s3 * F32Tile<D>::TILE + row * F32Tile<D>::KP + col, v[s3][i]);
+  for (int off = 32; off >= 1; off >>= 1) {
+    const int other = __shfl_xor(emax, off, kWave);
+    emax = other > emax ? other : emax;
+  }
+  if (threadIdx.x < 64) {
+#pragma unroll
+    for (int i = 0; i < D / 64; ++i) {
+      t.k[lane + 64 * i] = 13 - ek[i];
+      t.q[lane + 64 * i] = ek[i] + 12 - emax;
+    }
+    if (lane == 0) t.logit = emax - 25;
+  }
+  __syncthreads();
+}
+// After RMSNorm |x_d| <= sqrt(D) |w_d|; |DyT(x)_d| <= |gamma_d| + |beta_d| (`dyt` = [alpha, gamma, beta]).
+template <int D>
+__device__ __forceinline__ auto rms_bound(const float* __restrict__ w) {
+  return [w](int d) { return sqrtf(static_cast<float>(D)) * fabsf(w[d]); };
+}
+template <int D>
+__device__ __forceinline__ auto dyt_bound(const float* __restrict__ dyt) {
+  return [dyt](int d) { return fabsf(dyt[1 + d]) + fabsf(dyt[1 + D + d]); };
+}
+
+// The 8 dims of group g, scaled and split, into chunk `at` of a hi plane and of the lo plane `plane` halves on.
+__device__ __forceinline__ void st_split(uint16_t* __restrict__ hi, int plane, const float (&x)[8], const int* exps) {
+  float y[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) y[j] = ldexpf(x[j], exps[j]);
+  u32x4 h, l;
+  split8(y, h, l);
+  *reinterpret_cast<u32x4*>(hi) = h;
+  *reinterpret_cast<u32x4*>(hi + plane) = l;
+}
+
+// V of one key tile in registers: a lane per dim, so that a wave's loads are whole rows and the transpose costs no
+// shuffle. The tile's exponent e (V 2^-e fills the half range) travels with the tile: its 8 bits (e + 128) replace the
+// lowest bits of the first 8 lo halves (dim 0, positions 0-7), a change below 2^-21 of those values' share.
+template <int D>
+struct VTile {
+  using T = SplitTile<D>;
+  float v[T::VN][8];
+  // Rows k0 .. of `V`, `pitch` floats apart, times `mask` (null: 1); rows at or past `end` are zeros.
+  __device__ __forceinline__ void fetch(const float* __restrict__ V, int64_t pitch, int k0, int end,
+                                        const float* __restrict__ mask) {
+#pragma unroll
+    for (int i = 0; i < T::VN; ++i) {
+      const int at = threadIdx.x + 256 * i, d = at % D;
+      const int key0 = k0 + v_tile_key(8 * (at / D));  // position p0 + j holds key key0 + 8 (j / 4) + j % 4
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int key = key0 + 8 * (j >> 2) + (j & 3);
+        v[i][j] = key < end ? V[key * pitch + d] : 0.f;
+        if (mask && key < end) v[i][j] *= mask[key];
       }
+    }
+  }
+  __device__ __forceinline__ float wave_amax() const {
+    float a = 0.f;
+#pragma unroll
+    for (int i = 0; i < T::VN; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) a = fmaxf(a, fabsf(v[i][j]));
+    return wave_max(a);
+  }
+  // `amax`: the tile's largest magnitude.
+  __device__ __forceinline__ void store(uint16_t* __restrict__ hi, float amax) const {
+    const int lead = static_cast<int>((__float_as_uint(amax) >> 23) & 255u) - 127;
+    const int e = (lead < -100 ? -100 : lead) - 13;  // -113 .. 115: V 2^-e is below 2^14
+#pragma unroll
+    for (int i = 0; i < T::VN; ++i) {
+      const int at = threadIdx.x + 256 * i;
+      float y[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) y[j] = ldexpf(v[i][j], -e);
+      u32x4 h, l;
+      split8(y, h, l);
+      if (i == 0 && threadIdx.x == 0) {
+        const uint32_t code = e + 128;
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+          l[w] = (l[w] & 0xfffefffeu) | ((code >> (2 * w)) & 1u) | (((code >> (2 * w + 1)) & 1u) << 16);
+      }
+      uint16_t* dst = hi + T::v_at(at % D, at / D);
+      *reinterpret_cast<u32x4*>(dst) = h;
+      *reinterpret_cast<u32x4*>(dst + T::PLANE) = l;
+    }
+  }
+  // The exponent of the tile whose V hi plane is at `hi` in LDS, wave-uniform.
+  __device__ static __forceinline__ int exponent(const uint16_t* __restrict__ hi) {
+    const u32x4 l = lds16(hi + T::PLANE + T::v_at(0, 0));
+    uint32_t code = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const uint32_t x = __builtin_amdgcn_readfirstlane(l[w]);
+      code |= ((x & 1u) | ((x >> 15) & 2u)) << (2 * w);
+    }
+    return static_cast<int>(code) - 128;
   }
 };
 
-// One 64-key tile for one wave: 32 queries (lane % 32) of one branch. `valid(k)` says whether key k of the tile
-// (0..63) takes part for this lane's query.
+// Copies tile t from the workspace into an LDS stage (byte address), 1 KB blocks by DMA, no registers.
+template <int D>
+struct SplitCopy {
+  const uint16_t* src[3];
+  uint32_t voff;
+  __device__ __forceinline__ SplitCopy(const float* ws, int64_t region, int64_t row0) {
+#pragma unroll
+    for (int s = 0; s < 3; ++s) src[s] = reinterpret_cast<const uint16_t*>(ws + s * region + row0 * D);
+    voff = wave_id() * 1024 + (threadIdx.x & 63) * 16;
+  }
+  __device__ __forceinline__ void operator()(int t, uint32_t stage) const {
+    using T = SplitTile<D>;
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+#pragma unroll
+      for (int u = 0; u < 2 * T::TENSOR / 4096; ++u)
+        lds_dma16(src[s] + static_cast<int64_t>(t) * T::TENSOR, voff + 4096 * u,
+                  stage + 2 * s * T::TENSOR + 4096 * u + wave_id() * 1024);
+  }
+};
+
+// Online-softmax state of one wave: 32 queries (lane % 32) of one branch; O holds the sum of P V times
+// 2^(14 - E).
+template <int D>
+struct Branch {
+  f32x16 o[D / 32];
+  float l, m;
+  int E;
+  __device__ __forceinline__ Branch() : l(0.f), m(-INFINITY), E(-1000) {
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt) o[dt] = f32x16{};
+  }
+};
+
+// One key tile for one wave. `sK`, `sV`: the hi planes of the branch's K and of V. `q`: this lane's query, hi and lo,
+// in MFMA B operand order (dims 16 kk + 8 lh .. +8). `masked` (wave-uniform): `valid(k)` says whether key k of the tile
+// takes part for this lane's query. The state is rescaled only when some lane's maximum or the V exponent moves (it
+// would multiply by exactly 1).
 template <int D, class Valid>
-__device__ __forceinline__ void attend_tile_f32(const float* __restrict__ sK, const float* __restrict__ sV,
-                                                const float (&qreg)[D / 2], f32x16 (&o)[D / 32], float& lsum,
-                                                float& m, float c, Valid valid) {
-  constexpr int KP = F32Tile<D>::KP;
+__device__ __forceinline__ void attend_tile_f32(const uint16_t* __restrict__ sK, const uint16_t* __restrict__ sV,
+                                                const u32x4 (&q)[2][D / 16], Branch<D>& b, float c, bool masked,
+                                                Valid valid) {
+  using T = SplitTile<D>;
   const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
-  f32x16 s[2];
+  const int e = VTile<D>::exponent(sV);
+  f32x16 s = f32x16{};
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    s[rt] = f32x16{};
-    const float* krow = sK + (32 * rt + lr) * KP + lh * (D / 2);
+  for (int kk = 0; kk < D / 16; ++kk) {
+    const u32x4 hi = lds16(sK + T::k_at(lr, 2 * kk + lh)), lo = lds16(sK + T::PLANE + T::k_at(lr, 2 * kk + lh));
+    s = mfma_f16_32x32x16(lo, q[0][kk], s);
+    s = mfma_f16_32x32x16(hi, q[1][kk], s);
+    s = mfma_f16_32x32x16(hi, q[0][kk], s);
+  }
+  if (masked) {
 #pragma unroll
-    for (int j4 = 0; j4 < D / 8; ++j4) {
-      const f32x4 kv = ld4(krow + 4 * j4);
+    for (int r = 0; r < 16; ++r) s[r] = valid(acc_key(0, r, lh)) ? s[r] : -INFINITY;
+  }
+  float mx = s[0];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s[rt] = mfma_f32_32x32x2(kv[e], qreg[4 * j4 + e], s[rt]);
+  for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+  mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+  const float mnew = fmaxf(b.m, mx * c);
+  const float muse = mnew == -INFINITY ? 0.f : mnew;  // a query with no valid key so far keeps O = l = 0
+  const int En = e > b.E ? e : b.E;
+  if (En != b.E || __any(mnew != b.m)) {
+    const float alpha = fast_exp2(b.m - muse), beta = ldexpf(alpha, b.E - En);
+    b.l *= alpha;
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt) b.o[dt] *= beta;
+    b.m = mnew;
+    b.E = En;
+  }
+  const float up = ldexpf(1.f, 14 + e - En);  // applied to P itself: in the exponent it would cost 4 bits of argument
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {  // 16 keys: their probabilities, then their products with V
+    float p[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      p[j] = fast_exp2(__fmaf_rn(s[8 * g + j], c, -muse));
+      b.l += p[j];
+      p[j] *= up;
+    }
+    u32x4 ph, pl;
+    split8(p, ph, pl);
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt) {
+      const int at = T::v_at(32 * dt + lr, 2 * g + lh);
+      const u32x4 hi = lds16(sV + at), lo = lds16(sV + T::PLANE + at);
+      b.o[dt] = mfma_f16_32x32x16(lo, ph, b.o[dt]);
+      b.o[dt] = mfma_f16_32x32x16(hi, pl, b.o[dt]);
+      b.o[dt] = mfma_f16_32x32x16(hi, ph, b.o[dt]);
     }
   }
-  float mx = -INFINITY;
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float v = valid(acc_key(rt, r, lh)) ? s[rt][r] : -INFINITY;
-      s[rt][r] = v;
-      mx = fmaxf(mx, v);
-    }
-  mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-  const float mnew = fmaxf(m, mx * c);
-  const float muse = mnew == -INFINITY ? 0.f : mnew;  // a query with no valid key so far keeps O = l = 0
-  const float alpha = fast_exp2(m - muse);
-  m = mnew;
-  lsum *= alpha;
-#pragma unroll
-  for (int dt = 0; dt < D / 32; ++dt) o[dt] *= alpha;
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float p = fast_exp2(__fmaf_rn(s[rt][r], c, -muse));
-      s[rt][r] = p;
-      lsum += p;
-    }
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt)
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const float* vrow = sV + acc_key(rt, j, lh) * KP + lr;
-#pragma unroll
-      for (int dt = 0; dt < D / 32; ++dt) o[dt] = mfma_f32_32x32x2(vrow[32 * dt], s[rt][j], o[dt]);
-    }
 }
 
-// Epilogue shared by both kernels: out[q] = O1 / l1 - lam * O2 / l2 in fp32, each product rounded on its own so
+// Epilogue shared by the kernels: out[q] = O1 / l1 - lam * O2 / l2 in fp32, each product rounded on its own so
 // that identical branches cancel exactly. Must follow a barrier after the last use of the tiles.
 template <int D>
-__device__ __forceinline__ void store_diff_f32(float* __restrict__ smem, const f32x16 (&o)[D / 32], float lsum,
-                                               int br, float lamh, float* __restrict__ orow) {
+__device__ __forceinline__ void store_diff_f32(uint16_t* __restrict__ stages, const Branch<D>& b, int br, float lamh,
+                                               float* __restrict__ orow) {
+  float* smem = reinterpret_cast<float*>(stages);
   const int lane = threadIdx.x & 63, lh = lane >> 5, wave = wave_id();
   const int slot0 = (wave & 1) * (D / 32) * 16;
-  const float inv = __frcp_rn(lsum + __shfl_xor(lsum, 32, kWave));
+  const float inv = ldexpf(__frcp_rn(b.l + __shfl_xor(b.l, 32, kWave)), b.E - 14);
   if (br == 1) {
     const float i1 = __fmul_rn(lamh, inv);
 #pragma unroll
     for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) smem[(slot0 + dt * 16 + r) * 64 + lane] = __fmul_rn(o[dt][r], i1);
+      for (int r = 0; r < 16; ++r) smem[(slot0 + dt * 16 + r) * 64 + lane] = __fmul_rn(b.o[dt][r], i1);
   }
   __syncthreads();
   if (br == 0 && orow) {
@@ -143,16 +326,143 @@ __device__ __forceinline__ void store_diff_f32(float* __restrict__ smem, const f
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int r = 4 * g + j;
-          v[j] = __fsub_rn(__fmul_rn(o[dt][r], inv), smem[(slot0 + dt * 16 + r) * 64 + lane]);
+          v[j] = __fsub_rn(__fmul_rn(b.o[dt][r], inv), smem[(slot0 + dt * 16 + r) * 64 + lane]);
         }
         st4(orow + 32 * dt + 8 * g + 4 * lh, v);
       }
   }
 }
 
-// RMSNorm (dit.py:45-57) and rotate-half RoPE (dit.py:90-98) of k and k_diff and V * mask for 64 tokens of one
-// head, all in fp32, into the workspace regions k', k_diff', v'. Thread task = (token, RoPE group pair) as in the
-// bf16 prep: the rotation partner of every dim is in the thread's own registers.
+// The workspace's V^T tiles of the 64 keys from l0, by the whole workgroup: through LDS, so that the stores are whole
+// lines. `ws`: the first of the 64 rows in the V region.
+template <int D>
+__device__ __forceinline__ void store_v_tiles(const float* __restrict__ V, int64_t pitch, int l0, int end,
+                                              const float* __restrict__ mask, float* __restrict__ ws) {
+  using T = SplitTile<D>;
+  constexpr int NT = 64 / T::KT;
+  __shared__ __attribute__((aligned(16))) uint16_t image[NT * T::TENSOR];
+  __shared__ float amax[NT][4];
+  VTile<D> v[NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i) v[i].fetch(V, pitch, l0 + T::KT * i, end, mask);
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    const float a = v[i].wave_amax();
+    if ((threadIdx.x & 63) == 0) amax[i][wave_id()] = a;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+    v[i].store(image + i * T::TENSOR, fmaxf(fmaxf(amax[i][0], amax[i][1]), fmaxf(amax[i][2], amax[i][3])));
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NT * T::TENSOR / 8 / 256; ++i) {
+    const int at = 8 * (threadIdx.x + 256 * i);
+    st16(reinterpret_cast<uint16_t*>(ws) + at, lds16(image + at));
+  }
+}
+
+// Where the hi chunk of row r (0..63) and group g of a 64-row block lies among the block's K tiles.
+template <int D>
+__device__ __forceinline__ int k_block_at(int r, int g) {
+  using T = SplitTile<D>;
+  return r / T::KT * T::TENSOR + T::k_at(r % T::KT, g);
+}
+
+// RMSNorm (dit.py:45-57) and rotate-half RoPE (dit.py:90-98) in fp32 of two tensors (row offsets offA, offB) for the
+// ROWS positions from pos0 (of the batch whose rows start at `xb`): `sink(tensor, row, group, values)` takes each 8-dim
+// group; positions at or past L give zeros. One (row, RoPE group pair) per thread and pass: the rotation partner of
+// every dim is in the thread's own registers; the mean of squares is reduced over the D / 16 lanes of a row.
+template <int D, int ROWS, class Sink>
+__device__ __forceinline__ void rms_rows_f32(const float* __restrict__ xb, int64_t rs, int64_t offA, int64_t offB,
+                                             int pos0, int L, int half, const float* __restrict__ w, float eps,
+                                             const float* __restrict__ cosT, const float* __restrict__ sinT,
+                                             Sink sink) {
+  constexpr int PAIRS = D / 16, TASKS = ROWS * PAIRS / 256;
+  static_assert(ROWS * PAIRS % 256 == 0, "whole passes of the workgroup");
+  const int p = threadIdx.x % PAIRS;
+  int m1, m2;
+  pair_groups(p, half / 8, m1, m2);
+  const bool rot = p < half / 8;
+#pragma unroll
+  for (int i = 0; i < TASKS; ++i) {
+    const int r = (threadIdx.x + 256 * i) / PAIRS, pos = pos0 + r;
+    const bool in = pos < L;
+    const float* row = xb + static_cast<int64_t>(in ? pos : 0) * rs;
+    f32x4 x[2][2][2], cs[2], sn[2];
+#pragma unroll
+    for (int tsr = 0; tsr < 2; ++tsr)
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) {
+        x[tsr][0][hf] = ld4(row + (tsr ? offB : offA) + 8 * m1 + 4 * hf);
+        x[tsr][1][hf] = ld4(row + (tsr ? offB : offA) + 8 * m2 + 4 * hf);
+      }
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      cs[hf] = f32x4{1.f, 1.f, 1.f, 1.f};
+      sn[hf] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (rot) {
+        const int64_t at = static_cast<int64_t>(in ? pos : 0) * half + 8 * m1 + 4 * hf;
+        cs[hf] = ld4(cosT + at);
+        sn[hf] = ld4(sinT + at);
+      }
+    }
+#pragma unroll
+    for (int tsr = 0; tsr < 2; ++tsr) {
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        ss = __fmaf_rn(x[tsr][1][j >> 2][j & 3], x[tsr][1][j >> 2][j & 3],
+                       __fmaf_rn(x[tsr][0][j >> 2][j & 3], x[tsr][0][j >> 2][j & 3], ss));
+#pragma unroll
+      for (int off = 1; off < PAIRS; off <<= 1) ss += __shfl_xor(ss, off, kWave);
+      const float inv = rsqrtf(ss / static_cast<float>(D) + eps);
+      float o1[8], o2[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float y1 = __fmul_rn(__fmul_rn(x[tsr][0][j >> 2][j & 3], inv), w[8 * m1 + j]);
+        const float y2 = __fmul_rn(__fmul_rn(x[tsr][1][j >> 2][j & 3], inv), w[8 * m2 + j]);
+        const float c = cs[j >> 2][j & 3], s = sn[j >> 2][j & 3];
+        const float r1 = rot ? __fadd_rn(__fmul_rn(y1, c), __fmul_rn(-y2, s)) : y1;
+        const float r2 = rot ? __fadd_rn(__fmul_rn(y2, c), __fmul_rn(y1, s)) : y2;
+        o1[j] = in ? r1 : 0.f;
+        o2[j] = in ? r2 : 0.f;
+      }
+      sink(tsr, r, m1, o1);
+      sink(tsr, r, m2, o2);
+    }
+  }
+}
+
+// The split q and q_diff of the workgroup's 64 queries, through LDS in passes of 64 rows (32 at head_dim 128):
+// `rows(r0, sink)` prepares the pass that starts at row r0. Ends with a barrier, the stages free.
+template <int D>
+constexpr int kQueryRows = 4096 / D;
+template <int D, class Rows>
+__device__ __forceinline__ void queries_f32(const ScaleTable& scale, uint16_t* __restrict__ smem,
+                                            u32x4 (&qf)[2][D / 16], Rows rows) {
+  constexpr int ROWS = kQueryRows<D>, PLANE = 4096;
+  static_assert(4 * PLANE <= SplitTile<D>::ELEMS, "q and q_diff of one pass must fit in the stages");
+  const int lane = threadIdx.x & 63, wave = wave_id(), lr = lane & 31, lh = lane >> 5;
+  const int row = (wave & 1) * 32 + lr;
+#pragma unroll
+  for (int r0 = 0; r0 < 64; r0 += ROWS) {
+    rows(r0, [&](int tsr, int r, int g, const float (&x)[8]) {
+      st_split(smem + 2 * tsr * PLANE + swz<D>(r, g), PLANE, x, scale.q + 8 * g);
+    });
+    __syncthreads();
+    if (row / ROWS == r0 / ROWS) {  // wave-uniform
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int kk = 0; kk < D / 16; ++kk)
+          qf[i][kk] = lds16(smem + (2 * (wave >> 1) + i) * PLANE + swz<D>(row % ROWS, 2 * kk + lh));
+    }
+    __syncthreads();
+  }
+}
+
+// k and k_diff after RMSNorm and RoPE and V * mask for 64 tokens of one head into the workspace's tiles.
 template <int D>
 __global__ __launch_bounds__(256) void dense_prep_f32(const float* __restrict__ qkv, int64_t rs, int sk, int skd,
                                                       int sv, const float* __restrict__ kw,
@@ -160,165 +470,85 @@ __global__ __launch_bounds__(256) void dense_prep_f32(const float* __restrict__ 
                                                       const float* __restrict__ sinT,
                                                       int half, const float* __restrict__ vmask, int L, int Lp, int H,
                                                       float eps, int64_t region, float* __restrict__ ws) {
-  constexpr int PAIRS = D / 16;
-  constexpr int TASKS = 64 * PAIRS / 256;
-  constexpr int VCH = 64 * D / 4 / 256;
-  const int tile = blockIdx.x, h = blockIdx.y, b = blockIdx.z, t = threadIdx.x;
-  const int l0 = tile * 64;
-  const int64_t bh = static_cast<int64_t>(b) * H + h;
-  const int64_t HD = static_cast<int64_t>(H) * D;
-  const int h8 = half / 8;
-#pragma unroll
-  for (int i = 0; i < TASKS; ++i) {
-    const int task = t + 256 * i, p = task % PAIRS, l = l0 + task / PAIRS;
-    int m1, m2;
-    pair_groups(p, h8, m1, m2);
-    const bool rot = p < h8, in = l < L;
-    const float* row = qkv + (static_cast<int64_t>(b) * L + (in ? l : 0)) * rs + h * D;
-    float c[8] = {}, s[8] = {};
-    if (rot && in) {
-      const float* cp = cosT + static_cast<int64_t>(l) * half + 8 * m1;
-      const float* sp = sinT + static_cast<int64_t>(l) * half + 8 * m1;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        c[j] = cp[j];
-        s[j] = sp[j];
-      }
+  __shared__ ScaleTable scale;
+  const int l0 = blockIdx.x * 64, h = blockIdx.y, b = blockIdx.z;
+  const int64_t HD = static_cast<int64_t>(H) * D, bh = static_cast<int64_t>(b) * H + h;
+  const float* xb = qkv + static_cast<int64_t>(b) * L * rs + h * D;
+  float* block = ws + (bh * Lp + l0) * D;
+  scale_table<D>(scale, half, rms_bound<D>(kw), [](int) { return 1.f; });  // only the key's part is used here
+  rms_rows_f32<D, 64>(xb, rs, sk * HD, skd * HD, l0, L, half, kw, eps, cosT, sinT,
+                      [&](int tsr, int r, int g, const float (&x)[8]) {
+                        uint16_t* dst = reinterpret_cast<uint16_t*>(block + tsr * region) + k_block_at<D>(r, g);
+                        st_split(dst, SplitTile<D>::PLANE, x, scale.k + 8 * g);
+                      });
+  store_v_tiles<D>(xb + sv * HD, rs, l0, L, vmask ? vmask + static_cast<int64_t>(b) * L : nullptr, block + 2 * region);
+}
+
+// The key tiles [t_lo, t_hi) through the stages: `attend(stage, t)` for each.
+template <int D, class Attend>
+__device__ __forceinline__ void stream_tiles(const SplitCopy<D>& copy, int t_lo, int t_hi,
+                                             uint16_t* __restrict__ smem, Attend attend) {
+  using T = SplitTile<D>;
+  const uint32_t ldsA = lds_addr(smem);
+  if constexpr (T::STAGES == 2) {
+    // The next tile is copied into the other stage while the current one is attended; unrolled over the two stages so
+    // that both have fixed addresses.
+    const uint32_t ldsB = ldsA + 2 * T::STAGE;
+    copy(t_lo, ldsA);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    for (int t = t_lo; t < t_hi; t += 2) {
+      if (t + 1 < t_hi) copy(t + 1, ldsB);
+      attend(smem, t);
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+      if (t + 1 >= t_hi) break;
+      if (t + 2 < t_hi) copy(t + 2, ldsA);
+      attend(smem + T::STAGE, t + 1);
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
     }
-#pragma unroll
-    for (int si = 0; si < 2; ++si) {
-      const int sec = si == 0 ? sk : skd;
-      const float* w = kw;
-      float x1[8] = {}, x2[8] = {};
-      if (in) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          x1[j] = row[sec * HD + 8 * m1 + j];
-          x2[j] = row[sec * HD + 8 * m2 + j];
-        }
-      }
-      float ss = 0.f;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) ss = __fmaf_rn(x2[j], x2[j], __fmaf_rn(x1[j], x1[j], ss));
-#pragma unroll
-      for (int off = 1; off < PAIRS; off <<= 1) ss += __shfl_xor(ss, off, kWave);
-      const float inv = rsqrtf(ss / static_cast<float>(D) + eps);
-      float o1[8], o2[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float y1 = __fmul_rn(__fmul_rn(x1[j], inv), w[8 * m1 + j]);
-        const float y2 = __fmul_rn(__fmul_rn(x2[j], inv), w[8 * m2 + j]);
-        if (rot) {
-          o1[j] = __fadd_rn(__fmul_rn(y1, c[j]), __fmul_rn(-y2, s[j]));
-          o2[j] = __fadd_rn(__fmul_rn(y2, c[j]), __fmul_rn(y1, s[j]));
-        } else {
-          o1[j] = y1;
-          o2[j] = y2;
-        }
-        if (!in) o1[j] = o2[j] = 0.f;
-      }
-      float* dst = ws + si * region + (bh * Lp + l) * D;
-      st4(dst + 8 * m1, f32x4{o1[0], o1[1], o1[2], o1[3]});
-      st4(dst + 8 * m1 + 4, f32x4{o1[4], o1[5], o1[6], o1[7]});
-      st4(dst + 8 * m2, f32x4{o2[0], o2[1], o2[2], o2[3]});
-      st4(dst + 8 * m2 + 4, f32x4{o2[4], o2[5], o2[6], o2[7]});
+  } else {  // the other workgroup on the CU works while this one's copy is under way
+    for (int t = t_lo; t < t_hi; ++t) {
+      copy(t, ldsA);
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+      attend(smem, t);
+      __syncthreads();
     }
-  }
-#pragma unroll
-  for (int i = 0; i < VCH; ++i) {
-    const int ch = t + 256 * i, key = ch / (D / 4), col = (ch % (D / 4)) * 4, l = l0 + key;
-    f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (l < L) {
-      v = ld4(qkv + (static_cast<int64_t>(b) * L + l) * rs + sv * HD + h * D + col);
-      v *= vmask ? vmask[static_cast<int64_t>(b) * L + l] : 1.f;
-    }
-    st4(ws + 2 * region + (bh * Lp + l) * D + col, v);
   }
 }
 
 template <int D>
-__global__ __launch_bounds__(256) void dense_attend_f32(const float* __restrict__ qkv, int64_t rs, int sqd,
-                                                        const float* __restrict__ qw, const float* __restrict__ cosT,
-                                                        const float* __restrict__ sinT, int half, float eps,
-                                                        const float* __restrict__ ws, int64_t region, int B, int L,
-                                                        int Lp, int Lk, int Lkp, int H,
-                                                        const float* __restrict__ lam, float* __restrict__ out) {
-  using T = F32Tile<D>;
-  __shared__ __attribute__((aligned(16))) float smem[T::LDS_FLOATS];
-  const int nqb = Lp / 64;
+__global__ __launch_bounds__(256, SplitTile<D>::OCC) void dense_attend_f32(
+    const float* __restrict__ qkv, int64_t rs, int sqd, const float* __restrict__ qw, const float* __restrict__ kw,
+    const float* __restrict__ cosT, const float* __restrict__ sinT, int half, float eps, const float* __restrict__ ws,
+    int64_t region, int B, int L, int Lk, int Lkp, int H, const float* __restrict__ lam, float* __restrict__ out) {
+  using T = SplitTile<D>;
+  __shared__ __attribute__((aligned(16))) uint16_t smem[T::ELEMS];
+  __shared__ ScaleTable scale;
+  const int nqb = (L + 63) / 64;
   const int tile = xcd_remap(blockIdx.x, B * H * nqb);
   const int qb = tile % nqb, bh = tile / nqb, h = bh % H, b = bh / H;
-  const int lane = threadIdx.x & 63, wave = wave_id(), lr = lane & 31, lh = lane >> 5;
-  const int br = wave >> 1, q0 = qb * 64 + (wave & 1) * 32;
-  const int64_t rowbase = static_cast<int64_t>(bh) * Lkp;
+  const int wave = wave_id(), br = wave >> 1, q = qb * 64 + (wave & 1) * 32 + (threadIdx.x & 31);
+  scale_table<D>(scale, half, rms_bound<D>(kw), rms_bound<D>(qw));
 
-  // RMSNorm (dit.py:45-57) and rotate-half RoPE (dit.py:90-98) of this lane's half row (dims lh D/2 ..) of q
-  // (branch 1, section 0) or q_diff (branch 2, section sqd), from qkv; the RoPE partner (d +- half) of each group
-  // of 4 dims is loaded directly. Rows at or past L give zeros.
-  float qreg[D / 2];
-  {
-    const int q = q0 + lr, qc = q < L ? q : L - 1, h4 = half / 4;
-    const float* row = qkv + (static_cast<int64_t>(b) * L + qc) * rs + static_cast<int64_t>(br ? sqd : 0) * H * D + h * D;
-    float xp[D / 2];
-    float ss = 0.f;
-#pragma unroll
-    for (int j4 = 0; j4 < D / 8; ++j4) {
-      const int g = lh * (D / 8) + j4;
-      const int pg = g < h4 ? g + h4 : g < 2 * h4 ? g - h4 : g;
-      const f32x4 v = ld4(row + 4 * g), p = ld4(row + 4 * pg);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        qreg[4 * j4 + e] = v[e];
-        xp[4 * j4 + e] = p[e];
-        ss = __fmaf_rn(v[e], v[e], ss);
-      }
-    }
-    ss += __shfl_xor(ss, 32, kWave);
-    const float inv = rsqrtf(ss / static_cast<float>(D) + eps);
-#pragma unroll
-    for (int j = 0; j < D / 2; ++j) {
-      const int d = lh * (D / 2) + j;
-      const bool first = d < half, rot = d < 2 * half;
-      const int pd = first ? d + half : rot ? d - half : d;
-      const float y = __fmul_rn(__fmul_rn(qreg[j], inv), qw[d]);
-      const float yp = __fmul_rn(__fmul_rn(xp[j], inv), qw[pd]);
-      float r = y;
-      if (rot) {  // d < half takes -x[d + half], d >= half takes x[d - half]
-        const int64_t t = static_cast<int64_t>(qc) * half + (first ? d : d - half);
-        r = first ? __fadd_rn(__fmul_rn(y, cosT[t]), __fmul_rn(-yp, sinT[t]))
-                  : __fadd_rn(__fmul_rn(y, cosT[t]), __fmul_rn(yp, sinT[t]));
-      }
-      qreg[j] = q < L ? r : 0.f;
-    }
-  }
-  f32x16 o[D / 32];
-#pragma unroll
-  for (int dt = 0; dt < D / 32; ++dt) o[dt] = f32x16{};
-  float lsum = 0.f, m = -INFINITY;
-  const float c = kLog2e / sqrtf(static_cast<float>(D));
-
-  const float* src[3] = {ws + rowbase * D, ws + region + rowbase * D, ws + 2 * region + rowbase * D};
-  const int nkt = (Lk + 63) / 64;
-  // Loaded through registers into one LDS stage per tile: a register prefetch of the next tile (TileRegs, as in the
-  // band kernel) measured 1.6 % slower here, where the 48 extra registers leave the waves less room.
-  for (int t = 0; t < nkt; ++t) {
-    // 3 tensors x 64 rows x D floats; rows past Lk are the zero padding of the workspace (t * 64 + 63 < Lkp)
-#pragma unroll
-    for (int s3 = 0; s3 < 3; ++s3)
-#pragma unroll
-      for (int i = 0; i < D / 16; ++i) {
-        const int ch = threadIdx.x + 256 * i, row = ch / (D / 4), col = (ch % (D / 4)) * 4;
-        st4(smem + s3 * T::TILE + row * T::KP + col, ld4(src[s3] + static_cast<int64_t>(t * 64 + row) * D + col));
-      }
-    __syncthreads();
-    const int k0 = t * 64;
-    attend_tile_f32<D>(smem + br * T::TILE, smem + 2 * T::TILE, qreg, o, lsum, m, c,
-                       [&](int k) { return k0 + k < Lk; });
-    __syncthreads();
-  }
-  const int q = q0 + lr;
+  u32x4 qf[2][D / 16];
+  const float* xb = qkv + static_cast<int64_t>(b) * L * rs + h * D;
+  queries_f32<D>(scale, smem, qf, [&](int r0, auto sink) {
+    rms_rows_f32<D, kQueryRows<D>>(xb, rs, 0, static_cast<int64_t>(sqd) * H * D, qb * 64 + r0, L, half, qw, eps, cosT,
+                                   sinT, sink);
+  });
+  Branch<D> state;
+  const float c = ldexpf(kLog2e / sqrtf(static_cast<float>(D)), scale.logit);
+  // Keys past Lk are zeros in the workspace (Lkp is a multiple of 128).
+  const SplitCopy<D> copy(ws, region, static_cast<int64_t>(bh) * Lkp);
+  stream_tiles<D>(copy, 0, (Lk + T::KT - 1) / T::KT, smem, [&](const uint16_t* s, int t) {
+    attend_tile_f32<D>(s + br * T::TENSOR, s + 2 * T::TENSOR, qf, state, c, (t + 1) * T::KT > Lk,
+                       [&](int k) { return t * T::KT + k < Lk; });
+  });
   float* orow = q < L ? out + (static_cast<int64_t>(b) * L + q) * (static_cast<int64_t>(H) * D) + h * D : nullptr;
-  store_diff_f32<D>(smem, o, lsum, br, lam ? lam[h] : 1.f, orow);
+  store_diff_f32<D>(smem, state, br, lam ? lam[h] : 1.f, orow);
 }
 
 // tanh in fp32. Below 0.625: y + y^3 Q(y^2), Q a degree-5 least-maximum fit of (tanh(y)/y - 1)/y^2 (made for this
@@ -371,18 +601,20 @@ struct DytPair {
   }
 };
 
-// DyT (same_l.py:58-69) and RoPE (same_l.py:92-100) in fp32 of two tensors (sections secA, secB) for the 64
-// positions pos0 .. pos0+63 into rows of pitch P floats (LDS rows by default, or workspace rows); positions
-// outside [0, S) give zero rows. One (row, RoPE group pair) per thread and pass: the rotation partner of every dim is
-// in the thread's own registers, and the pass's 16-byte loads are all issued before its arithmetic. Measured at S = 16384, 8
-// heads of 64: the key kernel 199.6 -> 42.0 us (201 MB at the rate of a large copy) and, with the same rows prepared
-// for the queries, the call 467 -> 263 us, against the library tanhf with the parameters read per element.
-template <int D, int P = F32Tile<D>::KP>
-__device__ __forceinline__ void band_prep_f32(const float* __restrict__ xb, int64_t rs, int64_t offA, int64_t offB,
+// DyT (same_l.py:58-69) and RoPE (same_l.py:92-100) in fp32 of two tensors (row offsets offA, offB) for the ROWS
+// positions from pos0: `sink(tensor, row, group, values)` takes each 8-dim group; positions outside [0, S) give zeros.
+// One (row, RoPE group pair) per thread and pass: the rotation partner of every dim is in the thread's own registers,
+// and the pass's 16-byte loads are all issued before its arithmetic. Measured at S = 16384, 8 heads of 64: the key
+// kernel 199.6 -> 42.0 us (201 MB at the rate of a large copy) against the library tanhf with the parameters read per
+// element.
+template <int D, int ROWS, class Sink>
+__device__ __forceinline__ void band_rows_f32(const float* __restrict__ xb, int64_t rs, int64_t offA, int64_t offB,
                                               int pos0, int S, int half, const DytPair<D>& dp,
                                               const float* __restrict__ cosT, const float* __restrict__ sinT,
-                                              float* __restrict__ dA, float* __restrict__ dB) {
-  constexpr int PAIRS = D / 16, TASKS = 64 * PAIRS / 256;
+                                              Sink sink) {
+  constexpr int PAIRS = D / 16, TASKS = (ROWS * PAIRS + 255) / 256;
+  static_assert(ROWS * PAIRS % 256 == 0 || ROWS * PAIRS < 256, "whole passes of the workgroup, or part of one");
+  if (ROWS * PAIRS < 256 && threadIdx.x >= ROWS * PAIRS) return;
 #pragma unroll
   for (int i = 0; i < TASKS; ++i) {
     const int r = (threadIdx.x + 256 * i) / PAIRS, pos = pos0 + r;
@@ -408,10 +640,9 @@ __device__ __forceinline__ void band_prep_f32(const float* __restrict__ xb, int6
     }
 #pragma unroll
     for (int tsr = 0; tsr < 2; ++tsr) {
-      float* dst = (tsr ? dB : dA) + r * P;
+      float o1[8], o2[8];
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf) {
-        f32x4 o1, o2;
+      for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int j = 4 * hf + e;
@@ -419,157 +650,101 @@ __device__ __forceinline__ void band_prep_f32(const float* __restrict__ xb, int6
           const float y2 = __fadd_rn(__fmul_rn(dp.g2[j], tanh_f32(__fmul_rn(dp.alpha, x[tsr][1][hf][e]))), dp.b2[j]);
           const float r1 = dp.rot ? __fadd_rn(__fmul_rn(y1, cs[hf][e]), __fmul_rn(-y2, sn[hf][e])) : y1;
           const float r2 = dp.rot ? __fadd_rn(__fmul_rn(y2, cs[hf][e]), __fmul_rn(y1, sn[hf][e])) : y2;
-          o1[e] = in ? r1 : 0.f;
-          o2[e] = in ? r2 : 0.f;
+          o1[j] = in ? r1 : 0.f;
+          o2[j] = in ? r2 : 0.f;
         }
-        st4(dst + 8 * dp.m1 + 4 * hf, o1);
-        st4(dst + 8 * dp.m2 + 4 * hf, o2);
-      }
+      sink(tsr, r, dp.m1, o1);
+      sink(tsr, r, dp.m2, o2);
     }
   }
 }
 
-template <int D>
-__global__ __launch_bounds__(256) void band_attend_f32(const float* __restrict__ qkv, int64_t rs, int B, int S, int H,
-                                                       int w, const float* __restrict__ qdyt,
-                                                       const float* __restrict__ kdyt, const float* __restrict__ cosT,
-                                                       const float* __restrict__ sinT, int half,
-                                                       const float* __restrict__ lam, float* __restrict__ out) {
-  using T = F32Tile<D>;
-  __shared__ __attribute__((aligned(16))) float smem[T::LDS_FLOATS];
-  // query-block-major order: the heads of one query block run together and share key rows in L2
-  const int qb = blockIdx.x / (B * H), bh = blockIdx.x % (B * H), h = bh % H, b = bh / H;
-  const int lane = threadIdx.x & 63, wave = wave_id(), lr = lane & 31, lh = lane >> 5;
-  const int br = wave >> 1, q0 = qb * 64, qw0 = q0 + (wave & 1) * 32, q = qw0 + lr;
-  const int64_t HD = static_cast<int64_t>(H) * D;
-  const float* xb = qkv + static_cast<int64_t>(b) * S * rs + h * D;
-  float* sA = smem;
-  float* sB = smem + T::TILE;
-  float* sV = smem + 2 * T::TILE;
-
-  // q and q_diff of the block, then each wave takes its branch's half-rows into registers
-  band_prep_f32<D>(xb, rs, 0, 3 * HD, q0, S, half, DytPair<D>(qdyt, half), cosT, sinT, sA, sB);
-  __syncthreads();
-  float qreg[D / 2];
-  const float* qrow = (br ? sB : sA) + ((wave & 1) * 32 + lr) * T::KP + lh * (D / 2);
-#pragma unroll
-  for (int j4 = 0; j4 < D / 8; ++j4) {
-    const f32x4 v = ld4(qrow + 4 * j4);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) qreg[4 * j4 + e] = v[e];
-  }
-  __syncthreads();
-
-  f32x16 o[D / 32];
-#pragma unroll
-  for (int dt = 0; dt < D / 32; ++dt) o[dt] = f32x16{};
-  float lsum = 0.f, m = -INFINITY;
-  const float c = kLog2e / sqrtf(static_cast<float>(D));
-  const int kbeg = q0 - w > 0 ? q0 - w : 0;
-  const int kend = q0 + 64 + w < S ? q0 + 64 + w : S;
-  const DytPair<D> kp(kdyt, half);
-  for (int k0 = kbeg; k0 < kend; k0 += 64) {
-    band_prep_f32<D>(xb, rs, HD, 4 * HD, k0, S, half, kp, cosT, sinT, sA, sB);
-#pragma unroll
-    for (int i = 0; i < D / 16; ++i) {
-      const int ch = threadIdx.x + 256 * i, row = ch / (D / 4), col = (ch % (D / 4)) * 4, pos = k0 + row;
-      st4(sV + row * T::KP + col, pos < S ? ld4(xb + static_cast<int64_t>(pos) * rs + 2 * HD + col)
-                                          : f32x4{0.f, 0.f, 0.f, 0.f});
-    }
-    __syncthreads();
-    // the tile reaches this wave's band iff k0 <= qw0 + 31 + w and k0 + 63 >= qw0 - w
-    if (k0 <= qw0 + 31 + w && k0 + 63 >= qw0 - w)
-      attend_tile_f32<D>(br ? sB : sA, sV, qreg, o, lsum, m, c, [&](int k) {
-        const int kk = k0 + k, dist = kk - q;
-        return kk < S && dist <= w && -dist <= w;
-      });
-    __syncthreads();
-  }
-  float* orow = q < S ? out + (static_cast<int64_t>(b) * S + q) * HD + h * D : nullptr;
-  store_diff_f32<D>(smem, o, lsum, br, lam ? lam[h] : 1.f, orow);
-}
-
-// The keys of the band prepared once: DyT and RoPE of k and k_diff (the same steps as band_prep_f32 inside
-// band_attend_f32) and V as it is, for 64-key tile blockIdx.x of (batch blockIdx.z, head blockIdx.y), into the
-// fp32 workspace regions k', k_diff', v' (rows of D floats, Sp rows per (batch, head), zeros past S).
+// The keys of the band prepared once: DyT and RoPE of k and k_diff (the same steps as inside band_attend_f32 without
+// a workspace) and V as it is, for 64-key block blockIdx.x of (batch blockIdx.z, head blockIdx.y), into the workspace's
+// tiles (Sp rows per (batch, head), zeros past S).
 template <int D>
 __global__ __launch_bounds__(256) void band_keys_f32(const float* __restrict__ qkv, int64_t rs, int S, int Sp, int H,
                                                      const float* __restrict__ kdyt, const float* __restrict__ cosT,
                                                      const float* __restrict__ sinT, int half, int64_t region,
                                                      float* __restrict__ ws) {
+  __shared__ ScaleTable scale;
   const int t = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   const int64_t HD = static_cast<int64_t>(H) * D, bh = static_cast<int64_t>(b) * H + h;
   const float* xb = qkv + static_cast<int64_t>(b) * S * rs + h * D;
-  float* kA = ws + (bh * Sp + 64 * t) * D;
-  band_prep_f32<D, D>(xb, rs, HD, 4 * HD, 64 * t, S, half, DytPair<D>(kdyt, half), cosT, sinT, kA, kA + region);
-#pragma unroll
-  for (int i = 0; i < D / 16; ++i) {
-    const int ch = threadIdx.x + 256 * i, row = ch / (D / 4), col = (ch % (D / 4)) * 4, pos = 64 * t + row;
-    st4(ws + 2 * region + (bh * Sp + pos) * D + col,
-        pos < S ? ld4(xb + static_cast<int64_t>(pos) * rs + 2 * HD + col) : f32x4{0.f, 0.f, 0.f, 0.f});
-  }
+  float* block = ws + (bh * Sp + 64 * t) * D;
+  scale_table<D>(scale, half, dyt_bound<D>(kdyt), [](int) { return 1.f; });  // only the key's part is used here
+  band_rows_f32<D, 64>(xb, rs, HD, 4 * HD, 64 * t, S, half, DytPair<D>(kdyt, half), cosT, sinT,
+                       [&](int tsr, int r, int g, const float (&x)[8]) {
+                         uint16_t* dst = reinterpret_cast<uint16_t*>(block + tsr * region) + k_block_at<D>(r, g);
+                         st_split(dst, SplitTile<D>::PLANE, x, scale.k + 8 * g);
+                       });
+  store_v_tiles<D>(xb + 2 * HD, rs, 64 * t, S, nullptr, block + 2 * region);
 }
 
-// band_attend_f32 over prepared keys: the 64-aligned key tiles that meet the block's band are loaded from the
-// workspace of band_keys_f32 instead of being prepared per query block.
-template <int D>
-__global__ __launch_bounds__(256) void band_attend_ws_f32(const float* __restrict__ qkv, int64_t rs, int B, int S,
-                                                          int Sp, int H, int w, const float* __restrict__ qdyt,
-                                                          const float* __restrict__ cosT,
-                                                          const float* __restrict__ sinT, int half,
-                                                          const float* __restrict__ ws, int64_t region,
-                                                          const float* __restrict__ lam, float* __restrict__ out) {
-  using T = F32Tile<D>;
-  __shared__ __attribute__((aligned(16))) float smem[T::LDS_FLOATS];
+// WS: the key tiles that meet the block's band come from the workspace of band_keys_f32; otherwise each query block
+// prepares its own from qkv.
+template <int D, bool WS>
+__global__ __launch_bounds__(256, SplitTile<D>::OCC) void band_attend_f32(
+    const float* __restrict__ qkv, int64_t rs, int B, int S, int Sp, int H, int w, const float* __restrict__ qdyt,
+    const float* __restrict__ kdyt, const float* __restrict__ cosT, const float* __restrict__ sinT, int half,
+    const float* __restrict__ ws, int64_t region, const float* __restrict__ lam, float* __restrict__ out) {
+  using T = SplitTile<D>;
+  __shared__ __attribute__((aligned(16))) uint16_t smem[T::ELEMS];
+  __shared__ ScaleTable scale;
   // query-block-major order: the heads of one query block run together and share key rows in L2
   const int qb = blockIdx.x / (B * H), bh = blockIdx.x % (B * H), h = bh % H, b = bh / H;
-  const int lane = threadIdx.x & 63, wave = wave_id(), lr = lane & 31, lh = lane >> 5;
+  const int lane = threadIdx.x & 63, wave = wave_id(), lr = lane & 31;
   const int br = wave >> 1, q0 = qb * 64, qw0 = q0 + (wave & 1) * 32, q = qw0 + lr;
   const int64_t HD = static_cast<int64_t>(H) * D;
   const float* xb = qkv + static_cast<int64_t>(b) * S * rs + h * D;
 
-  band_prep_f32<D>(xb, rs, 0, 3 * HD, q0, S, half, DytPair<D>(qdyt, half), cosT, sinT, smem,
-                   smem + T::TILE);
-  __syncthreads();
-  float qreg[D / 2];
-  const float* qrow = smem + br * T::TILE + ((wave & 1) * 32 + lr) * T::KP + lh * (D / 2);
-#pragma unroll
-  for (int j4 = 0; j4 < D / 8; ++j4) {
-    const f32x4 v = ld4(qrow + 4 * j4);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) qreg[4 * j4 + e] = v[e];
+  scale_table<D>(scale, half, dyt_bound<D>(kdyt), dyt_bound<D>(qdyt));
+  u32x4 qf[2][D / 16];
+  {
+    const DytPair<D> dp(qdyt, half);
+    queries_f32<D>(scale, smem, qf, [&](int r0, auto sink) {
+      band_rows_f32<D, kQueryRows<D>>(xb, rs, 0, 3 * HD, q0 + r0, S, half, dp, cosT, sinT, sink);
+    });
   }
-  __syncthreads();
 
-  f32x16 o[D / 32];
-#pragma unroll
-  for (int dt = 0; dt < D / 32; ++dt) o[dt] = f32x16{};
-  float lsum = 0.f, m = -INFINITY;
-  const float c = kLog2e / sqrtf(static_cast<float>(D));
-  const int64_t rowbase = static_cast<int64_t>(bh) * Sp;
-  const float* const src[3] = {ws + rowbase * D, ws + region + rowbase * D, ws + 2 * region + rowbase * D};
-  const int kbeg = (q0 - w > 0 ? q0 - w : 0) / 64 * 64;
-  const int kend = q0 + 64 + w < S ? q0 + 64 + w : S;
-  TileRegs<D> nxt;  // every tile's rows k0 .. k0 + 63 lie below Sp: Sp is a multiple of 128 and k0 < S
-  nxt.fetch(src, kbeg);
-  nxt.store(smem);
-  __syncthreads();
-  for (int k0 = kbeg; k0 < kend; k0 += 64) {
-    const bool more = k0 + 64 < kend;
-    if (more) nxt.fetch(src, k0 + 64);
-    if (k0 <= qw0 + 31 + w && k0 + 63 >= qw0 - w)
-      attend_tile_f32<D>(smem + br * T::TILE, smem + 2 * T::TILE, qreg, o, lsum, m, c, [&](int k) {
-        const int kk = k0 + k, dist = kk - q;
-        return kk < S && dist <= w && -dist <= w;
-      });
-    __syncthreads();
-    if (more) {
-      nxt.store(smem);
+  Branch<D> state;
+  const float c = ldexpf(kLog2e / sqrtf(static_cast<float>(D)), scale.logit);
+  const int t_lo = (q0 - w > 0 ? q0 - w : 0) / T::KT;
+  const int t_hi = ((q0 + 64 + w < S ? q0 + 64 + w : S) + T::KT - 1) / T::KT;
+  auto attend = [&](const uint16_t* s, int t) {
+    const int k0 = t * T::KT, k1 = k0 + T::KT - 1;
+    // the tile reaches this wave's band, and lies inside the band of every one of its queries
+    if (k0 > qw0 + 31 + w || k1 < qw0 - w) return;
+    const bool inside = k1 <= qw0 + w && k0 >= qw0 + 31 - w && k1 < S;
+    attend_tile_f32<D>(s + br * T::TENSOR, s + 2 * T::TENSOR, qf, state, c, !inside, [&](int k) {
+      const int kk = k0 + k, dist = kk - q;
+      return kk < S && dist <= w && -dist <= w;
+    });
+  };
+  if constexpr (WS) {  // every tile's rows lie below Sp: Sp is a multiple of 128 and k0 < S
+    const SplitCopy<D> copy(ws, region, static_cast<int64_t>(bh) * Sp);
+    stream_tiles<D>(copy, t_lo, t_hi, smem, attend);
+  } else {
+    __shared__ float amax[4];
+    const DytPair<D> kp(kdyt, half);
+    for (int t = t_lo; t < t_hi; ++t) {
+      VTile<D> v;
+      v.fetch(xb + 2 * HD, rs, t * T::KT, S, nullptr);
+      const float a = v.wave_amax();
+      if (lane == 0) amax[wave] = a;
+      band_rows_f32<D, T::KT>(xb, rs, HD, 4 * HD, t * T::KT, S, half, kp, cosT, sinT,
+                              [&](int tsr, int r, int g, const float (&x)[8]) {
+                                st_split(smem + tsr * T::TENSOR + T::k_at(r, g), T::PLANE, x, scale.k + 8 * g);
+                              });
+      __syncthreads();
+      v.store(smem + 2 * T::TENSOR, fmaxf(fmaxf(amax[0], amax[1]), fmaxf(amax[2], amax[3])));
+      __syncthreads();
+      attend(smem, t);
       __syncthreads();
     }
   }
   float* orow = q < S ? out + (static_cast<int64_t>(b) * S + q) * HD + h * D : nullptr;
-  store_diff_f32<D>(smem, o, lsum, br, lam ? lam[h] : 1.f, orow);
+  store_diff_f32<D>(smem, state, br, lam ? lam[h] : 1.f, orow);
 }
 
 static int launched(const char* what) {
@@ -594,21 +769,17 @@ int launch_dense_prep_f32(hipStream_t stream, const void* qkv, int64_t rs, int s
   return launched("dense_prep_f32");
 }
 
-int launch_dense_attend_f32(hipStream_t stream, const void* qkv, int64_t rs, int sqd, const float* qw,
+int launch_dense_attend_f32(hipStream_t stream, const void* qkv, int64_t rs, int sqd, const float* qw, const float* kw,
                             const float* cosT, const float* sinT, int half, float eps, const void* ws, const float* lam,
                             void* out, int B, int L, int Lk, int H, int D, const DenseLayout& lay) {
-  const int Lp = (L + 127) / 128 * 128;
-  const int nblocks = B * H * (Lp / 64);
+  const int nblocks = B * H * ((L + 63) / 64);
   const float* x = static_cast<const float*>(qkv);
   const float* w = static_cast<const float*>(ws);
   float* o = static_cast<float*>(out);
   const int Lkp = static_cast<int>(lay.Lp);
-  if (D == 64)
-    hipLaunchKernelGGL(dense_attend_f32<64>, dim3(nblocks), dim3(256), 0, stream, x, rs, sqd, qw, cosT, sinT, half, eps,
-                       w, lay.region_elems, B, L, Lp, Lk, Lkp, H, lam, o);
-  else
-    hipLaunchKernelGGL(dense_attend_f32<128>, dim3(nblocks), dim3(256), 0, stream, x, rs, sqd, qw, cosT, sinT, half,
-                       eps, w, lay.region_elems, B, L, Lp, Lk, Lkp, H, lam, o);
+  auto attend = D == 64 ? dense_attend_f32<64> : dense_attend_f32<128>;
+  hipLaunchKernelGGL(attend, dim3(nblocks), dim3(256), 0, stream, x, rs, sqd, qw, kw, cosT, sinT, half, eps, w,
+                     lay.region_elems, B, L, Lk, Lkp, H, lam, o);
   return launched("dense_attend_f32");
 }
 
@@ -622,18 +793,12 @@ int launch_band_f32_ws(hipStream_t stream, const void* qkv, int64_t rs, const fl
   float* o = static_cast<float*>(out);
   const dim3 kgrid(static_cast<unsigned>(Sp / 64), static_cast<unsigned>(H), static_cast<unsigned>(B));
   const int nblocks = B * H * ((S + 63) / 64);
-  if (D == 64) {
-    hipLaunchKernelGGL(band_keys_f32<64>, kgrid, dim3(256), 0, stream, x, rs, S, Sp, H, kdyt, cosT, sinT, half,
-                       lay.region_elems, ws);
-    hipLaunchKernelGGL(band_attend_ws_f32<64>, dim3(nblocks), dim3(256), 0, stream, x, rs, B, S, Sp, H, window, qdyt,
-                       cosT, sinT, half, ws, lay.region_elems, lam, o);
-  } else {
-    hipLaunchKernelGGL(band_keys_f32<128>, kgrid, dim3(256), 0, stream, x, rs, S, Sp, H, kdyt, cosT, sinT, half,
-                       lay.region_elems, ws);
-    hipLaunchKernelGGL(band_attend_ws_f32<128>, dim3(nblocks), dim3(256), 0, stream, x, rs, B, S, Sp, H, window,
-                       qdyt, cosT, sinT, half, ws, lay.region_elems, lam, o);
-  }
-  return launched("band_attend_ws_f32");
+  auto keys = D == 64 ? band_keys_f32<64> : band_keys_f32<128>;
+  auto attend = D == 64 ? band_attend_f32<64, true> : band_attend_f32<128, true>;
+  hipLaunchKernelGGL(keys, kgrid, dim3(256), 0, stream, x, rs, S, Sp, H, kdyt, cosT, sinT, half, lay.region_elems, ws);
+  hipLaunchKernelGGL(attend, dim3(nblocks), dim3(256), 0, stream, x, rs, B, S, Sp, H, window, qdyt, kdyt, cosT, sinT,
+                     half, ws, lay.region_elems, lam, o);
+  return launched("band_attend_f32");
 }
 
 int launch_band_f32(hipStream_t stream, const void* qkv, int64_t rs, const float* qdyt, const float* kdyt,
@@ -642,12 +807,9 @@ int launch_band_f32(hipStream_t stream, const void* qkv, int64_t rs, const float
   const int nblocks = B * H * ((S + 63) / 64);
   const float* x = static_cast<const float*>(qkv);
   float* o = static_cast<float*>(out);
-  if (D == 64)
-    hipLaunchKernelGGL(band_attend_f32<64>, dim3(nblocks), dim3(256), 0, stream, x, rs, B, S, H, window, qdyt, kdyt,
-                       cosT, sinT, half, lam, o);
-  else
-    hipLaunchKernelGGL(band_attend_f32<128>, dim3(nblocks), dim3(256), 0, stream, x, rs, B, S, H, window, qdyt, kdyt,
-                       cosT, sinT, half, lam, o);
+  auto attend = D == 64 ? band_attend_f32<64, false> : band_attend_f32<128, false>;
+  hipLaunchKernelGGL(attend, dim3(nblocks), dim3(256), 0, stream, x, rs, B, S, S, H, window, qdyt, kdyt, cosT, sinT,
+                     half, static_cast<const float*>(nullptr), int64_t(0), lam, o);
   return launched("band_attend_f32");
 }
 
