@@ -10,8 +10,8 @@
 //                (same_l.py:92-100) of k and k_diff in fp32 with one bf16 rounding, and V, written to a
 //                workspace of three (B, H, Sp, D) regions; V is stored transposed per 64-key tile in the order
 //                the PV MFMA consumes it. Keys at or past S are zero.
-//   band_attend  one workgroup of 4 waves per (batch, head, 128-query block): each lane prepares one query row
-//                (DyT, RoPE and the softmax scale, one rounding), then the 64-key tiles of the block's window
+//   band_attend  one workgroup of 4 waves per (batch, head, 128-query block): the lanes prepare the query
+//                rows (query.h: DyT, RoPE and the softmax scale, one rounding), then the 64-key tiles of the block's window
 //                [q0 - w, q0 + 128 + w) stream through LDS (global_load_lds, double-buffered). Each wave skips
 //                the tiles outside its band, runs the tiles inside |k - q| <= w for all of its queries unmasked
 //                and masks the others per score (band_attention.py:108-110); the branches are subtracted in fp32
@@ -21,6 +21,7 @@
 #include "api.h"
 #include "attn_tile.h"
 #include "common.h"
+#include "query.h"
 #include "tiles.h"
 
 namespace hb {
@@ -134,55 +135,6 @@ __global__ __launch_bounds__(256) void band_prep(const uint16_t* __restrict__ qk
   }
 }
 
-// DyT, rotate-half RoPE over the first 2 * 8 H8 dims and the softmax scale of one query row held whole by this
-// lane, in fp32 with one bf16 rounding (the reference fused kernel's cast points, band_attention.py:82-85, 104).
-// `row`: its D elements in qkv; `cs` / `sn`: its (half) columns of the tables; `qdyt` = [alpha, gamma, beta].
-template <class IO, int D, int H8>
-__device__ __forceinline__ void prep_q_row(const uint16_t* __restrict__ row, const float* __restrict__ qdyt,
-                                           const float* __restrict__ cs, const float* __restrict__ sn, float qscale,
-                                           u32x4 (&out)[D / 8]) {
-  u32x4 raw[D / 8];
-#pragma unroll
-  for (int c = 0; c < D / 8; ++c) raw[c] = ld16(row + 8 * c);
-  float cv[8 * H8 + 1], sv[8 * H8 + 1];
-#pragma unroll
-  for (int j4 = 0; j4 < 2 * H8; ++j4) {
-    const f32x4 c4 = *reinterpret_cast<const f32x4*>(cs + 4 * j4);
-    const f32x4 s4 = *reinterpret_cast<const f32x4*>(sn + 4 * j4);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      cv[4 * j4 + e] = c4[e];
-      sv[4 * j4 + e] = s4[e];
-    }
-  }
-  const float a2 = 2.f * kLog2e * qdyt[0];
-  float y[D];
-#pragma unroll
-  for (int c = 0; c < D / 8; ++c) {
-    float x[8];
-    IO::unpack8(raw[c], x);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int d = 8 * c + j;
-      const float g = qdyt[1 + d], be = qdyt[1 + D + d];
-      y[d] = dyt_tanh(x[j], a2, -2.f * g, g + be);
-    }
-  }
-#pragma unroll
-  for (int d = 0; d < 8 * H8; ++d) {
-    const float y1 = y[d], y2 = y[d + 8 * H8];
-    y[d] = __fmaf_rn(y1, cv[d], -(y2 * sv[d]));
-    y[d + 8 * H8] = __fmaf_rn(y2, cv[d], y1 * sv[d]);
-  }
-#pragma unroll
-  for (int c = 0; c < D / 8; ++c) {
-    float o[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = y[8 * c + j] * qscale;
-    out[c] = pack8(o);  // the single bf16 rounding
-  }
-}
-
 // The window's tiles, double-buffered: tile t_lo has already been issued into stage A by the caller. A wave
 // attends a tile only if it meets its band, unmasked when every (key, query) pair of the tile and the wave is in
 // band and the keys exist; `qa` is the wave's first query, `nq` its query count (64 or 32).
@@ -253,54 +205,34 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void band_attend(
   const int qa = q0 + (T::SPLIT ? (wave & 1) * 64 : wave * 32);  // this wave's first query
   const int64_t rowbase = static_cast<int64_t>(bh) * Sp;
 
+  // The block's key window [q0 - w, q0 + 127 + w] clipped to [0, S), in 64-key tiles.
+  const int klo = q0 - w > 0 ? q0 - w : 0;
+  const int khi = q0 + 127 + w < S - 1 ? q0 + 127 + w : S - 1;
+  const int t_lo = klo / 64, t_hi = khi / 64;
+  const TileCopy<D> copy(ws + rowbase * D, ws + region + rowbase * D, ws + 2 * region + rowbase * D);
+  copy(t_lo, lds_addr(smem));
+
+  // The queries of this wave, row qa + 32 ct + lr of column tile ct per lane (query.h). Rows at or past S are
+  // prepared from row S - 1 and never stored.
+  using Query = DytQuery<IO, D>;
+  const Query query{qdyt};
+  QueryRows<Query, D, NB, NCT> rows;
+  const float *cs[NCT], *sn[NCT];
+#pragma unroll
+  for (int ct = 0; ct < NCT; ++ct) {
+    const int qrow = qa + 32 * ct + lr, qc = qrow < S ? qrow : S - 1;
+#pragma unroll
+    for (int bi = 0; bi < NB; ++bi)  // q is section 0 of a qkv row, q_diff section 3
+      rows.row[ct][bi] = qkv + (static_cast<int64_t>(b) * S + qc) * rs +
+                         3 * (br0 + bi) * static_cast<int64_t>(H) * D + h * D;
+    cs[ct] = cosT + static_cast<int64_t>(qc) * half;
+    sn[ct] = sinT + static_cast<int64_t>(qc) * half;
+  }
+  rows.load(query, lh);
   // Launch-uniform softmax plan from the DyT bounds (|DyT(x)_d| <= |gamma_d| + |beta_d|; RoPE is a rotation).
   const SoftmaxPlan plan = softmax_plan(dyt_row_bound<D>(qdyt), dyt_row_bound<D>(kdyt), D);
-
-  // The queries: each lane prepares one whole row (D = 64: row qa + lane of this wave's branch; D = 128: row
-  // qa + lane % 32 of branch lane / 32), then v_permlane32_swap moves the chunks into the MFMA B-operand layout
-  // (as in the dense kernel). Rows at or past S are prepared from row S - 1 and never stored.
   u32x4 qf[NB][NCT][D / 16];
-  {
-    const int64_t HD = static_cast<int64_t>(H) * D;
-    const int qrow = T::SPLIT ? qa + lane : qa + lr;
-    const int sec = 3 * (T::SPLIT ? br0 : lh);  // q is section 0 of a qkv row, q_diff section 3
-    const int qc = qrow < S ? qrow : S - 1;
-    const uint16_t* row = qkv + (static_cast<int64_t>(b) * S + qc) * rs + sec * HD + h * D;
-    const float* cs = cosT + static_cast<int64_t>(qc) * half;
-    const float* sn = sinT + static_cast<int64_t>(qc) * half;
-    u32x4 whole[D / 8];
-    switch (half / 8) {  // half % 8 == 0 and half <= D / 2 are checked on the host
-      case 0: prep_q_row<IO, D, 0>(row, qdyt, cs, sn, plan.qscale, whole); break;
-      case 1: prep_q_row<IO, D, 1>(row, qdyt, cs, sn, plan.qscale, whole); break;
-      case 2: prep_q_row<IO, D, 2>(row, qdyt, cs, sn, plan.qscale, whole); break;
-      case 3: prep_q_row<IO, D, 3>(row, qdyt, cs, sn, plan.qscale, whole); break;
-      default:
-        if constexpr (D == 64) {
-          prep_q_row<IO, D, 4>(row, qdyt, cs, sn, plan.qscale, whole);
-        } else {
-          switch (half / 8) {
-            case 4: prep_q_row<IO, D, 4>(row, qdyt, cs, sn, plan.qscale, whole); break;
-            case 5: prep_q_row<IO, D, 5>(row, qdyt, cs, sn, plan.qscale, whole); break;
-            case 6: prep_q_row<IO, D, 6>(row, qdyt, cs, sn, plan.qscale, whole); break;
-            case 7: prep_q_row<IO, D, 7>(row, qdyt, cs, sn, plan.qscale, whole); break;
-            default: prep_q_row<IO, D, 8>(row, qdyt, cs, sn, plan.qscale, whole); break;
-          }
-        }
-    }
-#pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const auto r = __builtin_amdgcn_permlane32_swap(whole[2 * kk][e], whole[2 * kk + 1][e], false, false);
-        if constexpr (T::SPLIT) {
-          qf[0][0][kk][e] = r[0];
-          qf[0][1][kk][e] = r[1];
-        } else {
-          qf[0][0][kk][e] = r[0];
-          qf[1][0][kk][e] = r[1];
-        }
-      }
-  }
+  rows.prep(query, cs, sn, half, lh, plan.qscale, qf);
 
   f32x16 o[NB][NCT][D / 32];
   float lsum[NB][NCT];
@@ -313,12 +245,6 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void band_attend(
       for (int dt = 0; dt < D / 32; ++dt) o[bi][ct][dt] = f32x16{};
     }
 
-  // The block's key window [q0 - w, q0 + 127 + w] clipped to [0, S), in 64-key tiles.
-  const int klo = q0 - w > 0 ? q0 - w : 0;
-  const int khi = q0 + 127 + w < S - 1 ? q0 + 127 + w : S - 1;
-  const int t_lo = klo / 64, t_hi = khi / 64;
-  const TileCopy<D> copy(ws + rowbase * D, ws + region + rowbase * D, ws + 2 * region + rowbase * D);
-  copy(t_lo, lds_addr(smem));
   const int nq = T::SPLIT ? 64 : 32;
   if (plan.fast)
     band_tiles<D, true>(copy, S, w, t_lo, t_hi, qa, nq, br0, smem, smem + T::STAGE, qf, o, lsum, plan.c);

@@ -6,9 +6,9 @@
 //   dense_prep    one pass over the key side of qkv: per-head RMSNorm (dit.py:45-57) and rotate-half RoPE
 //                 (dit.py:90-98) of k and k_diff, and V * mask (dit.py:174-175), written in bf16 to a workspace;
 //                 V is stored transposed per 64-key tile, in the order the PV MFMA consumes it.
-//   dense_attend  flash-style single pass per (batch, head, 128-query block). Each lane first prepares one
-//                 query row straight from qkv (RMSNorm, RoPE and the softmax scale, the same cast points), so
-//                 q and q_diff never round-trip through HBM. K, K_diff and V tiles of 64 keys are then
+//   dense_attend  flash-style single pass per (batch, head, 128-query block). The lanes first prepare
+//                 the query rows straight from qkv (query.h: RMSNorm, RoPE and the softmax scale, the same cast
+//                 points), so q and q_diff never round-trip through HBM. K, K_diff and V tiles of 64 keys are then
 //                 double-buffered through LDS; S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_32x32x16_bf16 with
 //                 fp32 accumulation; both branches share each V tile; scores never leave registers; the
 //                 subtraction is done in fp32 with one cast (dense_attention.py:94).
@@ -25,6 +25,7 @@
 #include "api.h"
 #include "attn_tile.h"
 #include "common.h"
+#include "query.h"
 #include "tiles.h"
 
 namespace hb {
@@ -247,110 +248,12 @@ __device__ __forceinline__ void dense_attend_loop(
   }
 }
 
-// RMSNorm (dit.py:45-57), rotate-half RoPE over the first 2 * 8 H8 dims (dit.py:90-98) and the softmax scale of
-// one query row, held whole by this lane: `row` points at its D elements in qkv, `cs` / `sn` at its (half)
-// columns of the tables. Cast points are those of the reference fused kernel: the compute dtype IO after the gain
-// and after the rotation, bf16 after the scale. The rotary width is a template parameter so that the partner of every dim is a
-// fixed register. Rows at or past L are prepared from row L - 1 (the caller clamps `row`); their outputs are
-// never stored, and real rows keep the logits within the softmax plan's bound.
-template <class IO, int D, int H8, bool STREAM>
-__device__ __forceinline__ void prep_q_row(const uint16_t* __restrict__ row, const float* __restrict__ qw,
-                                           const float* __restrict__ cs, const float* __restrict__ sn, float eps,
-                                           float qscale, u32x4 (&out)[D / 8]) {
-  u32x4 raw[D / 8];
-#pragma unroll
-  for (int c = 0; c < D / 8; ++c) raw[c] = ld16(row + 8 * c);
-  float cv[8 * H8 + 1], sv[8 * H8 + 1];
-#pragma unroll
-  for (int j4 = 0; j4 < (STREAM ? 0 : 2 * H8); ++j4) {  // the streamed form loads its slices chunk by chunk
-    const f32x4 c4 = *reinterpret_cast<const f32x4*>(cs + 4 * j4);
-    const f32x4 s4 = *reinterpret_cast<const f32x4*>(sn + 4 * j4);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      cv[4 * j4 + e] = c4[e];
-      sv[4 * j4 + e] = s4[e];
-    }
-  }
-  if constexpr (STREAM) {
-    // The same arithmetic chunk pair by chunk pair, so that the whole fp32 row and its tables are never live at
-    // once (head_dim 128 with two waves per SIMD, at most 256 registers each).
-    float ss = 0.f;
-#pragma unroll
-    for (int c = 0; c < D / 8; ++c) {
-      float t[8];
-      IO::unpack8(raw[c], t);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) ss = __fmaf_rn(t[j], t[j], ss);
-    }
-    const float inv = rsqrtf(ss / static_cast<float>(D) + eps);
-    auto normed = [&](int c, float (&y)[8]) {
-      IO::unpack8(raw[c], y);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) y[j] = IO::round((y[j] * inv) * qw[8 * c + j]);
-    };
-    auto emit = [&](int c, const float (&y)[8]) {
-      float o[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] = y[j] * qscale;
-      out[c] = pack8(o);
-    };
-#pragma unroll
-    for (int c = 0; c < H8; ++c) {  // chunk c rotates with chunk c + H8 (dims d and d + half)
-      float y1[8], y2[8], r1[8], r2[8];
-      normed(c, y1);
-      normed(c + H8, y2);
-      const f32x4 c0 = *reinterpret_cast<const f32x4*>(cs + 8 * c), c1 = *reinterpret_cast<const f32x4*>(cs + 8 * c + 4);
-      const f32x4 s0 = *reinterpret_cast<const f32x4*>(sn + 8 * c), s1 = *reinterpret_cast<const f32x4*>(sn + 8 * c + 4);
-      const float cvv[8] = {c0[0], c0[1], c0[2], c0[3], c1[0], c1[1], c1[2], c1[3]};
-      const float svv[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        r1[j] = IO::round(y1[j] * cvv[j] + (-y2[j]) * svv[j]);
-        r2[j] = IO::round(y2[j] * cvv[j] + y1[j] * svv[j]);
-      }
-      emit(c, r1);
-      emit(c + H8, r2);
-    }
-#pragma unroll
-    for (int c = 2 * H8; c < D / 8; ++c) {
-      float y[8];
-      normed(c, y);
-      emit(c, y);
-    }
-    return;
-  }
-  float y[D];
-  float ss = 0.f;
-#pragma unroll
-  for (int c = 0; c < D / 8; ++c) {
-    IO::unpack8(raw[c], *reinterpret_cast<float(*)[8]>(y + 8 * c));
-#pragma unroll
-    for (int j = 0; j < 8; ++j) ss = __fmaf_rn(y[8 * c + j], y[8 * c + j], ss);
-  }
-  const float inv = rsqrtf(ss / static_cast<float>(D) + eps);
-#pragma unroll
-  for (int d = 0; d < D; ++d) y[d] = IO::round((y[d] * inv) * qw[d]);
-#pragma unroll
-  for (int d = 0; d < 8 * H8; ++d) {  // d < half takes -x[d + half], d >= half takes x[d - half]
-    const float y1 = y[d], y2 = y[d + 8 * H8];
-    y[d] = IO::round(y1 * cv[d] + (-y2) * sv[d]);
-    y[d + 8 * H8] = IO::round(y2 * cv[d] + y1 * sv[d]);
-  }
-#pragma unroll
-  for (int c = 0; c < D / 8; ++c) {
-    float o[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = y[8 * c + j] * qscale;
-    out[c] = pack8(o);  // the packing conversion is the final bf16 rounding
-  }
-}
-
 // `qkv` rows hold q at section 0 and q_diff at section `sqd` (units of H * D); the L queries are padded to Lp (a
 // multiple of 128), the Lk keys of the workspace to Lkp. Self-attention has Lk = L. QB: queries per workgroup;
 // the 64-query form runs three workgroups per CU.
-// IO: the element type of qkv and out (bf16 or half); the attention operands are bf16 either way. QB: queries per
-// workgroup; the 64-query form runs three workgroups per CU.
-template <class IO, int D, int QB, int NW>
+// ROPE: false for half = 0 (the cross-attention), whose workgroups are short enough for the rotary forms they would
+// only jump over to show: 29.0 -> 28.2 us at B = 2, L = 2584, 257 keys, 24 heads of 64 (28.8 before query.h).
+template <class IO, int D, int QB, int NW, bool ROPE>
 __global__ __launch_bounds__(64 * NW, D == 64 ? (QB == 64 ? 3 : 2) : 1) void dense_attend(
     const uint16_t* __restrict__ qkv, int64_t rs, int sqd, const float* __restrict__ cosT,
     const float* __restrict__ sinT, int half, float eps, const uint16_t* __restrict__ ws, int64_t region, int B,
@@ -360,7 +263,7 @@ __global__ __launch_bounds__(64 * NW, D == 64 ? (QB == 64 ? 3 : 2) : 1) void den
   constexpr int NB = T::NB, NCT = T::NCT;
   // Stages A and B of the K/V tiles; the epilogue reuses the array as its exchange buffer.
   __shared__ __attribute__((aligned(16))) uint16_t smem[T::SMEM_ELEMS];
-  const int nqb = Lp / QB;
+  const int nqb = (L + QB - 1) / QB;
   const int tile = xcd_remap(blockIdx.x, B * H * nqb);
   const int qb = tile % nqb, bh = tile / nqb, h = bh % H, b = bh / H;
   const int lane = threadIdx.x & 63, wave = wave_id(), lr = lane & 31, lh = lane >> 5;
@@ -368,59 +271,30 @@ __global__ __launch_bounds__(64 * NW, D == 64 ? (QB == 64 ? 3 : 2) : 1) void den
   const int q0 = qb * QB + (T::SPLIT ? (wave % (NW / 2)) * 32 * NCT : wave * 32);  // first query of this wave
   const int64_t rowbase = static_cast<int64_t>(bh) * Lkp;
 
-  constexpr bool kStream = D == 128 && NW == 8;  // the query prologue in the register budget of two waves per SIMD
+  const TileCopy<D, NW> copy(ws + rowbase * D, ws + region + rowbase * D, ws + 2 * region + rowbase * D);
+  copy(0, lds_addr(smem));
+
+  // The queries of this wave, row q0 + 32 ct + lr of column tile ct per lane (query.h). Rows at or past L are
+  // prepared from row L - 1: their outputs are never stored, and real rows keep the logits within the plan's bound.
+  using Query = RmsQuery<IO, D>;
+  const Query query{qw, eps};
+  QueryRows<Query, D, NB, NCT> rows;
+  const float *cs[NCT], *sn[NCT];
+#pragma unroll
+  for (int ct = 0; ct < NCT; ++ct) {
+    const int qrow = q0 + 32 * ct + lr, qc = qrow < L ? qrow : L - 1;
+#pragma unroll
+    for (int bi = 0; bi < NB; ++bi)
+      rows.row[ct][bi] = qkv + (static_cast<int64_t>(b) * L + qc) * rs +
+                         (br0 + bi ? sqd : 0) * static_cast<int64_t>(H) * D + h * D;
+    cs[ct] = cosT + static_cast<int64_t>(qc) * half;
+    sn[ct] = sinT + static_cast<int64_t>(qc) * half;
+  }
+  rows.load(query, lh);
   // Launch-uniform choice between the max-free and the running-max softmax (see the file comment).
   const SoftmaxPlan plan = dense_plan<D>(qw, kw);
-
-  // The queries: each lane prepares one whole row from qkv (D = 64: row q0 + lane of this wave's branch, or
-  // q0 + lane % 32 with one column tile; D = 128: row q0 + lane % 32 of branch lane / 32), then v_permlane32_swap
-  // moves the 16-byte chunks into the MFMA B operand layout (lane (lr, lh) holds chunks 2 kk + lh of its row): for
-  // chunk pair (2 kk, 2 kk + 1) the swap gives [lanes 0-31 of chunk 2 kk | lanes 0-31 of chunk 2 kk + 1] and the
-  // same for lanes 32-63. With one column tile both lane halves hold the same rows and the first half suffices.
   u32x4 qf[NB][NCT][D / 16];
-  {
-    const int64_t HD = static_cast<int64_t>(H) * D;
-    const int qrow = T::SPLIT && NCT == 2 ? q0 + lane : q0 + lr;
-    const int sec = (T::SPLIT ? br0 : lh) ? sqd : 0;
-    const int qc = qrow < L ? qrow : L - 1;
-    const uint16_t* row = qkv + (static_cast<int64_t>(b) * L + qc) * rs + sec * HD + h * D;
-    const float* cs = cosT + static_cast<int64_t>(qc) * half;
-    const float* sn = sinT + static_cast<int64_t>(qc) * half;
-    u32x4 whole[D / 8];
-    switch (half / 8) {  // half % 8 == 0 and half <= D / 2 are checked on the host
-      case 0: prep_q_row<IO, D, 0, kStream>(row, qw, cs, sn, eps, plan.qscale, whole); break;
-      case 1: prep_q_row<IO, D, 1, kStream>(row, qw, cs, sn, eps, plan.qscale, whole); break;
-      case 2: prep_q_row<IO, D, 2, kStream>(row, qw, cs, sn, eps, plan.qscale, whole); break;
-      case 3: prep_q_row<IO, D, 3, kStream>(row, qw, cs, sn, eps, plan.qscale, whole); break;
-      default:
-        if constexpr (D == 64) {
-          prep_q_row<IO, D, 4, kStream>(row, qw, cs, sn, eps, plan.qscale, whole);
-        } else {
-          switch (half / 8) {
-            case 4: prep_q_row<IO, D, 4, kStream>(row, qw, cs, sn, eps, plan.qscale, whole); break;
-            case 5: prep_q_row<IO, D, 5, kStream>(row, qw, cs, sn, eps, plan.qscale, whole); break;
-            case 6: prep_q_row<IO, D, 6, kStream>(row, qw, cs, sn, eps, plan.qscale, whole); break;
-            case 7: prep_q_row<IO, D, 7, kStream>(row, qw, cs, sn, eps, plan.qscale, whole); break;
-            default: prep_q_row<IO, D, 8, kStream>(row, qw, cs, sn, eps, plan.qscale, whole); break;
-          }
-        }
-    }
-#pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const auto r = __builtin_amdgcn_permlane32_swap(whole[2 * kk][e], whole[2 * kk + 1][e], false, false);
-        if constexpr (T::SPLIT && NCT == 2) {  // lanes 0-31 held rows q0 .. q0 + 31 (column tile 0), 32-63 the next
-          qf[0][0][kk][e] = r[0];
-          qf[0][1][kk][e] = r[1];
-        } else if constexpr (T::SPLIT) {  // both lane halves held rows q0 .. q0 + 31
-          qf[0][0][kk][e] = r[0];
-        } else {  // lanes 0-31 held branch 1, lanes 32-63 branch 2, both for rows q0 .. q0 + 31
-          qf[0][0][kk][e] = r[0];
-          qf[1][0][kk][e] = r[1];
-        }
-      }
-  }
+  rows.template prep<ROPE>(query, cs, sn, half, lh, plan.qscale, qf);
 
   f32x16 o[NB][NCT][D / 32];
   float lsum[NB][NCT];
@@ -433,8 +307,6 @@ __global__ __launch_bounds__(64 * NW, D == 64 ? (QB == 64 ? 3 : 2) : 1) void den
       for (int dt = 0; dt < D / 32; ++dt) o[bi][ct][dt] = f32x16{};
     }
 
-  const TileCopy<D, NW> copy(ws + rowbase * D, ws + region + rowbase * D, ws + 2 * region + rowbase * D);
-  copy(0, lds_addr(smem));
   if (plan.fast)
     dense_attend_loop<D, QB, NW, true>(copy, Lk, br0, smem, smem + T::STAGE, qf, o, lsum, plan.c);
   else
@@ -520,6 +392,11 @@ int launch_dense_prep_16bit(hipStream_t stream, int dtype, const void* kv, int64
   return launch_status("dense_prep");
 }
 
+template <class IO, int D, int QB, int NW>
+static auto attend_kernel(int half) {
+  return half ? dense_attend<IO, D, QB, NW, true> : dense_attend<IO, D, QB, NW, false>;
+}
+
 int launch_dense_attend_16bit(hipStream_t stream, int dtype, const void* q, int64_t rs, int sqd, const float* qw,
                               const float* kw, const float* cos, const float* sin, int half, float eps,
                               const float* lam, void* out, int B, int L, int Lk, int H, int D, const DenseLayout& lay,
@@ -541,8 +418,8 @@ int launch_dense_attend_16bit(hipStream_t stream, int dtype, const void* q, int6
   const bool spread = 2 * blocks128 <= ncu || (blocks128 > ncu && 2 * blocks128 <= 3 * ncu) ||
                       (blocks128 > 2 * ncu && 8 * blocks128 <= 17 * ncu);
   if (D == 64 && spread) {
-    const int nblocks = B * H * (Lp / 64);
-    auto kernel = f16 ? dense_attend<F16Io, 64, 64, 4> : dense_attend<Bf16Io, 64, 64, 4>;
+    const int nblocks = B * H * ((L + 63) / 64);
+    auto kernel = f16 ? attend_kernel<F16Io, 64, 64, 4>(half) : attend_kernel<Bf16Io, 64, 64, 4>(half);
     hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(DenseTile<64, 64>::NT), 0, stream, x, rs, sqd, cos, sin, half, eps,
                        ws, lay.region_elems, B, L, Lp, Lk, Lkp, H, qw, kw, lam, o);
   } else {
@@ -550,9 +427,9 @@ int launch_dense_attend_16bit(hipStream_t stream, int dtype, const void* q, int6
     // form, whose fixed part per workgroup is smaller (measured: 7 % faster at L = 1292 and 2584, 17 % slower at
     // L = 216 with 48 workgroups)
     const bool w8 = D == 128 && blocks128 >= ncu;
-    auto kernel = D == 64 ? (f16 ? dense_attend<F16Io, 64, 128, 4> : dense_attend<Bf16Io, 64, 128, 4>)
-                  : w8    ? (f16 ? dense_attend<F16Io, 128, 128, 8> : dense_attend<Bf16Io, 128, 128, 8>)
-                          : (f16 ? dense_attend<F16Io, 128, 128, 4> : dense_attend<Bf16Io, 128, 128, 4>);
+    auto kernel = D == 64 ? (f16 ? attend_kernel<F16Io, 64, 128, 4>(half) : attend_kernel<Bf16Io, 64, 128, 4>(half))
+                  : w8    ? (f16 ? attend_kernel<F16Io, 128, 128, 8>(half) : attend_kernel<Bf16Io, 128, 128, 8>(half))
+                          : (f16 ? attend_kernel<F16Io, 128, 128, 4>(half) : attend_kernel<Bf16Io, 128, 128, 4>(half));
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks128)), dim3(w8 ? 512 : 256), 0, stream, x, rs, sqd,
                        cos, sin, half, eps, ws, lay.region_elems, B, L, Lp, Lk, Lkp, H, qw, kw, lam, o);
   }

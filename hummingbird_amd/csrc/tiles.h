@@ -3,6 +3,8 @@
 // workgroup. Shared by dense.hip and band_tiled.hip.
 #pragma once
 
+#include <type_traits>
+
 #include "attn_tile.h"
 #include "common.h"
 
@@ -99,11 +101,13 @@ struct TileCopy {
   }
 };
 
-// out[q, h*D + d] = O1 / l1 - lam * O2 / l2 for the QB queries of a 4-wave workgroup laid out as DenseTile<D, QB>
+// out[q, h*D + d] = O1 / l1 - lam * O2 / l2 for the QB queries of a workgroup laid out as DenseTile<D, QB, NW>
 // describes (q0w: this wave's first query, br0: its first branch), written in the output type IO for q < N.
-// D = 64: the branch-2 waves publish lam * O2 / l2 (rounded per element) through LDS (`xbuf_mem`, at least
-// 32 KB, free of tile reads: the caller has passed a barrier after its last tile) and the branch-1 waves
-// subtract it from O1 / l1; D = 128: each wave holds both branches. Every lane of the workgroup must call it.
+// Split layouts: the two waves of the same queries each finish half of their 32 x 32 tiles. Each publishes its
+// normalised other half (rounded per element) through LDS (`xbuf_mem`, free of tile reads: the caller has passed a
+// barrier after its last tile), 16 bytes per lane and access, and subtracts, in the same order in both, what it gets
+// back. Handing everything to the branch-1 waves left the others idle: the call at B = 1, L = 1422, 24 x 64
+// 46.1 -> 45.5 us, tiled band S = 16384, w = 256 104.3 -> 103.9. Other layouts: each wave holds both branches. Every lane of the workgroup must call it.
 template <int D, int QB = 128, class IO = Bf16Io, int NW = 4>
 __device__ __forceinline__ void store_diff_split(
     uint16_t* __restrict__ out, int64_t b, int N, int H, int h, int q0w, int br0, float lamh,
@@ -114,45 +118,59 @@ __device__ __forceinline__ void store_diff_split(
   const int lane = threadIdx.x & 63, wave = wave_id(), lr = lane & 31, lh = lane >> 5;
   const int64_t HD = static_cast<int64_t>(H) * D;
   if constexpr (T::SPLIT) {
-    float* xbuf = reinterpret_cast<float*>(xbuf_mem);  // 2 query halves x NCT x D/32 x 16 registers x 64 lanes
-    const int slot0 = (wave % (NW / 2)) * NCT * (D / 32) * 16;
-    if (br0 == 1) {
+    constexpr int HALF = NCT * (D / 32) / 2;  // tiles a wave finishes: column tile 0 or 1, or half of the dims
+    f32x4* xbuf = reinterpret_cast<f32x4*>(xbuf_mem);  // [branch][query group][HALF][4][64 lanes]
+    const int pair = wave % (NW / 2);
+    float f[NCT];
 #pragma unroll
-      for (int ct = 0; ct < NCT; ++ct) {
-        const float i1 = __fmul_rn(lamh, inv_rowsum(lsum, 0, ct));
-#pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            xbuf[(slot0 + (ct * (D / 32) + dt) * 16 + r) * 64 + lane] = __fmul_rn(o[0][ct][dt][r], i1);
-      }
+    for (int ct = 0; ct < NCT; ++ct) {
+      f[ct] = inv_rowsum(lsum, 0, ct);
+      if (br0 == 1) f[ct] = __fmul_rn(lamh, f[ct]);
     }
-    __syncthreads();
-    if (br0 == 0) {
+    auto publish = [&](auto first) {
 #pragma unroll
-      for (int ct = 0; ct < NCT; ++ct) {
-        const float i0 = inv_rowsum(lsum, 0, ct);
+      for (int k = 0; k < HALF; ++k) {
+        const int i = decltype(first)::value + k, ct = i / (D / 32), dt = i % (D / 32);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          f32x4 v;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = __fmul_rn(o[0][ct][dt][4 * g + j], f[ct]);
+          xbuf[(((br0 * (NW / 2) + pair) * HALF + k) * 4 + g) * 64 + lane] = v;
+        }
+      }
+    };
+    auto finish = [&](auto first) {
+#pragma unroll
+      for (int k = 0; k < HALF; ++k) {
+        const int i = decltype(first)::value + k, ct = i / (D / 32), dt = i % (D / 32);
         const int q = q0w + 32 * ct + lr;
         uint16_t* orow = out + (b * N + q) * HD + h * D;
 #pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt)
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 x = xbuf[((((1 - br0) * (NW / 2) + pair) * HALF + k) * 4 + g) * 64 + lane];
+          float v[4];
 #pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            float v[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const int r = 4 * g + j;
-              v[j] = __fsub_rn(__fmul_rn(o[0][ct][dt][r], i0), xbuf[(slot0 + (ct * (D / 32) + dt) * 16 + r) * 64 + lane]);
-            }
-            if (q < N) {
-              u32x2 pk;
-              pk[0] = IO::pack2(v[0], v[1]);
-              pk[1] = IO::pack2(v[2], v[3]);
-              *reinterpret_cast<u32x2*>(orow + 32 * dt + 8 * g + 4 * lh) = pk;
-            }
+          for (int j = 0; j < 4; ++j) {
+            const float y = __fmul_rn(o[0][ct][dt][4 * g + j], f[ct]);
+            v[j] = decltype(first)::value == 0 ? __fsub_rn(y, x[j]) : __fsub_rn(x[j], y);
           }
+          if (q < N) {
+            u32x2 pk;
+            pk[0] = IO::pack2(v[0], v[1]);
+            pk[1] = IO::pack2(v[2], v[3]);
+            *reinterpret_cast<u32x2*>(orow + 32 * dt + 8 * g + 4 * lh) = pk;
+          }
+        }
       }
-    }
+    };
+    const std::integral_constant<int, 0> lower;
+    const std::integral_constant<int, HALF> upper;
+    if (br0 == 0) publish(upper);
+    else publish(lower);
+    __syncthreads();
+    if (br0 == 0) finish(lower);
+    else finish(upper);
   } else {
 #pragma unroll
     for (int ct = 0; ct < NCT; ++ct) {
