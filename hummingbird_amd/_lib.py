@@ -10,6 +10,8 @@ import os
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 from pathlib import Path
 
+import torch
+
 # HUMMINGBIRD_AMD_LIB names another build of the same library (the host-sanitizer build of `_build.py`).
 LIB_PATH = Path(os.environ.get("HUMMINGBIRD_AMD_LIB") or Path(__file__).resolve().parent / "libhummingbird_amd.so")
 
@@ -91,6 +93,12 @@ def load() -> ctypes.CDLL:
             fn.restype, fn.argtypes = res, args
         _lib = lib
     return _lib
+
+
+def current_stream(device: torch.device) -> int:
+    """The handle of torch's current stream on a tensor's device. `torch.cuda.current_stream(device).cuda_stream` is
+    the same handle, but builds a Stream object for it: 1.8 us a call against 0.1, on calls of 10 us and more."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def check(status: int, what: str) -> None:

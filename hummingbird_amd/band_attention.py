@@ -11,8 +11,8 @@ import torch
 
 from hummingbird_amd import _lib, rotary
 from hummingbird_amd._derived import derived
-from hummingbird_amd.dense_attention import (SUPPORTED_HEAD_DIMS, _f32, _require_gpu, _row_stride, dtype_code,
-                                             rope_tables)
+from hummingbird_amd.dense_attention import (SUPPORTED_HEAD_DIMS, _f32, _f32_vector, _require_gpu, _row_stride,
+                                             dtype_code, rope_tables)
 
 __all__ = ["band_attention", "band_workspace", "rope_tables", "pack_dyt"]
 
@@ -119,7 +119,7 @@ def band_attention(qkv: torch.Tensor, q_norm: dict, k_norm: dict, inv_freq: torc
         cos_p, sin_p = cos.data_ptr(), sin.data_ptr()
     lam_p = 0
     if lam is not None:
-        lam = _f32(lam, dev).reshape(-1)
+        lam = _f32_vector(lam, dev)
         if lam.numel() != num_heads:
             raise ValueError("lam must have num_heads elements")
         lam_p = lam.data_ptr()
@@ -134,7 +134,7 @@ def band_attention(qkv: torch.Tensor, q_norm: dict, k_norm: dict, inv_freq: torc
             if workspace.numel() * workspace.element_size() < need or workspace.device != dev:
                 raise ValueError(f"workspace must hold {need} bytes on {dev}")
             ws_p, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _lib.current_stream(dev)
     status = lib.hb_band_diffattn(stream, qkv.data_ptr(), code, rs, qd.data_ptr(), kd.data_ptr(), cos_p, sin_p, half,
                                   int(window), lam_p, out.data_ptr(), batch, length, num_heads, head_dim, ws_p,
                                   ws_bytes)

@@ -15,7 +15,7 @@ from dataclasses import dataclass
 import torch
 
 from hummingbird_amd import _lib
-from hummingbird_amd.dense_attention import SUPPORTED_HEAD_DIMS, _f32, _require_gpu, _row_stride, dtype_code
+from hummingbird_amd.dense_attention import SUPPORTED_HEAD_DIMS, _f32_vector, _require_gpu, _row_stride, dtype_code
 
 
 @dataclass(frozen=True)
@@ -53,7 +53,7 @@ def prepare_cross_kv(kv: torch.Tensor, k_weight: torch.Tensor, num_heads: int, h
     dev = kv.device
     code = dtype_code(kv.dtype)
     batch, length, _ = kv.shape
-    kw = _f32(k_weight, dev).reshape(-1)
+    kw = _f32_vector(k_weight, dev)
     if kw.numel() != head_dim:
         raise ValueError("k_weight must have head_dim elements")
     lib = _lib.load()
@@ -62,7 +62,7 @@ def prepare_cross_kv(kv: torch.Tensor, k_weight: torch.Tensor, num_heads: int, h
         workspace = torch.empty(need, dtype=torch.uint8, device=dev)
     elif workspace.numel() * workspace.element_size() < need or workspace.device != dev:
         raise ValueError(f"workspace must hold {need} bytes on {dev}")
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _lib.current_stream(dev)
     status = lib.hb_cross_prep(stream, kv.data_ptr(), code, _row_stride(kv), kw.data_ptr(), batch, length, num_heads,
                                head_dim, float(eps), workspace.data_ptr(), workspace.numel() * workspace.element_size())
     _lib.check(status, "prepare_cross_kv")
@@ -87,18 +87,18 @@ def cross_attention(q: torch.Tensor, context: CrossKV, q_weight: torch.Tensor, e
     dev = q.device
     if context.workspace.device != dev:
         raise ValueError("q and the prepared context must be on the same device")
-    qw = _f32(q_weight, dev).reshape(-1)
+    qw = _f32_vector(q_weight, dev)
     if qw.numel() != dim:
         raise ValueError("q_weight must have head_dim elements")
     lam_p = 0
     if lam is not None:
-        lam = _f32(lam, dev).reshape(-1)
+        lam = _f32_vector(lam, dev)
         if lam.numel() != heads:
             raise ValueError("lam must have num_heads elements")
         lam_p = lam.data_ptr()
     out = torch.empty((batch, length, heads * dim), dtype=q.dtype, device=dev)
     lib = _lib.load()
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _lib.current_stream(dev)
     ws = context.workspace
     status = lib.hb_cross_attend(stream, q.data_ptr(), dtype_code(q.dtype), _row_stride(q), qw.data_ptr(),
                                  context.k_weight.data_ptr(), lam_p, out.data_ptr(), batch, length, context.length,

@@ -34,7 +34,17 @@ def _require_gpu(t: torch.Tensor, name: str) -> None:
 
 
 def _f32(t: torch.Tensor, device: torch.device) -> torch.Tensor:
+    """`t` as contiguous fp32 on `device`. What is that already is returned as it is, without the calls that would
+    find so: with them, the views of 1-D operands and the Stream object of `current_stream` the self-attention of a
+    10 s clip, which waits for the host, took 15.9 us, without 11.8."""
+    if t.dtype is torch.float32 and t.device == device and t.is_contiguous():
+        return t
     return t.to(device=device, dtype=torch.float32).contiguous()
+
+
+def _f32_vector(t: torch.Tensor, device: torch.device) -> torch.Tensor:
+    t = _f32(t, device)
+    return t if t.dim() == 1 else t.reshape(-1)
 
 
 def _row_stride(qkv: torch.Tensor) -> int:
@@ -55,7 +65,7 @@ def rope_tables(length: int, inv_freq: torch.Tensor) -> tuple[torch.Tensor, torc
     cos = torch.empty((length, half), dtype=torch.float32, device=inv_freq.device)
     sin = torch.empty_like(cos)
     lib = _lib.load()
-    stream = torch.cuda.current_stream(inv_freq.device).cuda_stream
+    stream = _lib.current_stream(inv_freq.device)
     _lib.check(lib.hb_rope_tables(stream, freq.data_ptr(), half, length, cos.data_ptr(), sin.data_ptr()),
                "rope_tables")
     return cos, sin
@@ -108,7 +118,7 @@ def dense_attention(qkv: torch.Tensor, q_weight: torch.Tensor, k_weight: torch.T
     dev = qkv.device
     code = dtype_code(qkv.dtype)
     rs = _row_stride(qkv)
-    qw, kw = _f32(q_weight, dev).reshape(-1), _f32(k_weight, dev).reshape(-1)
+    qw, kw = _f32_vector(q_weight, dev), _f32_vector(k_weight, dev)
     if qw.numel() != head_dim or kw.numel() != head_dim:
         raise ValueError("q_weight and k_weight must have head_dim elements")
     cos_p = sin_p = 0
@@ -132,7 +142,7 @@ def dense_attention(qkv: torch.Tensor, q_weight: torch.Tensor, k_weight: torch.T
         mask_p = mask.data_ptr()
     lam_p = 0
     if lam is not None:
-        lam = _f32(lam, dev).reshape(-1)
+        lam = _f32_vector(lam, dev)
         if lam.numel() != num_heads:
             raise ValueError("lam must have num_heads elements")
         lam_p = lam.data_ptr()
@@ -143,7 +153,7 @@ def dense_attention(qkv: torch.Tensor, q_weight: torch.Tensor, k_weight: torch.T
     elif workspace.numel() * workspace.element_size() < need or workspace.device != dev:
         raise ValueError(f"workspace must hold {need} bytes on {dev}")
     out = torch.empty((batch, length, num_heads * head_dim), dtype=qkv.dtype, device=dev)
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _lib.current_stream(dev)
     status = lib.hb_dense_diffattn(stream, qkv.data_ptr(), code, rs, qw.data_ptr(), kw.data_ptr(), cos_p, sin_p, half,
                                    mask_p, lam_p, out.data_ptr(), batch, length, num_heads, head_dim, float(eps),
                                    workspace.data_ptr(), workspace.numel() * workspace.element_size())

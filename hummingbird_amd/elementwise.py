@@ -41,7 +41,7 @@ def dyt(x: torch.Tensor, norm: dict) -> torch.Tensor:
     params = pack_dyt(norm, channels, x.device)
     rows, stride = _rows(x, "x")
     out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = _lib.current_stream(x.device)
     _lib.check(_lib.load().hb_dyt(stream, x.data_ptr(), dtype_code(x.dtype), stride, params.data_ptr(), out.data_ptr(),
                                   channels, rows, channels), "dyt")
     return out
@@ -65,7 +65,7 @@ def glu(proj: torch.Tensor, sinusoidal: bool, bias: torch.Tensor | None = None) 
             raise ValueError(f"bias must have {width} elements")
         bias_p = bias.data_ptr()
     out = torch.empty((*proj.shape[:-1], inner), dtype=proj.dtype, device=proj.device)
-    stream = torch.cuda.current_stream(proj.device).cuda_stream
+    stream = _lib.current_stream(proj.device)
     _lib.check(_lib.load().hb_glu(stream, proj.data_ptr(), dtype_code(proj.dtype), stride, bias_p,
                                   int(bool(sinusoidal)), out.data_ptr(), inner, rows, inner), "glu")
     return out
@@ -92,7 +92,7 @@ def residual_dyt(h: torch.Tensor, x: torch.Tensor, bias: torch.Tensor | None = N
     params = pack_dyt(norm, channels, h.device) if norm is not None else None
     out_h = torch.empty(h.shape, dtype=h.dtype, device=h.device)
     out_y = torch.empty(h.shape, dtype=h.dtype, device=h.device) if norm is not None else None
-    stream = torch.cuda.current_stream(h.device).cuda_stream
+    stream = _lib.current_stream(h.device)
     _lib.check(_lib.load().hb_residual_dyt(stream, h.data_ptr(), dtype_code(h.dtype), hs, x.data_ptr(), xs, bias_p,
                                            params.data_ptr() if params is not None else 0, out_h.data_ptr(),
                                            out_y.data_ptr() if out_y is not None else 0, channels, rows, channels),
@@ -133,7 +133,7 @@ def rms_modulate(x: torch.Tensor, weight: torch.Tensor, eps: float, scale: torch
     if scale is not None and ms != ms2:
         raise ValueError("scale and shift must share their batch stride")
     out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = _lib.current_stream(x.device)
     _lib.check(_lib.load().hb_rms_modulate(stream, x.data_ptr(), dtype_code(x.dtype), stride, w.data_ptr(), float(eps),
                                            sp, hp, ms, length, out.data_ptr(), channels, rows, channels),
                "rms_modulate")
@@ -161,7 +161,7 @@ def gated_residual(h: torch.Tensor, x: torch.Tensor, gate: torch.Tensor | None =
             raise ValueError(f"{name} must be ({channels},) of {h.dtype} with unit stride")
         return t.data_ptr()
     out = torch.empty(h.shape, dtype=h.dtype, device=h.device)
-    stream = torch.cuda.current_stream(h.device).cuda_stream
+    stream = _lib.current_stream(h.device)
     _lib.check(_lib.load().hb_gated_residual(stream, h.data_ptr(), dtype_code(h.dtype), hs, x.data_ptr(), xs,
                                              vec(x_bias, "x_bias"), gp, gs, vec(local, "local"), int(memory), length,
                                              out.data_ptr(), channels, rows, channels), "gated_residual")
@@ -201,7 +201,7 @@ def residual_rms(h: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, eps: fl
         return t.data_ptr()
     out_h = torch.empty(h.shape, dtype=h.dtype, device=h.device)
     out_y = torch.empty(h.shape, dtype=h.dtype, device=h.device)
-    stream = torch.cuda.current_stream(h.device).cuda_stream
+    stream = _lib.current_stream(h.device)
     _lib.check(_lib.load().hb_residual_rms(stream, h.data_ptr(), dtype_code(h.dtype), hs, x.data_ptr(), xs,
                                            vec(x_bias, "x_bias"), gp, gs, vec(local, "local"), int(memory),
                                            w.data_ptr(), float(eps), sp, hp, ms, length, out_h.data_ptr(),

@@ -15,7 +15,7 @@ import torch
 from hummingbird_amd import _lib
 from hummingbird_amd._derived import f32_vector
 from hummingbird_amd.band_attention import pack_dyt
-from hummingbird_amd.dense_attention import _f32, _require_gpu, dtype_code
+from hummingbird_amd.dense_attention import _f32, _f32_vector, _require_gpu, dtype_code
 
 FUSED_DTYPES = (torch.bfloat16, torch.float16)
 
@@ -65,7 +65,7 @@ def qkv_projection(h: torch.Tensor, w_qkv: torch.Tensor, k_weight: torch.Tensor,
         raise ValueError(f"w_qkv must be (5*H*D, E) = ({5 * num_heads * head_dim}, {width}), got {tuple(w.shape)}")
     _, hs = _rows(h, "h")
     _, ws_ = _rows(w, "w_qkv")
-    kw = _f32(k_weight, dev).reshape(-1)
+    kw = _f32_vector(k_weight, dev)
     cos_p = sin_p = 0
     if half > 0:
         cos, sin = _f32(cos, dev), _f32(sin, dev)
@@ -82,7 +82,7 @@ def qkv_projection(h: torch.Tensor, w_qkv: torch.Tensor, k_weight: torch.Tensor,
     elif workspace.numel() * workspace.element_size() < need or workspace.device != dev:
         raise ValueError(f"workspace must hold {need} bytes on {dev}")
     qq = torch.empty((batch, length, 2 * num_heads * head_dim), dtype=h.dtype, device=dev)
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _lib.current_stream(dev)
     _lib.check(lib.hb_dit_qkv_proj(stream, h.data_ptr(), code, hs, w.data_ptr(), ws_, width, kw.data_ptr(), cos_p,
                                    sin_p, half, mask_p, qq.data_ptr(), batch, length, num_heads, head_dim, float(eps),
                                    workspace.data_ptr(), workspace.numel() * workspace.element_size()), "qkv_projection")
@@ -98,18 +98,18 @@ def attend_projected(qq: torch.Tensor, q_weight: torch.Tensor, k_weight: torch.T
     batch, length, _ = qq.shape
     dev = qq.device
     _, rs = _rows(qq, "qq")
-    qw, kw = _f32(q_weight, dev).reshape(-1), _f32(k_weight, dev).reshape(-1)
+    qw, kw = _f32_vector(q_weight, dev), _f32_vector(k_weight, dev)
     cos_p = sin_p = 0
     if half > 0:
         cos, sin = _f32(cos, dev), _f32(sin, dev)
         cos_p, sin_p = cos.data_ptr(), sin.data_ptr()
     lam_p = 0
     if lam is not None:
-        lam = _f32(lam, dev).reshape(-1)
+        lam = _f32_vector(lam, dev)
         lam_p = lam.data_ptr()
     out = torch.empty((batch, length, num_heads * head_dim), dtype=qq.dtype, device=dev)
     lib = _lib.load()
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _lib.current_stream(dev)
     _lib.check(lib.hb_dense_attend_qq(stream, qq.data_ptr(), dtype_code(qq.dtype), rs, qw.data_ptr(), kw.data_ptr(),
                                       cos_p, sin_p, half, lam_p, out.data_ptr(), batch, length, num_heads, head_dim,
                                       float(eps), workspace.data_ptr(), workspace.numel() * workspace.element_size()),
@@ -130,7 +130,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     if x.shape[-1] != k:
         raise ValueError(f"x has {x.shape[-1]} columns, weight {k}")
     out = torch.empty((*x.shape[:-1], f), dtype=x.dtype, device=x.device)
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = _lib.current_stream(x.device)
     _lib.check(_lib.load().hb_proj(stream, x.data_ptr(), dtype_code(x.dtype), xs, w.data_ptr(), wstride, out.data_ptr(),
                                    f, n, k, f), "linear")
     return out
@@ -158,7 +158,7 @@ def glu_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
             raise ValueError(f"bias must have {f2} elements")
         bias_p = bias.data_ptr()
     out = torch.empty((*x.shape[:-1], f), dtype=x.dtype, device=x.device)
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = _lib.current_stream(x.device)
     _lib.check(_lib.load().hb_proj_glu(stream, x.data_ptr(), dtype_code(x.dtype), xs, w.data_ptr(), wstride, bias_p,
                                        int(bool(sinusoidal)), out.data_ptr(), f, n, k, f), "glu_linear")
     return out
@@ -192,7 +192,7 @@ def residual_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | 
     params = pack_dyt(norm, f, x.device) if norm is not None else None
     out_h = torch.empty(h.shape, dtype=x.dtype, device=x.device)
     out_y = torch.empty(h.shape, dtype=x.dtype, device=x.device) if norm is not None else None
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = _lib.current_stream(x.device)
     _lib.check(_lib.load().hb_proj_residual(stream, x.data_ptr(), dtype_code(x.dtype), xs, w.data_ptr(), wstride,
                                             bias_p, h.data_ptr(), hs, params.data_ptr() if params is not None else 0,
                                             out_h.data_ptr(), out_y.data_ptr() if out_y is not None else 0, f, n, k,
