@@ -21,8 +21,6 @@
 
 namespace hb {
 
-typedef f32x4 f32x4_align4 __attribute__((aligned(4)));  // the norm parameters need only be aligned as floats
-
 // RMSNorm (dit.py:45-57) with the dense path's cast points: the compute dtype IO after the gain and after the
 // rotation (dense_attention.py:66, 69).
 template <class IO, int D>
