@@ -11,8 +11,8 @@
 // results are nearer to the 64-bit ones than the fp32 chain's were: relative error (2-norm) 6.4e-7 against 9.1e-7 on
 // dense B = 2, L = 1292, 8.4e-7 against 1.3e-6 at L = 2584, 7.0e-7 against 7.9e-7 on the band at w = 17 (24 heads, no
 // lambda), 1.2e-6 against 1.6e-6 at w = 100, 3.9e-7 against 5.4e-7 on the cross-attention. Times, whole calls against
-// the fp32 matrix cores fed through registers: dense (2, 1292, 24 heads) 534 -> 179 us, L = 2584 1565 -> 580, head_dim
-// 128 (2, 1292, 12 heads) 690 -> 180, cross (2, 2584 x 257) 205 -> 78, band S = 16384, w = 128 263 -> 138. Three bf16 terms
+// the fp32 matrix cores fed through registers: dense (2, 1292, 24 heads) 534 -> 171 us, L = 2584 1565 -> 571, head_dim
+// 128 (2, 1292, 12 heads) 690 -> 166, cross (2, 2584 x 257) 205 -> 70, band S = 16384, w = 128 263 -> 133. Three bf16 terms
 // and six products, which need no scaling, were measured too: 290 us for the first of these. The matrix cores slow down
 // on such operands (about 27 ns per 32x32x16 product and SIMD), so the number of products sets the time.
 //
@@ -65,17 +65,27 @@ struct SplitTile {
   __device__ static __forceinline__ int v_at(int d, int chunk) { return d * KT + 8 * (chunk ^ ((d >> 2) & 3)); }
 };
 
-// 8 values as hi + lo halves.
+// x - h for the low (hi false) or high half h of a pair, in one instruction (the compiler converts, then subtracts).
+template <bool HI>
+__device__ __forceinline__ float minus_half(float x, uint32_t pair) {
+  float r;
+  if constexpr (HI) asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(x));
+  else asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(x));
+  return r;
+}
+
+// 8 values as hi + lo halves: per pair, two packed conversions (v_cvt_pk_f16_f32) and two mixed subtractions. Written
+// value by value the pair took ten instructions, six of them at half rate; the splits of P are a fifth of a tile's
+// vector work. With the key tile's fragments read ahead of the products (attend_tile_f32): dense (2, 1292, 24 heads)
+// 181 -> 171 us, cross (2, 2584 x 257) 74 -> 70, band S = 16384, w = 128 137 -> 133; the same bits.
 __device__ __forceinline__ void split8(const float (&x)[8], u32x4& hi, u32x4& lo) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    f16x2 h, l;
-    h[0] = static_cast<_Float16>(x[2 * i]);
-    h[1] = static_cast<_Float16>(x[2 * i + 1]);
-    l[0] = static_cast<_Float16>(__fmaf_rn(static_cast<float>(h[0]), -1.f, x[2 * i]));
-    l[1] = static_cast<_Float16>(__fmaf_rn(static_cast<float>(h[1]), -1.f, x[2 * i + 1]));
-    hi[i] = __builtin_bit_cast(uint32_t, h);
-    lo[i] = __builtin_bit_cast(uint32_t, l);
+    const f32x2 v = {x[2 * i], x[2 * i + 1]};
+    const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2));
+    const f32x2 r = {minus_half<false>(v[0], h), minus_half<true>(v[1], h)};
+    hi[i] = h;
+    lo[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, f16x2));
   }
 }
 
@@ -251,9 +261,15 @@ __device__ __forceinline__ void attend_tile_f32(const uint16_t* __restrict__ sK,
   const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
   const int e = VTile<D>::exponent(sV);
   f32x16 s = f32x16{};
+  u32x4 kf[2][D / 16];  // all in flight before the first product: one wait for LDS instead of one per product pair
+#pragma unroll
+  for (int kk = 0; kk < D / 16; ++kk)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) kf[i][kk] = lds16(sK + i * T::PLANE + T::k_at(lr, 2 * kk + lh));
+  if constexpr (D == 64) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int kk = 0; kk < D / 16; ++kk) {
-    const u32x4 hi = lds16(sK + T::k_at(lr, 2 * kk + lh)), lo = lds16(sK + T::PLANE + T::k_at(lr, 2 * kk + lh));
+    const u32x4 hi = kf[0][kk], lo = kf[1][kk];
     s = mfma_f16_32x32x16(lo, q[0][kk], s);
     s = mfma_f16_32x32x16(hi, q[1][kk], s);
     s = mfma_f16_32x32x16(hi, q[0][kk], s);
