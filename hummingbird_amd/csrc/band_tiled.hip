@@ -30,6 +30,9 @@ namespace band_tiled {
 // DyT + RoPE of k and k_diff (and V transposed) for 64 keys of one head. Thread task = (key, RoPE group pair) as
 // in the dense prep: the rotation partner and the cos / sin slice are in the thread's own registers.
 // `kdyt` = [alpha, gamma[D], beta[D]]; `half` % 8 == 0 (checked on the host).
+// Bound by bytes and by how many loads are in flight: every load is issued first, and V goes out before the arithmetic
+// of the keys, so that its registers are free there (58 instead of 70: 8 waves per SIMD, and the 2048 workgroups of
+// S = 16384, 8 heads of 64 all run at once): 30.4 -> 27.6 us there (101 MB), the call at w = 256 103.9 -> 99.8.
 // IO: the element type of qkv (bf16 or half); the keys are prepared in bf16 either way.
 template <class IO, int D>
 __global__ __launch_bounds__(256) void band_prep(const uint16_t* __restrict__ qkv, int64_t rs,
@@ -83,6 +86,28 @@ __global__ __launch_bounds__(256) void band_prep(const uint16_t* __restrict__ qk
                     : u32x4{0u, 0u, 0u, 0u};
   }
 
+  // V (rounded to bf16, band_attention.py:94), transposed per 64-key tile (v_tile_key order) through LDS, the
+  // 16-byte chunks of row r XOR-swizzled by (r / 8) % 8.
+  __shared__ __attribute__((aligned(16))) uint16_t vt[64 * D];
+  auto vt_at = [](int row, int col) { return row * D + 8 * ((col >> 3) ^ ((row >> 3) & 7)) + (col & 7); };
+#pragma unroll
+  for (int i = 0; i < VCH; ++i) {
+    const int ch = t + 256 * i, key = ch / (D / 8), col = (ch % (D / 8)) * 8;
+    *reinterpret_cast<u32x4*>(vt + vt_at(key, col)) = IO::to_bf16x8(vraw[i]);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < VCH; ++i) {
+    const int ch = t + 256 * i, d = ch / 8, pos0 = (ch % 8) * 8;
+    uint16_t e[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) e[j] = vt[vt_at(v_tile_key(pos0 + j), d)];
+    u32x4 w;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = static_cast<uint32_t>(e[2 * j]) | (static_cast<uint32_t>(e[2 * j + 1]) << 16);
+    st16(ws + 2 * region + (bh * Sp + l0) * D + d * 64 + pos0, w);
+  }
+
 #pragma unroll
   for (int i = 0; i < TASKS; ++i) {
     const int task = t + 256 * i, l = l0 + task / PAIRS;
@@ -112,27 +137,6 @@ __global__ __launch_bounds__(256) void band_prep(const uint16_t* __restrict__ qk
     }
   }
 
-  // V (rounded to bf16, band_attention.py:94), transposed per 64-key tile (v_tile_key order) through LDS, the
-  // 16-byte chunks of row r XOR-swizzled by (r / 8) % 8.
-  __shared__ __attribute__((aligned(16))) uint16_t vt[64 * D];
-  auto vt_at = [](int row, int col) { return row * D + 8 * ((col >> 3) ^ ((row >> 3) & 7)) + (col & 7); };
-#pragma unroll
-  for (int i = 0; i < VCH; ++i) {
-    const int ch = t + 256 * i, key = ch / (D / 8), col = (ch % (D / 8)) * 8;
-    *reinterpret_cast<u32x4*>(vt + vt_at(key, col)) = IO::to_bf16x8(vraw[i]);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < VCH; ++i) {
-    const int ch = t + 256 * i, d = ch / 8, pos0 = (ch % 8) * 8;
-    uint16_t e[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) e[j] = vt[vt_at(v_tile_key(pos0 + j), d)];
-    u32x4 w;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) w[j] = static_cast<uint32_t>(e[2 * j]) | (static_cast<uint32_t>(e[2 * j + 1]) << 16);
-    st16(ws + 2 * region + (bh * Sp + l0) * D + d * 64 + pos0, w);
-  }
 }
 
 // The window's tiles, double-buffered: tile t_lo has already been issued into stage A by the caller. A wave

@@ -12,9 +12,10 @@
 // dense B = 2, L = 1292, 8.4e-7 against 1.3e-6 at L = 2584, 7.0e-7 against 7.9e-7 on the band at w = 17 (24 heads, no
 // lambda), 1.2e-6 against 1.6e-6 at w = 100, 3.9e-7 against 5.4e-7 on the cross-attention. Times, whole calls against
 // the fp32 matrix cores fed through registers: dense (2, 1292, 24 heads) 534 -> 171 us, L = 2584 1565 -> 571, head_dim
-// 128 (2, 1292, 12 heads) 690 -> 166, cross (2, 2584 x 257) 205 -> 70, band S = 16384, w = 128 263 -> 133. Three bf16 terms
-// and six products, which need no scaling, were measured too: 290 us for the first of these. The matrix cores slow down
-// on such operands (about 27 ns per 32x32x16 product and SIMD), so the number of products sets the time.
+// 128 (2, 1292, 12 heads) 690 -> 166, cross (2, 2584 x 257) 205 -> 70, band S = 16384, w = 128 263 -> 133.
+// Three bf16 terms and six products, which need no scaling, were measured too: 290 us for the first of these. The
+// matrix cores slow down on such operands (about 27 ns per 32x32x16 product and SIMD), so the number of products sets
+// the time.
 //
 //   S^T[key][query] = K Q^T   A = K rows from LDS, B = q in registers
 //   P = exp2(S^T c - m)       m the running max of S^T c (online softmax), one FMA per score; masked scores are -inf
@@ -69,8 +70,10 @@ struct SplitTile {
 template <bool HI>
 __device__ __forceinline__ float minus_half(float x, uint32_t pair) {
   float r;
-  if constexpr (HI) asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(x));
-  else asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(x));
+  if constexpr (HI)
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(x));
+  else
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(x));
   return r;
 }
 
