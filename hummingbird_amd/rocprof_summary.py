@@ -38,6 +38,8 @@ def short_name(name: str) -> str:
         base, args = m.group(1), [a.strip() for a in (m.group(2) or "").split(",") if a.strip()]
         if args and args[0] in IO_SUFFIX:
             base, args = base + IO_SUFFIX[args[0]], args[1:]
+        if base.startswith("dense_attend_") and args[-1:] == ["true"]:
+            args.pop()  # the rotary form keeps the name it had before there was another
         return base + (f"<{','.join(args)}>" if args else "")
     if "at::native::" in name:  # torch: the kernel template and the operation it applies
         head = re.search(r"at::native::(?:\(anonymous namespace\)::)?(\w+)", name)
