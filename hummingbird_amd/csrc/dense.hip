@@ -267,8 +267,9 @@ __global__ __launch_bounds__(64 * NW, D == 64 ? (QB == 64 ? 3 : 2) : 1) void den
   const int tile = xcd_remap(blockIdx.x, B * H * nqb);
   const int qb = tile % nqb, bh = tile / nqb, h = bh % H, b = bh / H;
   const int lane = threadIdx.x & 63, wave = wave_id(), lr = lane & 31, lh = lane >> 5;
-  const int br0 = T::SPLIT ? wave / (NW / 2) : 0;                                 // first branch of this wave
-  const int q0 = qb * QB + (T::SPLIT ? (wave % (NW / 2)) * 32 * NCT : wave * 32);  // first query of this wave
+  static_assert(T::SPLIT, "a wave owns one branch");
+  const int br0 = wave / (NW / 2);                            // the branch of this wave
+  const int q0 = qb * QB + (wave % (NW / 2)) * 32 * NCT;      // first query of this wave
   const int64_t rowbase = static_cast<int64_t>(bh) * Lkp;
 
   const TileCopy<D, NW> copy(ws + rowbase * D, ws + region + rowbase * D, ws + 2 * region + rowbase * D);
@@ -314,7 +315,7 @@ __global__ __launch_bounds__(64 * NW, D == 64 ? (QB == 64 ? 3 : 2) : 1) void den
 
   // Both stages are free once every wave is past its last tile; the exchange reuses them.
   static_assert(T::XBUF_BYTES <= T::SMEM_ELEMS * 2, "exchange buffer exceeds the workgroup's LDS");
-  if constexpr (T::SPLIT) __syncthreads();
+  __syncthreads();
   store_diff_split<D, QB, IO, NW>(out, b, L, H, h, q0, br0, lam ? lam[h] : 1.f, o, lsum, smem);
 }
 
@@ -407,30 +408,28 @@ int launch_dense_attend_16bit(hipStream_t stream, int dtype, const void* q, int6
   uint16_t* o = static_cast<uint16_t*>(out);
   const int Lkp = static_cast<int>(lay.Lp);
   const bool f16 = dtype == HB_F16;
-  // 128-query workgroups run two per CU. With between one and one and a half of them per CU, some CUs would run
-  // two while most run one; 64-query workgroups (three per CU) spread the same work more evenly (measured: 6 %
-  // faster at 288 workgroups on 256 CUs; slower at exactly one per CU and at nearly two, where they cost more per
-  // query than they gain in balance). Just past two per CU (a nearly empty second round of 128-query workgroups)
-  // they win again: 3 % at 528 workgroups on 256 CUs (B = 2, L = 1292, H = 24). And on grids of at most half a
-  // 128-query workgroup per CU they halve the work of each busy CU: 9.8 against 11.4 us at B = 1, L = 216, H = 24.
+  // head_dim 64: 128-query workgroups run two per CU. With between one and one and a half of them per CU, some CUs would
+  // run two while most run one; 64-query workgroups (three per CU) spread the same work more evenly (3 to 9 % faster
+  // over that range, 4 % slower at exactly one per CU, 7 to 13 % between 1.6 and two, where they cost more per query
+  // than they gain in balance). Past two per CU, where the second round of 128-query workgroups is mostly empty, they
+  // win again: 7 % at 2.06, 5 % at 2.25, 4 % at 2.44 per CU; at 2.6 they lose 7 %. And on grids of at most half a
+  // 128-query workgroup per CU they halve the work of each busy CU: 16.2 against 19.6 us at B = 2, L = 512, H = 16.
   const int64_t blocks128 = static_cast<int64_t>(B) * H * (Lp / 128);
   const int64_t ncu = device_cus();
   const bool spread = 2 * blocks128 <= ncu || (blocks128 > ncu && 2 * blocks128 <= 3 * ncu) ||
-                      (blocks128 > 2 * ncu && 8 * blocks128 <= 17 * ncu);
+                      (blocks128 > 2 * ncu && 5 * blocks128 <= 12 * ncu);
   if (D == 64 && spread) {
     const int nblocks = B * H * ((L + 63) / 64);
     auto kernel = f16 ? attend_kernel<F16Io, 64, 64, 4>(half) : attend_kernel<Bf16Io, 64, 64, 4>(half);
     hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(DenseTile<64, 64>::NT), 0, stream, x, rs, sqd, cos, sin, half, eps,
                        ws, lay.region_elems, B, L, Lp, Lk, Lkp, H, qw, kw, lam, o);
   } else {
-    // head_dim 128: 8 waves of one branch each (two per SIMD) once the grid fills the GPU; below that the 4-wave
-    // form, whose fixed part per workgroup is smaller (measured: 7 % faster at L = 1292 and 2584, 17 % slower at
-    // L = 216 with 48 workgroups)
-    const bool w8 = D == 128 && blocks128 >= ncu;
+    // head_dim 128: 8 waves of one branch each, two per SIMD. With the queries of query.h they are faster on every grid
+    // than 4 waves holding both branches (12 heads, half 32: 29.0 against 32.7 us at B = 1, L = 512, 49.6 against 57.5
+    // at L = 1280, 185.7 against 202.7 at B = 2, L = 2584), which small grids ran before.
     auto kernel = D == 64 ? (f16 ? attend_kernel<F16Io, 64, 128, 4>(half) : attend_kernel<Bf16Io, 64, 128, 4>(half))
-                  : w8    ? (f16 ? attend_kernel<F16Io, 128, 128, 8>(half) : attend_kernel<Bf16Io, 128, 128, 8>(half))
-                          : (f16 ? attend_kernel<F16Io, 128, 128, 4>(half) : attend_kernel<Bf16Io, 128, 128, 4>(half));
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks128)), dim3(w8 ? 512 : 256), 0, stream, x, rs, sqd,
+                          : (f16 ? attend_kernel<F16Io, 128, 128, 8>(half) : attend_kernel<Bf16Io, 128, 128, 8>(half));
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks128)), dim3(D == 64 ? 256 : 512), 0, stream, x, rs, sqd,
                        cos, sin, half, eps, ws, lay.region_elems, B, L, Lp, Lk, Lkp, H, qw, kw, lam, o);
   }
   return launch_status("dense_attend");

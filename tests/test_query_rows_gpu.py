@@ -31,8 +31,8 @@ def check(got: torch.Tensor, ref: np.ndarray) -> None:
     assert_bf16_parity(got.float().cpu().numpy() / scale, ref / scale)
 
 
-# one 128-query block per head: 2 heads run as 64-query workgroups (D = 64) or 4 waves (D = 128), 130 heads as
-# 128-query workgroups of 4 waves, 256 heads of 128 as 8 waves
+# one 128-query block per head: at D = 64, 2 heads run as 64-query workgroups and 130 as 128-query ones; at D = 128
+# workgroups of 8 waves, one and a chip full
 @pytest.mark.parametrize("heads, dim, half", [(n, 64, h) for n in (2, 130) for h in (0, 8, 16, 24, 32)] +
                          [(n, 128, h) for n in (2, 256) for h in range(0, 65, 8)])
 def test_dense_rotary_widths(heads, dim, half):
@@ -60,3 +60,23 @@ def test_tiled_band_rotary_widths(dim, half):
                             lam=torch.from_numpy(b["lam"]).to(DEV))
     ref = oband.band_xla(b["qkv"], b["q_norm"], b["k_norm"], b["inv_freq"], 2, dim, window, b["lam"], "bf16")
     check(got, ref)
+
+
+@pytest.mark.parametrize("heads, length", [(100, 700), (101, 700), (102, 700), (110, 700)])
+def test_dense_forms_past_two_workgroups_a_cu(heads, length):
+    """6 blocks of 128 queries a head: 600 to 660 on 256 CUs, both sides of where 64-query workgroups end (2.4 a CU),
+    with a ragged last block; every head against the exact softmax of a sample of its queries."""
+    print(f"[case] dense {heads} heads, L = {length}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(heads)
+    qkv = torch.randn(1, length, 5 * heads * 64, device=DEV, generator=gen).bfloat16()
+    one = torch.ones(64, device=DEV)
+    got = da.dense_attention(qkv, one, one, None, None, None, heads, 64, 0, 1e-6).double().reshape(length, heads, 64)
+    q, k, v, qd, kd = (t.double().reshape(length, heads, 64).transpose(0, 1) for t in qkv[0].split(heads * 64, dim=-1))
+    rms = lambda t: t * torch.rsqrt((t * t).mean(-1, keepdim=True) + 1e-6)  # noqa: E731
+    rows = torch.tensor([0, 63, 64, 127, 128, 639, 640, 699], device=DEV)
+
+    def attend(a, b):
+        logits = (rms(a[:, rows])[:, :, None] * rms(b)[:, None]).sum(-1) / 8.0
+        return (torch.softmax(logits, -1)[..., None] * v[:, None]).sum(2)
+    ref = (attend(q, k) - attend(qd, kd)).transpose(0, 1)
+    assert (got[rows] - ref).abs().max() <= 2e-2  # the bf16 contract
