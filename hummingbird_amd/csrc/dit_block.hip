@@ -79,15 +79,24 @@ template <typename T>
 constexpr int kRowLanes = 2048 / Vec<T>::N;
 constexpr int kMaxRowBlocks = 1 << 20;  // workgroups of a launch; further rows are taken in turns
 
-// Sum over the workgroup, the same in every lane: waves added in order. `part` holds a value per wave.
-__device__ __forceinline__ float row_sum(float v, float* part) {
-  v = wave_sum(v);
-  if ((threadIdx.x & 63) == 0) part[wave_id()] = v;
+// Adds the squares of up to kRowLanes chunks of a row, one in each lane's `v` (zeros past the row), to `ss`: lane l of
+// every wave adds chunks l, l + 64, l + 128, ... in that order, and wave_sum of `ss` is then the row's sum, the same in
+// all waves. That is the order of one wave walking the row, so that a seed renders the same bits as with such waves;
+// adding the waves' own sums rounds otherwise in one of some thousand rows, which the 24 blocks of a denoiser grow to 2e-2.
+// `row` holds a chunk per lane and must be free of reads (a barrier lies between two calls).
+template <typename T>
+__device__ __forceinline__ void add_squares(const float (&v)[Vec<T>::N], T* row, float& ss) {
+  constexpr int V = Vec<T>::N;
+  Vec<T>::store(row + threadIdx.x * V, v);
   __syncthreads();
-  const int waves = blockDim.x / 64;
-  float sum = part[0];
-  for (int i = 1; i < waves; ++i) sum += part[i];
-  return sum;
+#pragma unroll
+  for (int k = 0; k < kRowLanes<T> / 64; ++k) {
+    if (64 * k >= static_cast<int>(blockDim.x)) break;
+    float u[V];
+    Vec<T>::load(row + (64 * k + (threadIdx.x & 63)) * V, u);
+#pragma unroll
+    for (int j = 0; j < V; ++j) ss = ss + u[j] * u[j];
+  }
 }
 
 template <typename T>
@@ -119,7 +128,7 @@ __global__ __launch_bounds__(kRowLanes<T>) void rms_modulate_kernel(
     const T* __restrict__ x, int64_t xs, const float* __restrict__ w, float eps, const T* __restrict__ scale,
     const T* __restrict__ shift, int64_t mod_stride, int L, T* __restrict__ out, int64_t os, int64_t N, int C) {
   constexpr int V = Vec<T>::N;
-  __shared__ float part[kRowLanes<T> / 64];
+  __shared__ __attribute__((aligned(16))) T squares[kRowLanes<T> * V];
   const int first = threadIdx.x * V, step = blockDim.x * V;
   for (int64_t n = blockIdx.x; n < N; n += gridDim.x) {
     const int64_t b = static_cast<unsigned>(n) / static_cast<unsigned>(L);  // N <= 2^31
@@ -135,15 +144,14 @@ __global__ __launch_bounds__(kRowLanes<T>) void rms_modulate_kernel(
       }
     }
     float ss = 0.f;
-#pragma unroll
-    for (int j = 0; j < V; ++j) ss = ss + v[j] * v[j];
-    for (int c0 = first + step; c0 < C; c0 += step) {
-      float u[V];
-      Vec<T>::load(row + c0, u);
-#pragma unroll
-      for (int j = 0; j < V; ++j) ss = ss + u[j] * u[j];
+    add_squares<T>(v, squares, ss);
+    for (int turn = step; turn < C; turn += step) {  // uniform: every lane joins every turn
+      float u[V] = {};
+      if (first + turn < C) Vec<T>::load(row + first + turn, u);
+      __syncthreads();
+      add_squares<T>(u, squares, ss);
     }
-    const float inv = rsqrtf(row_sum(ss, part) * (1.f / static_cast<float>(C)) + eps);
+    const float inv = rsqrtf(wave_sum(ss) * (1.f / static_cast<float>(C)) + eps);
     if (first < C) {
       norm_chunk<T>(v, inv, wv, scale != nullptr, s, t);
       Vec<T>::store(orow + first, v);
@@ -158,7 +166,7 @@ __global__ __launch_bounds__(kRowLanes<T>) void rms_modulate_kernel(
       norm_chunk<T>(v, inv, wv, scale != nullptr, s, t);
       Vec<T>::store(orow + c0, v);
     }
-    if (n + gridDim.x < N) __syncthreads();  // `part` is free again
+    if (n + gridDim.x < N) __syncthreads();  // `squares` is free again
   }
 }
 
@@ -217,7 +225,7 @@ __global__ __launch_bounds__(kRowLanes<T>) void residual_rms_kernel(
     const float* __restrict__ w, float eps, const T* __restrict__ scale, const T* __restrict__ shift,
     int64_t mod_stride, int L, T* __restrict__ out_h, T* __restrict__ out_y, int64_t os, int64_t N, int C) {
   constexpr int V = Vec<T>::N;
-  __shared__ float part[kRowLanes<T> / 64];
+  __shared__ __attribute__((aligned(16))) T squares[kRowLanes<T> * V];
   const int c0 = threadIdx.x * V;
   for (int64_t n = blockIdx.x; n < N; n += gridDim.x) {
     const int64_t b = static_cast<unsigned>(n) / static_cast<unsigned>(L);  // N <= 2^31
@@ -235,7 +243,6 @@ __global__ __launch_bounds__(kRowLanes<T>) void residual_rms_kernel(
         Vec<T>::load(shift + b * mod_stride + c0, t);
       }
     }
-    float ss = 0.f;
     if (c0 < C) {
       if (xbias) {
 #pragma unroll
@@ -255,15 +262,15 @@ __global__ __launch_bounds__(kRowLanes<T>) void residual_rms_kernel(
         for (int j = 0; j < V; ++j) r[j] = Vec<T>::round(r[j] + lv[j]);
       }
       Vec<T>::store(out_h + n * os + c0, r);
-#pragma unroll
-      for (int j = 0; j < V; ++j) ss = ss + r[j] * r[j];
     }
-    const float inv = rsqrtf(row_sum(ss, part) * (1.f / static_cast<float>(C)) + eps);
+    float ss = 0.f;
+    add_squares<T>(r, squares, ss);
+    const float inv = rsqrtf(wave_sum(ss) * (1.f / static_cast<float>(C)) + eps);
     if (c0 < C) {
       norm_chunk<T>(r, inv, wv, scale != nullptr, s, t);
       Vec<T>::store(out_y + n * os + c0, r);
     }
-    if (n + gridDim.x < N) __syncthreads();  // `part` is free again
+    if (n + gridDim.x < N) __syncthreads();  // `squares` is free again
   }
 }
 
