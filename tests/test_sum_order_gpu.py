@@ -7,9 +7,11 @@ with zeros in their place.
 """
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
+from hummingbird_amd import cross_attention as xattn
 from hummingbird_amd import elementwise
 
 pytestmark = pytest.mark.gpu
@@ -37,3 +39,26 @@ def test_row_norms_add_a_lane_s_chunks_in_order(channels):
         assert torch.equal(h, row)
         return torch.cat([plain, y[big]])
     assert torch.equal(norms(x), norms(ones))
+
+
+@pytest.mark.parametrize("length,heads,dim", [(100, 2, 64), (1000, 24, 64), (100, 2, 128)])
+def test_queries_add_their_squares_in_order(length, heads, dim):
+    """A query row is added dim by dim, by 64-query workgroups (one row per lane), 128-query ones (two) and at head_dim
+    128. Dim 0 is the one; its norm weight puts the normalised value just above a rounding midpoint (and a mean of
+    squares larger by 2^-19 / D would put it below), and the keys have no other dim."""
+    print(f"\n[case] query order L{length} H{heads} D{dim}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    bf16, width = torch.bfloat16, heads * dim
+    q = torch.full((1, length, 2 * width), TINY, device=DEV, dtype=bf16)
+    zeros = torch.zeros_like(q)
+    q[..., ::dim] = zeros[..., ::dim] = 1.0
+    assert float(q[0, 0, 1].float() ** 2) < 2.0 ** -24
+    kv = torch.zeros((1, 33, 3 * width), device=DEV, dtype=bf16)
+    kv[..., :width:dim] = torch.randn((1, 33, heads), generator=gen, device=DEV).to(bf16)  # k; k_diff weighs all alike
+    kv[..., 2 * width:] = torch.randn((1, 33, width), generator=gen, device=DEV).to(bf16)
+    weight = np.ones(dim)
+    weight[0] = (1 + 2.0 ** -8) * (1 + 2.0 ** -21) / np.sqrt(dim)
+    weight = torch.from_numpy(weight.astype(np.float32)).to(DEV)
+    context = xattn.prepare_cross_kv(kv, torch.ones(dim, device=DEV), heads, dim, 1e-6)
+    got = xattn.cross_attention(q, context, weight, 0.0)
+    assert torch.equal(got, xattn.cross_attention(zeros, context, weight, 0.0))
