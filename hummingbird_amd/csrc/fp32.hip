@@ -7,28 +7,30 @@
 // matrix cores (v_mfma_f32_32x32x16_f16, 16 times the rate of the fp32 ones) on operands split exactly enough not to
 // lose fp32 accuracy: x = hi + lo, hi = half(x), lo = half(x - hi), which leaves at most 2^-23 of x, and three products
 // lo hi + hi lo + hi hi (the lo lo one left out is below 2^-22 of the product at its largest, 2^-25 rms) accumulated in
-// fp32. An fp32 MFMA chain rounds its accumulator once per two dims; these round it three times per sixteen, so the
-// results are nearer to the 64-bit ones than the fp32 chain's were: relative error (2-norm) 6.4e-7 against 9.1e-7 on
-// dense B = 2, L = 1292, 8.4e-7 against 1.3e-6 at L = 2584, 7.0e-7 against 7.9e-7 on the band at w = 17 (24 heads, no
-// lambda), 1.2e-6 against 1.6e-6 at w = 100, 3.9e-7 against 5.4e-7 on the cross-attention. Times, whole calls against
-// the fp32 matrix cores fed through registers: dense (2, 1292, 24 heads) 534 -> 171 us, L = 2584 1565 -> 571, head_dim
-// 128 (2, 1292, 12 heads) 690 -> 166, cross (2, 2584 x 257) 205 -> 70, band S = 16384, w = 128 263 -> 133.
-// Three bf16 terms and six products, which need no scaling, were measured too: 290 us for the first of these. The
-// matrix cores slow down on such operands (about 27 ns per 32x32x16 product and SIMD), so the number of products sets
-// the time.
+// fp32. An fp32 MFMA chain rounds its accumulator once per two dims and key tile after key tile; these round it three
+// times per sixteen, and a tile's P V is added up apart, so the results are nearer to the 64-bit ones than the fp32
+// chain's were: relative error (2-norm) 3.3e-7 against 9.1e-7 on dense B = 2, L = 1292, 2.7e-7 against 5.4e-7 on the band
+// at S = 16384, w = 128. Times, whole calls against the fp32 matrix cores fed through registers: dense (2, 1292, 24
+// heads) 530 -> 188 us, L = 2584 1570 -> 599, head_dim 128 (2, 1292, 12 heads) 683 -> 171, cross (2, 2584 x 257) 204 ->
+// 74, band S = 16384, w = 128 468 -> 140. Three bf16 terms and six products, which need no scaling, were measured too:
+// 290 us for the first of these. The matrix cores slow down on such operands (about 27 ns per 32x32x16 product and SIMD),
+// so the number of products sets the time.
 //
 //   S^T[key][query] = K Q^T   A = K rows from LDS, B = q in registers
-//   P = exp2(S^T c - m)       m the running max of S^T c (online softmax), one FMA per score; masked scores are -inf
-//                             and give exactly 0
-//   O^T[d][query] += V^T P^T  A = V^T rows from LDS, B = P straight from the S^T accumulators
+//   P = exp2(S^T c - m)       m the max of the tile's S^T c, one FMA per score; masked scores are -inf and give exactly 0
+//   acc = V^T P^T             A = V^T rows from LDS, B = P straight from the S^T accumulators
+//   O^T[d][query] += acc      online softmax: one factor per query takes the tile's share to the running max
 //
 // Ranges. A half holds 2^-24 .. 65504, so every operand is scaled by powers of two (exact, undone in c and at the end):
 //   - dim d of the keys by 2^kx[d] and of the queries by 2^qx[d], chosen from the norm parameters alone, which bound a
 //     key's dim after RMSNorm, DyT and RoPE (see scale_table): each key dim fills the half range whatever its gain, and
 //     the query dim takes up the difference, so that the largest product bound over the dims fills it too. What falls
 //     below the range is below 2^-38 of the largest logit the parameters allow.
-//   - V by 2^-e per key tile, e from the tile's largest magnitude, stored with the tile; P by 2^(14 + e - E), E the
-//     largest e so far (O is rescaled when it grows, as for a growing maximum).
+//   - V by a power of two per key tile, from the tile's largest magnitude and stored with the tile. A tile whose keys or
+//     dims differ too much for that (VTile), or that holds an infinity or NaN, keeps its fp32 bits, and its P V runs on
+//     the fp32 matrix cores: every dim and every query has fp32 accuracy relative to its own size, whatever other values
+//     V holds.
+//   - P by 2^14, relative to the tile's own largest.
 //
 // Work split: a workgroup (4 waves) owns 64 queries of one (batch, head); waves 0-1 run branch 1 on 32 queries
 // each, waves 2-3 branch 2, and the branch-2 waves hand lam * O2 / l2 to the branch-1 waves through LDS. Keys
@@ -48,8 +50,8 @@ __device__ __forceinline__ void st4(float* p, f32x4 v) { *reinterpret_cast<f32x4
 // One key tile, the same bytes in LDS and in the workspace: K, K_diff and V, each a hi and a lo plane of KT x D halves.
 // K planes are [key][d], V planes V^T [d][position] in v_tile_key order; the 16-byte chunks of a row are XOR-swizzled,
 // so that the 16 rows that a pass of the operand reads takes fall in distinct banks.
-// D = 64: two stages (48 KB), three workgroups per CU (124 VGPRs). D = 128: one (48 KB), two workgroups per CU by
-// registers (196 VGPRs).
+// D = 64: two stages (48 KB), three workgroups per CU (156 VGPRs). D = 128: one (48 KB), two workgroups per CU by
+// registers (256 VGPRs).
 template <int D>
 struct SplitTile {
   static constexpr int KT = 32;
@@ -152,9 +154,52 @@ __device__ __forceinline__ void st_split(uint16_t* __restrict__ hi, int plane, c
   *reinterpret_cast<u32x4*>(hi + plane) = l;
 }
 
+// Reductions over 8 neighbouring lanes and over the wave without LDS (DPP and lane swaps); every lane gets the result.
+template <class Op>
+__device__ __forceinline__ uint32_t reduce8(uint32_t v, Op op) {
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, false));   // row_half_mirror: lanes i and 7 - i
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, false));    // quad_perm [1, 0, 3, 2]
+  return op(v, __builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, false));  // quad_perm [2, 3, 0, 1]
+}
+template <class Op>
+__device__ __forceinline__ uint32_t reduce64(uint32_t v, Op op) {
+  v = reduce8(v, op);
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, false));  // row_ror:8
+  const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  v = op(r[0], r[1]);
+  const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return op(h[0], h[1]);
+}
+struct MaxU32 {
+  __device__ uint32_t operator()(uint32_t a, uint32_t b) const { return a > b ? a : b; }
+};
+struct MinU32 {
+  __device__ uint32_t operator()(uint32_t a, uint32_t b) const { return a < b ? a : b; }
+};
+
+// The largest and smallest magnitudes of a V tile, as the bits of non-negative floats (which order as the floats do, with
+// infinities and then NaN last), collected in LDS by VTile::stats: of every key's row (over D / 64 waves), and the
+// smallest nonzero one of the 8-key pieces of dims.
+template <int D>
+struct VStats {
+  uint32_t rows[D / 64][SplitTile<D>::KT];
+  uint32_t cells[SplitTile<D>::VN * 4];
+};
+
 // V of one key tile in registers: a lane per dim, so that a wave's loads are whole rows and the transpose costs no
-// shuffle. The tile's exponent e (V 2^-e fills the half range) travels with the tile: its 8 bits (e + 128) replace the
-// lowest bits of the first 8 lo halves (dim 0, positions 0-7), a change below 2^-21 of those values' share.
+// shuffle. A tile is stored in one of two forms, told apart by the 8-bit code in it (v_code):
+//   - split: v 2^-e as hi + lo halves, the largest in [2^11, 2^12); code e + 128. What a half cannot hold costs up to
+//     2^-37 of the tile's largest value, so a tile takes this form only if every key and every 8-key piece of a dim has
+//     a value of at least 2^-12 of it (keys past the sequence aside, which no query weighs, and zero pieces): the error
+//     is then at most 2^-25 of any key's and any dim's own largest. A tile of zeros is exact.
+//   - wide: the fp32 bits, upper and lower halves in the two planes, for the fp32 matrix cores; code 0. Tiles with a key
+//     of zeros among others are wide too: a query may give that key nearly all of its weight, and then needs its small
+//     probabilities to fp32 accuracy, which P's halves have only near the tile's largest.
+// The code lies in the first 8 lo values (dim 0, positions 0-7), at bit 14 of each: a lo half is at most 1 there (half a
+// unit of a hi below 2^12), so that bit is free in a split tile; in a wide one it changes places with bit 0, which is
+// lost (those 8 values keep 23 bits).
+constexpr float kWideRange = 0x1p-12f;
+constexpr uint32_t kCodeBits = 0x40004000u;
 template <int D>
 struct VTile {
   using T = SplitTile<D>;
@@ -174,49 +219,100 @@ struct VTile {
       }
     }
   }
-  __device__ __forceinline__ float wave_amax() const {
-    float a = 0.f;
+  // This thread's share of `st`, which the workgroup may read after a barrier.
+  __device__ __forceinline__ void stats(VStats<D>& st) const {
+    const int lane = threadIdx.x & 63;
 #pragma unroll
-    for (int i = 0; i < T::VN; ++i)
+    for (int i = 0; i < T::VN; ++i) {
+      uint32_t m[8], cell = 0;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) a = fmaxf(a, fabsf(v[i][j]));
-    return wave_max(a);
+      for (int j = 0; j < 8; ++j) {
+        m[j] = __float_as_uint(v[i][j]) & 0x7fffffffu;
+        cell = m[j] > cell ? m[j] : cell;
+      }
+      // Over the wave's 64 dims: the first three steps halve the keys that a lane holds, the last three the dims.
+      const MaxU32 max;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const auto r = __builtin_amdgcn_permlane32_swap(m[j], m[j + 4], false, false);
+        m[j] = max(r[0], r[1]);
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const auto r = __builtin_amdgcn_permlane16_swap(m[j], m[j + 2], false, false);
+        m[j] = max(r[0], r[1]);
+      }
+      const bool up = lane & 8;
+      m[0] = max(up ? m[1] : m[0], __builtin_amdgcn_update_dpp(0, up ? m[0] : m[1], 0x128, 0xf, 0xf, false));
+      m[0] = reduce8(m[0], max);
+      cell = reduce64(cell ? cell : ~0u, MinU32());
+      const int at = threadIdx.x + 256 * i;  // lane l holds position 8 (at / D) + l / 8 of the wave's dims
+      if (lane % 8 == 0) st.rows[at % D / 64][8 * (at / D) + lane / 8] = m[0];
+      if (lane == 0) st.cells[4 * i + wave_id()] = cell;
+    }
   }
-  // `amax`: the tile's largest magnitude.
-  __device__ __forceinline__ void store(uint16_t* __restrict__ hi, float amax) const {
-    const int lead = static_cast<int>((__float_as_uint(amax) >> 23) & 255u) - 127;
-    const int e = (lead < -100 ? -100 : lead) - 13;  // -113 .. 115: V 2^-e is below 2^14
+  // The tile's code from `st`; `valid`: its keys before the end of the sequence. The same in every lane.
+  __device__ static __forceinline__ int code(const VStats<D>& st, int valid) {
+    const int lane = threadIdx.x & 63, pos = lane % T::KT;
+    uint32_t row = 0;
+#pragma unroll
+    for (int i = 0; i < D / 64; ++i) row = st.rows[i][pos] > row ? st.rows[i][pos] : row;
+    uint32_t least = st.cells[lane % (4 * T::VN)];
+    if (v_tile_key(pos) < valid && row < least) least = row;
+    const uint32_t amax = __builtin_amdgcn_readfirstlane(reduce64(row, MaxU32()));
+    const uint32_t amin = __builtin_amdgcn_readfirstlane(reduce64(least, MinU32()));
+    if (amax == 0) return 128;
+    const int lead = static_cast<int>(amax >> 23) - 127;
+    if (lead < -100 || lead > 127 || __uint_as_float(amin) < kWideRange * __uint_as_float(amax)) return 0;
+    return lead - 11 + 128;  // 17 .. 244
+  }
+  __device__ __forceinline__ void store(uint16_t* __restrict__ hi, int code) const {
 #pragma unroll
     for (int i = 0; i < T::VN; ++i) {
       const int at = threadIdx.x + 256 * i;
-      float y[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) y[j] = ldexpf(v[i][j], -e);
       u32x4 h, l;
-      split8(y, h, l);
-      if (i == 0 && threadIdx.x == 0) {
-        const uint32_t code = e + 128;
+      if (code) {
+        float y[8];
 #pragma unroll
-        for (int w = 0; w < 4; ++w)
-          l[w] = (l[w] & 0xfffefffeu) | ((code >> (2 * w)) & 1u) | (((code >> (2 * w + 1)) & 1u) << 16);
+        for (int j = 0; j < 8; ++j) y[j] = ldexpf(v[i][j], 128 - code);
+        split8(y, h, l);
+      } else {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          // a NaN whose payload lies in the bits that may be lost must stay one
+          const uint32_t x0 = __float_as_uint(v[i][2 * w] == v[i][2 * w] ? v[i][2 * w] : __uint_as_float(0x7fc00000u));
+          const uint32_t x1 =
+              __float_as_uint(v[i][2 * w + 1] == v[i][2 * w + 1] ? v[i][2 * w + 1] : __uint_as_float(0x7fc00000u));
+          h[w] = (x0 >> 16) | (x1 & 0xffff0000u);
+          l[w] = (x0 & 0xffffu) | (x1 << 16);
+        }
+      }
+      if (i == 0 && threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const uint32_t tag = (((code >> (2 * w)) & 1u) << 14) | (((code >> (2 * w + 1)) & 1u) << 30);
+          if (!code) l[w] = (l[w] & ~0x00010001u) | ((l[w] & kCodeBits) >> 14);
+          l[w] = (l[w] & ~kCodeBits) | tag;
+        }
       }
       uint16_t* dst = hi + T::v_at(at % D, at / D);
       *reinterpret_cast<u32x4*>(dst) = h;
       *reinterpret_cast<u32x4*>(dst + T::PLANE) = l;
     }
   }
-  // The exponent of the tile whose V hi plane is at `hi` in LDS, wave-uniform.
-  __device__ static __forceinline__ int exponent(const uint16_t* __restrict__ hi) {
-    const u32x4 l = lds16(hi + T::PLANE + T::v_at(0, 0));
-    uint32_t code = 0;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const uint32_t x = __builtin_amdgcn_readfirstlane(l[w]);
-      code |= ((x & 1u) | ((x >> 15) & 2u)) << (2 * w);
-    }
-    return static_cast<int>(code) - 128;
-  }
 };
+
+// The 8-bit code in bit 14 of the 8 halves at `p` in LDS, wave-uniform.
+__device__ __forceinline__ int read_code(const uint16_t* __restrict__ p) {
+  const u32x4 l = lds16(p);
+  uint32_t code = 0;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const uint32_t x = __builtin_amdgcn_readfirstlane(l[w]);
+    code |= (((x >> 14) & 1u) | ((x >> 29) & 2u)) << (2 * w);
+  }
+  return static_cast<int>(code);
+}
 
 // Copies tile t from the workspace into an LDS stage (byte address), 1 KB blocks by DMA, no registers.
 template <int D>
@@ -239,14 +335,12 @@ struct SplitCopy {
   }
 };
 
-// Online-softmax state of one wave: 32 queries (lane % 32) of one branch; O holds the sum of P V times
-// 2^(14 - E).
+// Online-softmax state of one wave: 32 queries (lane % 32) of one branch.
 template <int D>
 struct Branch {
   f32x16 o[D / 32];
   float l, m;
-  int E;
-  __device__ __forceinline__ Branch() : l(0.f), m(-INFINITY), E(-1000) {
+  __device__ __forceinline__ Branch() : l(0.f), m(-INFINITY) {
 #pragma unroll
     for (int dt = 0; dt < D / 32; ++dt) o[dt] = f32x16{};
   }
@@ -254,15 +348,20 @@ struct Branch {
 
 // One key tile for one wave. `sK`, `sV`: the hi planes of the branch's K and of V. `q`: this lane's query, hi and lo,
 // in MFMA B operand order (dims 16 kk + 8 lh .. +8). `masked` (wave-uniform): `valid(k)` says whether key k of the tile
-// takes part for this lane's query. The state is rescaled only when some lane's maximum or the V exponent moves (it
-// would multiply by exactly 1).
+// takes part for this lane's query.
+// The tile's probabilities are relative to its own largest logit (at most 1, and 1 somewhere), its products go into
+// accumulators of their own, and one factor per query then takes both to the state: so neither the halves of P nor the
+// power of two of V depends on what other tiles hold. That costs 16 FMAs per 32 dims: dense (2, 1292, 24 heads) 175 -> 187
+// us against products straight into O, and halves the error (6.2e-7 -> 3.3e-7); adding straight into O while a tile's
+// maximum and power of two are near the state's is 3 % faster and has neither that accuracy nor one path. The state is
+// rescaled only when some lane's maximum moves (it would multiply by exactly 1).
 template <int D, class Valid>
 __device__ __forceinline__ void attend_tile_f32(const uint16_t* __restrict__ sK, const uint16_t* __restrict__ sV,
                                                 const u32x4 (&q)[2][D / 16], Branch<D>& b, float c, bool masked,
                                                 Valid valid) {
   using T = SplitTile<D>;
   const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
-  const int e = VTile<D>::exponent(sV);
+  const int code = read_code(sV + T::PLANE + T::v_at(0, 0));
   f32x16 s = f32x16{};
   u32x4 kf[2][D / 16];  // all in flight before the first product: one wait for LDS instead of one per product pair
 #pragma unroll
@@ -284,37 +383,78 @@ __device__ __forceinline__ void attend_tile_f32(const uint16_t* __restrict__ sK,
   float mx = s[0];
 #pragma unroll
   for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
-  mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-  const float mnew = fmaxf(b.m, mx * c);
+  const float mt = fmaxf(mx, __shfl_xor(mx, 32, kWave)) * c;
+  const float mnew = fmaxf(b.m, mt);
   const float muse = mnew == -INFINITY ? 0.f : mnew;  // a query with no valid key so far keeps O = l = 0
-  const int En = e > b.E ? e : b.E;
-  if (En != b.E || __any(mnew != b.m)) {
-    const float alpha = fast_exp2(b.m - muse), beta = ldexpf(alpha, b.E - En);
+  if (__any(mnew != b.m)) {
+    const float alpha = fast_exp2(b.m - muse);
     b.l *= alpha;
 #pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt) b.o[dt] *= beta;
+    for (int dt = 0; dt < D / 32; ++dt) b.o[dt] *= alpha;
     b.m = mnew;
-    b.E = En;
   }
-  const float up = ldexpf(1.f, 14 + e - En);  // applied to P itself: in the exponent it would cost 4 bits of argument
+  const float beta = fast_exp2(mt - muse);        // 0 for a query with no valid key in the tile
+  const float mtile = mt == -INFINITY ? 0.f : mt;
+  float l = 0.f;
 #pragma unroll
-  for (int g = 0; g < 2; ++g) {  // 16 keys: their probabilities, then their products with V
-    float p[8];
+  for (int r = 0; r < 16; ++r) {
+    s[r] = fast_exp2(__fmaf_rn(s[r], c, -mtile));
+    l += s[r];
+  }
+  b.l = __fmaf_rn(l, beta, b.l);
+  auto add = [&](int dt, const f32x16& acc, float up) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      p[j] = fast_exp2(__fmaf_rn(s[8 * g + j], c, -muse));
-      b.l += p[j];
-      p[j] *= up;
+    for (int r = 0; r < 16; ++r) b.o[dt][r] = __fmaf_rn(acc[r], up, b.o[dt][r]);
+  };
+  if (code) {
+    u32x4 ph[2], pl[2];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      float p[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) p[j] = s[8 * g + j] * 0x1p14f;  // in the exponent it would cost 4 bits of argument
+      split8(p, ph[g], pl[g]);
     }
-    u32x4 ph, pl;
-    split8(p, ph, pl);
+    const float up = ldexpf(beta, code - 128 - 14);
+#pragma unroll
+    for (int d0 = 0; d0 < D / 32; d0 += 2) {
+      if constexpr (D == 128) __builtin_amdgcn_sched_barrier(0);  // no registers for the next pair's operands
+      f32x16 acc[2] = {};
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int at = T::v_at(32 * (d0 + i) + lr, 2 * g + lh);
+          const u32x4 hi = lds16(sV + at);
+          u32x4 lo = lds16(sV + T::PLANE + at);
+          if (g == 0 && d0 + i == 0) lo &= ~kCodeBits;  // the code's bit, clear in all other values
+          acc[i] = mfma_f16_32x32x16(lo, ph[g], acc[i]);
+          acc[i] = mfma_f16_32x32x16(hi, pl[g], acc[i]);
+          acc[i] = mfma_f16_32x32x16(hi, ph[g], acc[i]);
+        }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) add(d0 + i, acc[i], up);
+    }
+  } else {
 #pragma unroll
     for (int dt = 0; dt < D / 32; ++dt) {
-      const int at = T::v_at(32 * dt + lr, 2 * g + lh);
-      const u32x4 hi = lds16(sV + at), lo = lds16(sV + T::PLANE + at);
-      b.o[dt] = mfma_f16_32x32x16(lo, ph, b.o[dt]);
-      b.o[dt] = mfma_f16_32x32x16(hi, pl, b.o[dt]);
-      b.o[dt] = mfma_f16_32x32x16(hi, ph, b.o[dt]);
+      f32x16 acc = {};
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const int at = T::v_at(32 * dt + lr, 2 * g + lh);
+        const u32x4 hi = lds16(sV + at);
+        u32x4 lo = lds16(sV + T::PLANE + at);
+        if (g == 0 && dt == 0 && lane == 0) {
+#pragma unroll
+          for (int w = 0; w < 4; ++w) lo[w] = (lo[w] & ~(kCodeBits | 0x00010001u)) | ((lo[w] & 0x00010001u) << 14);
+        }
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          acc = mfma_f32_32x32x2(__uint_as_float((hi[w] << 16) | (lo[w] & 0xffffu)), s[8 * g + 2 * w], acc);
+          acc = mfma_f32_32x32x2(__uint_as_float((hi[w] & 0xffff0000u) | (lo[w] >> 16)), s[8 * g + 2 * w + 1], acc);
+        }
+      }
+      add(dt, acc, beta);
     }
   }
 }
@@ -327,7 +467,7 @@ __device__ __forceinline__ void store_diff_f32(uint16_t* __restrict__ stages, co
   float* smem = reinterpret_cast<float*>(stages);
   const int lane = threadIdx.x & 63, lh = lane >> 5, wave = wave_id();
   const int slot0 = (wave & 1) * (D / 32) * 16;
-  const float inv = ldexpf(__frcp_rn(b.l + __shfl_xor(b.l, 32, kWave)), b.E - 14);
+  const float inv = __frcp_rn(b.l + __shfl_xor(b.l, 32, kWave));
   if (br == 1) {
     const float i1 = __fmul_rn(lamh, inv);
 #pragma unroll
@@ -360,19 +500,15 @@ __device__ __forceinline__ void store_v_tiles(const float* __restrict__ V, int64
   using T = SplitTile<D>;
   constexpr int NT = 64 / T::KT;
   __shared__ __attribute__((aligned(16))) uint16_t image[NT * T::TENSOR];
-  __shared__ float amax[NT][4];
+  __shared__ VStats<D> st[NT];
   VTile<D> v[NT];
 #pragma unroll
   for (int i = 0; i < NT; ++i) v[i].fetch(V, pitch, l0 + T::KT * i, end, mask);
 #pragma unroll
-  for (int i = 0; i < NT; ++i) {
-    const float a = v[i].wave_amax();
-    if ((threadIdx.x & 63) == 0) amax[i][wave_id()] = a;
-  }
+  for (int i = 0; i < NT; ++i) v[i].stats(st[i]);
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < NT; ++i)
-    v[i].store(image + i * T::TENSOR, fmaxf(fmaxf(amax[i][0], amax[i][1]), fmaxf(amax[i][2], amax[i][3])));
+  for (int i = 0; i < NT; ++i) v[i].store(image + i * T::TENSOR, VTile<D>::code(st[i], end - (l0 + T::KT * i)));
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < NT * T::TENSOR / 8 / 256; ++i) {
@@ -701,9 +837,10 @@ __global__ __launch_bounds__(256) void band_keys_f32(const float* __restrict__ q
 }
 
 // WS: the key tiles that meet the block's band come from the workspace of band_keys_f32; otherwise each query block
-// prepares its own from qkv.
+// prepares its own from qkv, with one workgroup less per CU: the preparation's registers would spill (S = 16384, w = 128,
+// 8 x 64: 317 -> 286 us; 4 x 128, w = 300: 614 us spilling, 627 not).
 template <int D, bool WS>
-__global__ __launch_bounds__(256, SplitTile<D>::OCC) void band_attend_f32(
+__global__ __launch_bounds__(256, WS ? SplitTile<D>::OCC : SplitTile<D>::OCC - 1) void band_attend_f32(
     const float* __restrict__ qkv, int64_t rs, int B, int S, int Sp, int H, int w, const float* __restrict__ qdyt,
     const float* __restrict__ kdyt, const float* __restrict__ cosT, const float* __restrict__ sinT, int half,
     const float* __restrict__ ws, int64_t region, const float* __restrict__ lam, float* __restrict__ out) {
@@ -744,19 +881,18 @@ __global__ __launch_bounds__(256, SplitTile<D>::OCC) void band_attend_f32(
     const SplitCopy<D> copy(ws, region, static_cast<int64_t>(bh) * Sp);
     stream_tiles<D>(copy, t_lo, t_hi, smem, attend);
   } else {
-    __shared__ float amax[4];
+    __shared__ VStats<D> st;
     const DytPair<D> kp(kdyt, half);
     for (int t = t_lo; t < t_hi; ++t) {
       VTile<D> v;
       v.fetch(xb + 2 * HD, rs, t * T::KT, S, nullptr);
-      const float a = v.wave_amax();
-      if (lane == 0) amax[wave] = a;
+      v.stats(st);
       band_rows_f32<D, T::KT>(xb, rs, HD, 4 * HD, t * T::KT, S, half, kp, cosT, sinT,
                               [&](int tsr, int r, int g, const float (&x)[8]) {
                                 st_split(smem + tsr * T::TENSOR + T::k_at(r, g), T::PLANE, x, scale.k + 8 * g);
                               });
       __syncthreads();
-      v.store(smem + 2 * T::TENSOR, fmaxf(fmaxf(amax[0], amax[1]), fmaxf(amax[2], amax[3])));
+      v.store(smem + 2 * T::TENSOR, VTile<D>::code(st, S - t * T::KT));
       __syncthreads();
       attend(smem, t);
       __syncthreads();
