@@ -22,10 +22,10 @@
 //   O^T[d][query] += acc      online softmax: one factor per query takes the tile's share to the running max
 //
 // Ranges. A half holds 2^-24 .. 65504, so every operand is scaled by powers of two (exact, undone in c and at the end):
-//   - dim d of the keys by 2^kx[d] and of the queries by 2^qx[d], chosen from the norm parameters alone, which bound a
-//     key's dim after RMSNorm, DyT and RoPE (see scale_table): each key dim fills the half range whatever its gain, and
-//     the query dim takes up the difference, so that the largest product bound over the dims fills it too. What falls
-//     below the range is below 2^-38 of the largest logit the parameters allow.
+//   - dim d of the keys by 2^k[d] and of the queries by 2^q[d], from the norm parameters (scale_table), so that gains of
+//     many magnitudes leave no dim out; then each key tile and each query row by a power of two from its own largest
+//     value, so that neither tables that are no rotation nor norms far below their bounds leave the half range. What a half
+//     cannot hold is below 2^-37 of a tile's largest key value and 2^-39 of a row's largest query value, so scaled.
 //   - V by a power of two per key tile, from the tile's largest magnitude and stored with the tile. A tile whose keys or
 //     dims differ too much for that (VTile), or that holds an infinity or NaN, keeps its fp32 bits, and its P V runs on
 //     the fp32 matrix cores: every dim and every query has fp32 accuracy relative to its own size, whatever other values
@@ -100,10 +100,9 @@ __device__ __forceinline__ int bound_exp(float b) {
   return e < -100 ? -100 : e > 100 ? 100 : e;
 }
 
-// Powers of two for the operand dims: a key's dim d goes to the matrix cores times 2^k[d], a query's times 2^q[d], and
-// the logit is the product sum times 2^logit. `kb(d)`, `qb(d)`: bounds of dim d before RoPE, which mixes dims d and
-// d +- half (each stays below sqrt(2) times the larger bound). Key: below 2^14.5. Query: eq + ek <= emax, so below
-// 2^13.5.
+// Powers of two for the operand dims, from the norm parameters: a key's dim d is taken times 2^k[d], a query's times
+// 2^q[d], and the logit is the product sum times 2^logit; the products of no dim exceed those of another because of its
+// gains then. `kb(d)`, `qb(d)`: bounds of dim d before RoPE, which mixes dims d and d +- half.
 struct ScaleTable {
   int k[128], q[128], logit;
 };
@@ -126,10 +125,10 @@ __device__ __forceinline__ void scale_table(ScaleTable& t, int half, KBound kb, 
   if (threadIdx.x < 64) {
 #pragma unroll
     for (int i = 0; i < D / 64; ++i) {
-      t.k[lane + 64 * i] = 13 - ek[i];
-      t.q[lane + 64 * i] = ek[i] + 12 - emax;
+      t.k[lane + 64 * i] = -ek[i];
+      t.q[lane + 64 * i] = ek[i] - emax;
     }
-    if (lane == 0) t.logit = emax - 25;
+    if (lane == 0) t.logit = emax;
   }
   __syncthreads();
 }
@@ -143,15 +142,33 @@ __device__ __forceinline__ auto dyt_bound(const float* __restrict__ dyt) {
   return [dyt](int d) { return fabsf(dyt[1 + d]) + fabsf(dyt[1 + D + d]); };
 }
 
-// The 8 dims of group g, scaled and split, into chunk `at` of a hi plane and of the lo plane `plane` halves on.
-__device__ __forceinline__ void st_split(uint16_t* __restrict__ hi, int plane, const float (&x)[8], const int* exps) {
+// Exponent of the leading bit of the largest magnitude `amax` (its bits) of operands scaled by a ScaleTable, at least
+// -100. An infinite one (gains or tables) must not cost the finite ones beside it their place: they are about 1 or less.
+__device__ __forceinline__ int lead_exp(uint32_t amax) {
+  const int e = static_cast<int>(amax >> 23) - 127;
+  return e < -100 ? -100 : e > 127 ? 1 : e;
+}
+__device__ __forceinline__ uint32_t amax8(const float (&x)[8]) {
+  float a = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) a = fmaxf(a, fabsf(x[j]));  // passes over NaN
+  return __float_as_uint(a);
+}
+
+// 8 values times 2^up, split, into a hi chunk and the lo chunk `plane` halves on; `edit(l)` may change the lo ones first.
+template <class Edit>
+__device__ __forceinline__ void st_split(uint16_t* __restrict__ hi, int plane, const float (&x)[8], int up, Edit edit) {
   float y[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) y[j] = ldexpf(x[j], exps[j]);
+  for (int j = 0; j < 8; ++j) y[j] = ldexpf(x[j], up);
   u32x4 h, l;
   split8(y, h, l);
+  edit(l);
   *reinterpret_cast<u32x4*>(hi) = h;
   *reinterpret_cast<u32x4*>(hi + plane) = l;
+}
+__device__ __forceinline__ void st_split(uint16_t* __restrict__ hi, int plane, const float (&x)[8], int up) {
+  st_split(hi, plane, x, up, [](u32x4&) {});
 }
 
 // Reductions over 8 neighbouring lanes and over the wave without LDS (DPP and lane swaps); every lane gets the result.
@@ -200,6 +217,11 @@ struct VStats {
 // lost (those 8 values keep 23 bits).
 constexpr float kWideRange = 0x1p-12f;
 constexpr uint32_t kCodeBits = 0x40004000u;
+constexpr int kCodeKey = 16;  // the row of a K tile that holds its code (KeyRows)
+// The bits of `code` for values 2 w and 2 w + 1.
+__device__ __forceinline__ uint32_t code_bits(int code, int w) {
+  return (((code >> (2 * w)) & 1u) << 14) | (((code >> (2 * w + 1)) & 1u) << 30);
+}
 template <int D>
 struct VTile {
   using T = SplitTile<D>;
@@ -290,9 +312,8 @@ struct VTile {
       if (i == 0 && threadIdx.x == 0) {
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
-          const uint32_t tag = (((code >> (2 * w)) & 1u) << 14) | (((code >> (2 * w + 1)) & 1u) << 30);
           if (!code) l[w] = (l[w] & ~0x00010001u) | ((l[w] & kCodeBits) >> 14);
-          l[w] = (l[w] & ~kCodeBits) | tag;
+          l[w] = (l[w] & ~kCodeBits) | code_bits(code, w);
         }
       }
       uint16_t* dst = hi + T::v_at(at % D, at / D);
@@ -347,7 +368,8 @@ struct Branch {
 };
 
 // One key tile for one wave. `sK`, `sV`: the hi planes of the branch's K and of V. `q`: this lane's query, hi and lo,
-// in MFMA B operand order (dims 16 kk + 8 lh .. +8). `masked` (wave-uniform): `valid(k)` says whether key k of the tile
+// in MFMA B operand order (dims 16 kk + 8 lh .. +8); the logit is the product sum times 2^(n + the K tile's code).
+// `masked` (wave-uniform): `valid(k)` says whether key k of the tile
 // takes part for this lane's query.
 // The tile's probabilities are relative to its own largest logit (at most 1, and 1 somewhere), its products go into
 // accumulators of their own, and one factor per query then takes both to the state: so neither the halves of P nor the
@@ -357,11 +379,13 @@ struct Branch {
 // rescaled only when some lane's maximum moves (it would multiply by exactly 1).
 template <int D, class Valid>
 __device__ __forceinline__ void attend_tile_f32(const uint16_t* __restrict__ sK, const uint16_t* __restrict__ sV,
-                                                const u32x4 (&q)[2][D / 16], Branch<D>& b, float c, bool masked,
+                                                const u32x4 (&q)[2][D / 16], Branch<D>& b, int n, bool masked,
                                                 Valid valid) {
   using T = SplitTile<D>;
   const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
   const int code = read_code(sV + T::PLANE + T::v_at(0, 0));
+  const float c =
+      ldexpf(kLog2e / sqrtf(static_cast<float>(D)), n + read_code(sK + T::PLANE + T::k_at(kCodeKey, 0)) - 128);
   f32x16 s = f32x16{};
   u32x4 kf[2][D / 16];  // all in flight before the first product: one wait for LDS instead of one per product pair
 #pragma unroll
@@ -371,7 +395,9 @@ __device__ __forceinline__ void attend_tile_f32(const uint16_t* __restrict__ sK,
   if constexpr (D == 64) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int kk = 0; kk < D / 16; ++kk) {
-    const u32x4 hi = kf[0][kk], lo = kf[1][kk];
+    const u32x4 hi = kf[0][kk];
+    u32x4 lo = kf[1][kk];
+    if (kk == 0) lo &= ~kCodeBits;
     s = mfma_f16_32x32x16(lo, q[0][kk], s);
     s = mfma_f16_32x32x16(hi, q[1][kk], s);
     s = mfma_f16_32x32x16(hi, q[0][kk], s);
@@ -492,15 +518,86 @@ __device__ __forceinline__ void store_diff_f32(uint16_t* __restrict__ stages, co
   }
 }
 
-// The workspace's V^T tiles of the 64 keys from l0, by the whole workgroup: through LDS, so that the stores are whole
-// lines. `ws`: the first of the 64 rows in the V region.
+// The split forms of k and k_diff of ROWS keys (32-key tiles), a (row, RoPE group pair) per thread and pass as
+// rms_rows_f32 and band_rows_f32 hand them out: scaled by the ScaleTable as they come (`take`), then, when the workgroup
+// has found each tile's largest magnitude (`stats`, a barrier), by the tile's own power of two, so that the largest lies in
+// [2^11, 2^12) whatever the norms, the tables and the inputs made of it. What a half cannot hold is below 2^-37 of it.
+// The tile's code (its power of two + 128) lies in bit 14 of the first 8 lo values of key kCodeKey, which is free there
+// as in a split V tile.
+template <int D, int ROWS>
+struct KeyRows {
+  using T = SplitTile<D>;
+  static constexpr int PAIRS = D / 16, TASKS = (ROWS * PAIRS + 255) / 256, PARTS = 4 * TASKS;
+  static constexpr int PER_TILE = PAIRS / 2;  // waves (and passes) that share a tile's rows
+  struct Stats {
+    uint32_t part[2][PARTS];
+  };
+  float y[TASKS][2][2][8] = {};
+  int m1 = 0, m2 = 0;
+  __device__ __forceinline__ void take(const ScaleTable& scale, int tsr, int i, int g1, const float (&x1)[8], int g2,
+                                       const float (&x2)[8]) {
+    m1 = g1;
+    m2 = g2;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      y[i][tsr][0][j] = ldexpf(x1[j], scale.k[8 * g1 + j]);
+      y[i][tsr][1][j] = ldexpf(x2[j], scale.k[8 * g2 + j]);
+    }
+  }
+  __device__ __forceinline__ void stats(Stats& st) const {
+    const MaxU32 max;
+#pragma unroll
+    for (int i = 0; i < TASKS; ++i)
+#pragma unroll
+      for (int tsr = 0; tsr < 2; ++tsr) {
+        const uint32_t a = reduce64(max(amax8(y[i][tsr][0]), amax8(y[i][tsr][1])), max);
+        if ((threadIdx.x & 63) == 0) st.part[tsr][4 * i + wave_id()] = a;
+      }
+  }
+  // `planes(tensor, tile)`: the hi plane of a tile.
+  template <class Planes>
+  __device__ __forceinline__ void store(const Stats& st, Planes planes) const {
+    if (ROWS * PAIRS < 256 && threadIdx.x >= ROWS * PAIRS) return;
+#pragma unroll
+    for (int i = 0; i < TASKS; ++i) {
+      const int row = (threadIdx.x + 256 * i) / PAIRS, tile = row / T::KT, r = row % T::KT;
+#pragma unroll
+      for (int tsr = 0; tsr < 2; ++tsr) {
+        uint32_t amax = 0;
+#pragma unroll
+        for (int w = 0; w < PER_TILE; ++w) amax = MaxU32()(amax, st.part[tsr][PER_TILE * tile + w]);
+        const int up = 11 - lead_exp(amax);
+        uint16_t* hi = planes(tsr, tile);
+        st_split(hi + T::k_at(r, m1), T::PLANE, y[i][tsr][0], up, [&](u32x4& l) {
+          if (r == kCodeKey && m1 == 0) add_code(l, 128 - up);
+        });
+        st_split(hi + T::k_at(r, m2), T::PLANE, y[i][tsr][1], up);
+      }
+    }
+  }
+  // Puts a code into 8 split values. Only the lo halves of infinities and NaNs may have the bit set; they may lose it.
+  __device__ static __forceinline__ void add_code(u32x4& l, int code) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) l[w] = (l[w] & ~kCodeBits) | code_bits(code, w);
+  }
+};
+
+// The workspace's K, K_diff and V^T tiles of the 64 keys from l0, by the whole workgroup; V^T through LDS, so that the
+// stores are whole lines. `ws`: the first of the 64 rows in the K region.
 template <int D>
-__device__ __forceinline__ void store_v_tiles(const float* __restrict__ V, int64_t pitch, int l0, int end,
-                                              const float* __restrict__ mask, float* __restrict__ ws) {
+__device__ __forceinline__ void store_tiles(const KeyRows<D, 64>& keys, const float* __restrict__ V, int64_t pitch, int l0,
+                                            int end, const float* __restrict__ mask, float* __restrict__ ws,
+                                            int64_t region) {
   using T = SplitTile<D>;
   constexpr int NT = 64 / T::KT;
   __shared__ __attribute__((aligned(16))) uint16_t image[NT * T::TENSOR];
   __shared__ VStats<D> st[NT];
+  __shared__ typename KeyRows<D, 64>::Stats kst;
+  keys.stats(kst);
+  __syncthreads();
+  keys.store(kst, [&](int tsr, int tile) {
+    return reinterpret_cast<uint16_t*>(ws + tsr * region) + tile * T::TENSOR;
+  });
   VTile<D> v[NT];
 #pragma unroll
   for (int i = 0; i < NT; ++i) v[i].fetch(V, pitch, l0 + T::KT * i, end, mask);
@@ -513,21 +610,15 @@ __device__ __forceinline__ void store_v_tiles(const float* __restrict__ V, int64
 #pragma unroll
   for (int i = 0; i < NT * T::TENSOR / 8 / 256; ++i) {
     const int at = 8 * (threadIdx.x + 256 * i);
-    st16(reinterpret_cast<uint16_t*>(ws) + at, lds16(image + at));
+    st16(reinterpret_cast<uint16_t*>(ws + 2 * region) + at, lds16(image + at));
   }
 }
 
-// Where the hi chunk of row r (0..63) and group g of a 64-row block lies among the block's K tiles.
-template <int D>
-__device__ __forceinline__ int k_block_at(int r, int g) {
-  using T = SplitTile<D>;
-  return r / T::KT * T::TENSOR + T::k_at(r % T::KT, g);
-}
-
 // RMSNorm (dit.py:45-57) and rotate-half RoPE (dit.py:90-98) in fp32 of two tensors (row offsets offA, offB) for the
-// ROWS positions from pos0 (of the batch whose rows start at `xb`): `sink(tensor, row, group, values)` takes each 8-dim
-// group; positions at or past L give zeros. One (row, RoPE group pair) per thread and pass: the rotation partner of
-// every dim is in the thread's own registers; the mean of squares is reduced over the D / 16 lanes of a row.
+// ROWS positions from pos0 (of the batch whose rows start at `xb`): `sink(tensor, pass, row, group, values, group,
+// values)` takes the two 8-dim groups; positions at or past L give zeros. One (row, RoPE group pair) per thread and pass:
+// the rotation partner of every dim is in the thread's own registers; the mean of squares is reduced over the D / 16 lanes
+// of a row, neighbours in one wave.
 template <int D, int ROWS, class Sink>
 __device__ __forceinline__ void rms_rows_f32(const float* __restrict__ xb, int64_t rs, int64_t offA, int64_t offB,
                                              int pos0, int L, int half, const float* __restrict__ w, float eps,
@@ -583,27 +674,42 @@ __device__ __forceinline__ void rms_rows_f32(const float* __restrict__ xb, int64
         o1[j] = in ? r1 : 0.f;
         o2[j] = in ? r2 : 0.f;
       }
-      sink(tsr, r, m1, o1);
-      sink(tsr, r, m2, o2);
+      sink(tsr, i, r, m1, o1, m2, o2);
     }
   }
 }
 
 // The split q and q_diff of the workgroup's 64 queries, through LDS in passes of 64 rows (32 at head_dim 128):
-// `rows(r0, sink)` prepares the pass that starts at row r0. Ends with a barrier, the stages free.
+// `rows(r0, sink)` prepares the pass that starts at row r0. Besides the ScaleTable's, each row of each branch has a power
+// of two of its own, from its largest magnitude (then in [2^13, 2^14)). Returns the power of two of this lane's logits
+// but for the key tile's. Ends with a barrier, the stages free.
 template <int D>
 constexpr int kQueryRows = 4096 / D;
 template <int D, class Rows>
-__device__ __forceinline__ void queries_f32(const ScaleTable& scale, uint16_t* __restrict__ smem,
-                                            u32x4 (&qf)[2][D / 16], Rows rows) {
-  constexpr int ROWS = kQueryRows<D>, PLANE = 4096;
+__device__ __forceinline__ int queries_f32(const ScaleTable& scale, uint16_t* __restrict__ smem,
+                                           u32x4 (&qf)[2][D / 16], Rows rows) {
+  constexpr int ROWS = kQueryRows<D>, PLANE = 4096, PAIRS = D / 16;
+  __shared__ int lead[2][64];
   static_assert(4 * PLANE <= SplitTile<D>::ELEMS, "q and q_diff of one pass must fit in the stages");
   const int lane = threadIdx.x & 63, wave = wave_id(), lr = lane & 31, lh = lane >> 5;
   const int row = (wave & 1) * 32 + lr;
-#pragma unroll
+#pragma unroll 1
   for (int r0 = 0; r0 < 64; r0 += ROWS) {
-    rows(r0, [&](int tsr, int r, int g, const float (&x)[8]) {
-      st_split(smem + 2 * tsr * PLANE + swz<D>(r, g), PLANE, x, scale.q + 8 * g);
+    rows(r0, [&](int tsr, int, int r, int g1, const float (&x1)[8], int g2, const float (&x2)[8]) {
+      float y1[8], y2[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        y1[j] = ldexpf(x1[j], scale.q[8 * g1 + j]);
+        y2[j] = ldexpf(x2[j], scale.q[8 * g2 + j]);
+      }
+      const MaxU32 max;
+      uint32_t a = max(amax8(y1), amax8(y2));
+#pragma unroll
+      for (int off = 1; off < PAIRS; off <<= 1) a = max(a, __shfl_xor(a, off, kWave));
+      const int e = lead_exp(a);
+      if (threadIdx.x % PAIRS == 0) lead[tsr][r0 + r] = e;
+      st_split(smem + 2 * tsr * PLANE + swz<D>(r, g1), PLANE, y1, 13 - e);
+      st_split(smem + 2 * tsr * PLANE + swz<D>(r, g2), PLANE, y2, 13 - e);
     });
     __syncthreads();
     if (row / ROWS == r0 / ROWS) {  // wave-uniform
@@ -615,6 +721,7 @@ __device__ __forceinline__ void queries_f32(const ScaleTable& scale, uint16_t* _
     }
     __syncthreads();
   }
+  return scale.logit + lead[wave >> 1][row] - 13;
 }
 
 // k and k_diff after RMSNorm and RoPE and V * mask for 64 tokens of one head into the workspace's tiles.
@@ -631,12 +738,12 @@ __global__ __launch_bounds__(256) void dense_prep_f32(const float* __restrict__ 
   const float* xb = qkv + static_cast<int64_t>(b) * L * rs + h * D;
   float* block = ws + (bh * Lp + l0) * D;
   scale_table<D>(scale, half, rms_bound<D>(kw), [](int) { return 1.f; });  // only the key's part is used here
+  KeyRows<D, 64> keys;
   rms_rows_f32<D, 64>(xb, rs, sk * HD, skd * HD, l0, L, half, kw, eps, cosT, sinT,
-                      [&](int tsr, int r, int g, const float (&x)[8]) {
-                        uint16_t* dst = reinterpret_cast<uint16_t*>(block + tsr * region) + k_block_at<D>(r, g);
-                        st_split(dst, SplitTile<D>::PLANE, x, scale.k + 8 * g);
+                      [&](int tsr, int i, int, int g1, const float (&x1)[8], int g2, const float (&x2)[8]) {
+                        keys.take(scale, tsr, i, g1, x1, g2, x2);
                       });
-  store_v_tiles<D>(xb + sv * HD, rs, l0, L, vmask ? vmask + static_cast<int64_t>(b) * L : nullptr, block + 2 * region);
+  store_tiles<D>(keys, xb + sv * HD, rs, l0, L, vmask ? vmask + static_cast<int64_t>(b) * L : nullptr, block, region);
 }
 
 // The key tiles [t_lo, t_hi) through the stages: `attend(stage, t)` for each.
@@ -690,16 +797,15 @@ __global__ __launch_bounds__(256, SplitTile<D>::OCC) void dense_attend_f32(
 
   u32x4 qf[2][D / 16];
   const float* xb = qkv + static_cast<int64_t>(b) * L * rs + h * D;
-  queries_f32<D>(scale, smem, qf, [&](int r0, auto sink) {
+  const int n = queries_f32<D>(scale, smem, qf, [&](int r0, auto sink) {
     rms_rows_f32<D, kQueryRows<D>>(xb, rs, 0, static_cast<int64_t>(sqd) * H * D, qb * 64 + r0, L, half, qw, eps, cosT,
                                    sinT, sink);
   });
   Branch<D> state;
-  const float c = ldexpf(kLog2e / sqrtf(static_cast<float>(D)), scale.logit);
   // Keys past Lk are zeros in the workspace (Lkp is a multiple of 128).
   const SplitCopy<D> copy(ws, region, static_cast<int64_t>(bh) * Lkp);
   stream_tiles<D>(copy, 0, (Lk + T::KT - 1) / T::KT, smem, [&](const uint16_t* s, int t) {
-    attend_tile_f32<D>(s + br * T::TENSOR, s + 2 * T::TENSOR, qf, state, c, (t + 1) * T::KT > Lk,
+    attend_tile_f32<D>(s + br * T::TENSOR, s + 2 * T::TENSOR, qf, state, n, (t + 1) * T::KT > Lk,
                        [&](int k) { return t * T::KT + k < Lk; });
   });
   float* orow = q < L ? out + (static_cast<int64_t>(b) * L + q) * (static_cast<int64_t>(H) * D) + h * D : nullptr;
@@ -757,8 +863,7 @@ struct DytPair {
 };
 
 // DyT (same_l.py:58-69) and RoPE (same_l.py:92-100) in fp32 of two tensors (row offsets offA, offB) for the ROWS
-// positions from pos0: `sink(tensor, row, group, values)` takes each 8-dim group; positions outside [0, S) give zeros.
-// One (row, RoPE group pair) per thread and pass: the rotation partner of every dim is in the thread's own registers,
+// positions from pos0: `sink` as in rms_rows_f32; positions outside [0, S) give zeros. One (row, RoPE group pair) per thread and pass: the rotation partner of every dim is in the thread's own registers,
 // and the pass's 16-byte loads are all issued before its arithmetic. Measured at S = 16384, 8 heads of 64: the key
 // kernel 199.6 -> 42.0 us (201 MB at the rate of a large copy) against the library tanhf with the parameters read per
 // element.
@@ -808,8 +913,7 @@ __device__ __forceinline__ void band_rows_f32(const float* __restrict__ xb, int6
           o1[j] = in ? r1 : 0.f;
           o2[j] = in ? r2 : 0.f;
         }
-      sink(tsr, r, dp.m1, o1);
-      sink(tsr, r, dp.m2, o2);
+      sink(tsr, i, r, dp.m1, o1, dp.m2, o2);
     }
   }
 }
@@ -828,12 +932,12 @@ __global__ __launch_bounds__(256) void band_keys_f32(const float* __restrict__ q
   const float* xb = qkv + static_cast<int64_t>(b) * S * rs + h * D;
   float* block = ws + (bh * Sp + 64 * t) * D;
   scale_table<D>(scale, half, dyt_bound<D>(kdyt), [](int) { return 1.f; });  // only the key's part is used here
+  KeyRows<D, 64> keys;
   band_rows_f32<D, 64>(xb, rs, HD, 4 * HD, 64 * t, S, half, DytPair<D>(kdyt, half), cosT, sinT,
-                       [&](int tsr, int r, int g, const float (&x)[8]) {
-                         uint16_t* dst = reinterpret_cast<uint16_t*>(block + tsr * region) + k_block_at<D>(r, g);
-                         st_split(dst, SplitTile<D>::PLANE, x, scale.k + 8 * g);
+                       [&](int tsr, int i, int, int g1, const float (&x1)[8], int g2, const float (&x2)[8]) {
+                         keys.take(scale, tsr, i, g1, x1, g2, x2);
                        });
-  store_v_tiles<D>(xb + 2 * HD, rs, 64 * t, S, nullptr, block + 2 * region);
+  store_tiles<D>(keys, xb + 2 * HD, rs, 64 * t, S, nullptr, block, region);
 }
 
 // WS: the key tiles that meet the block's band come from the workspace of band_keys_f32; otherwise each query block
@@ -856,15 +960,15 @@ __global__ __launch_bounds__(256, WS ? SplitTile<D>::OCC : SplitTile<D>::OCC - 1
 
   scale_table<D>(scale, half, dyt_bound<D>(kdyt), dyt_bound<D>(qdyt));
   u32x4 qf[2][D / 16];
+  int n;
   {
     const DytPair<D> dp(qdyt, half);
-    queries_f32<D>(scale, smem, qf, [&](int r0, auto sink) {
+    n = queries_f32<D>(scale, smem, qf, [&](int r0, auto sink) {
       band_rows_f32<D, kQueryRows<D>>(xb, rs, 0, 3 * HD, q0 + r0, S, half, dp, cosT, sinT, sink);
     });
   }
 
   Branch<D> state;
-  const float c = ldexpf(kLog2e / sqrtf(static_cast<float>(D)), scale.logit);
   const int t_lo = (q0 - w > 0 ? q0 - w : 0) / T::KT;
   const int t_hi = ((q0 + 64 + w < S ? q0 + 64 + w : S) + T::KT - 1) / T::KT;
   auto attend = [&](const uint16_t* s, int t) {
@@ -872,7 +976,7 @@ __global__ __launch_bounds__(256, WS ? SplitTile<D>::OCC : SplitTile<D>::OCC - 1
     // the tile reaches this wave's band, and lies inside the band of every one of its queries
     if (k0 > qw0 + 31 + w || k1 < qw0 - w) return;
     const bool inside = k1 <= qw0 + w && k0 >= qw0 + 31 - w && k1 < S;
-    attend_tile_f32<D>(s + br * T::TENSOR, s + 2 * T::TENSOR, qf, state, c, !inside, [&](int k) {
+    attend_tile_f32<D>(s + br * T::TENSOR, s + 2 * T::TENSOR, qf, state, n, !inside, [&](int k) {
       const int kk = k0 + k, dist = kk - q;
       return kk < S && dist <= w && -dist <= w;
     });
@@ -882,16 +986,20 @@ __global__ __launch_bounds__(256, WS ? SplitTile<D>::OCC : SplitTile<D>::OCC - 1
     stream_tiles<D>(copy, t_lo, t_hi, smem, attend);
   } else {
     __shared__ VStats<D> st;
+    __shared__ typename KeyRows<D, T::KT>::Stats kst;
     const DytPair<D> kp(kdyt, half);
     for (int t = t_lo; t < t_hi; ++t) {
       VTile<D> v;
       v.fetch(xb + 2 * HD, rs, t * T::KT, S, nullptr);
       v.stats(st);
+      KeyRows<D, T::KT> keys;
       band_rows_f32<D, T::KT>(xb, rs, HD, 4 * HD, t * T::KT, S, half, kp, cosT, sinT,
-                              [&](int tsr, int r, int g, const float (&x)[8]) {
-                                st_split(smem + tsr * T::TENSOR + T::k_at(r, g), T::PLANE, x, scale.k + 8 * g);
+                              [&](int tsr, int i, int, int g1, const float (&x1)[8], int g2, const float (&x2)[8]) {
+                                keys.take(scale, tsr, i, g1, x1, g2, x2);
                               });
+      keys.stats(kst);
       __syncthreads();
+      keys.store(kst, [&](int tsr, int) { return smem + tsr * T::TENSOR; });
       v.store(smem + 2 * T::TENSOR, VTile<D>::code(st, S - t * T::KT));
       __syncthreads();
       attend(smem, t);

@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from hummingbird_amd import band_attention as ba
+from hummingbird_amd import dense_attention as da
 from hummingbird_amd import workloads
 from tests import test_band_gpu as band
 from tests import test_cross_gpu as cross
@@ -120,6 +121,39 @@ def test_cross_v_spike_costs_its_own_dim_only(spike):
     with np.errstate(invalid="ignore", over="ignore"):
         ref = cross.oracle(inp, "fp32")
     check_dims(cross.run_hip(inp, torch.float32)[0], ref[0], {3}, f"spike {spike}")
+
+
+@pytest.mark.parametrize("size", [2.0 ** -20, 4.0, 64.0])
+@pytest.mark.parametrize("dim", [64, 128])
+def test_dense_tables_of_any_size(dim, size):
+    """Tables times a power of two (a scaled rotary embedding) over all dims, with gains divided by it: exactly the results
+    of plain tables and gains, however far the operands are from what the gains bound."""
+    print(f"\n[case] fp32 dense tables x {size} D{dim}", flush=True)
+    inp = workloads.dense_inputs(1, 100, 2, dim, seed=18, dtype="fp32", half=dim // 2)
+    ref = dense.oracle(inp, "xla", compute="fp32")
+    small = dict(inp, q_weight=inp["q_weight"] / np.float32(size), k_weight=inp["k_weight"] / np.float32(size))
+    qkv, freq = torch.from_numpy(inp["qkv"]).to("cuda"), torch.from_numpy(inp["inv_freq"]).to("cuda")
+    cos, sin, mask = da.tables(100, freq, torch.from_numpy(inp["valid"]).to("cuda"), dim, torch.float32)
+    got = da.dense_attention(qkv, *(torch.from_numpy(small[n]).to("cuda") for n in ("q_weight", "k_weight")), cos * size,
+                             sin * size, mask, 2, dim, dim // 2, inp["eps"], lam=torch.from_numpy(inp["lam"]).to("cuda"))
+    assert_fp32_parity(got.cpu().numpy(), ref, f"tables x {size}")
+
+
+@pytest.mark.parametrize("workspace", [True, False], ids=["ws", "no-ws"])
+@pytest.mark.parametrize("power", [10, 20, 30])
+def test_band_dyt_far_below_its_bound(power, workspace):
+    """alpha 2^-power with gamma 2^power: keys and queries of ordinary size, 2^-power of what gamma bounds."""
+    print(f"\n[case] fp32 band DyT power {power} ws {workspace}", flush=True)
+    inp = workloads.band_inputs(1, 150, 2, 64, 40, seed=19, dtype="fp32", half=16, alpha=2.0 ** -power,
+                                gamma_mean=2.0 ** power)
+    ref = band.oracle(inp, "xla", compute="fp32")
+    cap = ba.FP32_WORKSPACE_CAP
+    try:
+        ba.FP32_WORKSPACE_CAP = cap if workspace else 0
+        got = band.run_hip(inp, dtype=torch.float32)
+    finally:
+        ba.FP32_WORKSPACE_CAP = cap
+    check_rows(got[0], ref[0], set(), f"power {power}")
 
 
 def test_identical_branches_cancel_in_split_and_wide_tiles():
