@@ -22,7 +22,7 @@ from hummingbird_amd.dense_attention import SUPPORTED_HEAD_DIMS, _f32_vector, _r
 class CrossKV:
     """The prepared context of one block: k, k_diff (normed) and v in the kernel-native layout."""
     workspace: torch.Tensor  # uint8, hb_cross_workspace_size bytes
-    k_weight: torch.Tensor   # (D,) fp32: bounds the logits in the attention kernel
+    k_weight: torch.Tensor   # (D,) fp32: bounds the logits of 16-bit calls (its largest magnitude is used)
     dtype: torch.dtype
     batch: int
     length: int              # Nk context tokens

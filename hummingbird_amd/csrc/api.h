@@ -75,7 +75,7 @@ int launch_dense_attend_16bit(hipStream_t stream, int dtype, const void* q, int6
 int launch_dense_prep_f32(hipStream_t stream, const void* qkv, int64_t rs, int sk, int skd, int sv, const float* kw,
                           const float* cosT, const float* sinT, int half, const float* vmask, int B, int L, int H,
                           int D, float eps, const DenseLayout& lay, void* ws);
-int launch_dense_attend_f32(hipStream_t stream, const void* qkv, int64_t rs, int sqd, const float* qw, const float* kw,
+int launch_dense_attend_f32(hipStream_t stream, const void* qkv, int64_t rs, int sqd, const float* qw,
                             const float* cosT, const float* sinT, int half, float eps, const void* ws, const float* lam,
                             void* out, int B, int L, int Lk, int H, int D, const DenseLayout& lay);
 // Streaming band kernel (band_ring.hip): bf16 or half, D = 64, half % 8 == 0, window <= 128. Arguments are

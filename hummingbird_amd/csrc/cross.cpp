@@ -115,8 +115,8 @@ int hb_cross_attend(hipStream_t stream, const void* q, int dtype, int64_t row_st
   }
   if (dtype == HB_F32) {
     if (reinterpret_cast<uintptr_t>(out) % 16) return fail(HB_ERR_STRIDE, "fp32 out must be 16-byte aligned");
-    return launch_dense_attend_f32(stream, q, row_stride, kQdSec, q_weight, k_weight, nullptr, nullptr, 0, eps, workspace,
-                                   lam, out, B, L, Nk, H, D, lay);
+    return launch_dense_attend_f32(stream, q, row_stride, kQdSec, q_weight, nullptr, nullptr, 0, eps, workspace, lam,
+                                   out, B, L, Nk, H, D, lay);
   }
   if (reinterpret_cast<uintptr_t>(out) % 8) return fail(HB_ERR_STRIDE, "out must be 8-byte aligned");
   return launch_dense_attend_16bit(stream, dtype, q, row_stride, kQdSec, q_weight, k_weight, nullptr, nullptr, 0, eps, lam,

@@ -485,8 +485,8 @@ extern "C" int hb_dense_attend(hipStream_t stream, const void* qkv, int dtype, i
   if (st) return st;
   if ((st = out_checks(qkv, dtype, row_stride, out, B, L, H, D, workspace, lay))) return st;
   if (dtype == HB_F32)
-    return launch_dense_attend_f32(stream, qkv, row_stride, kSecQd, q_weight, k_weight, cos, sin, half, eps, workspace,
-                                   lam, out, B, L, L, H, D, lay);
+    return launch_dense_attend_f32(stream, qkv, row_stride, kSecQd, q_weight, cos, sin, half, eps, workspace, lam, out,
+                                   B, L, L, H, D, lay);
   return launch_dense_attend_16bit(stream, dtype, qkv, row_stride, kSecQd, q_weight, k_weight, cos, sin, half, eps, lam,
                                    out, B, L, L, H, D, lay, workspace);
 }

@@ -106,15 +106,24 @@ __device__ __forceinline__ int bound_exp(float b) {
 struct ScaleTable {
   int k[128], q[128], logit;
 };
-template <int D, class KBound, class QBound>
-__device__ __forceinline__ void scale_table(ScaleTable& t, int half, KBound kb, QBound qb) {
+// The keys' part, before a barrier.
+template <int D, class KBound>
+__device__ __forceinline__ void key_scales(ScaleTable& t, int half, KBound kb) {
+  for (int d = threadIdx.x; d < D; d += 256) {
+    const int p = d < half ? d + half : d < 2 * half ? d - half : d;
+    t.k[d] = -bound_exp(fmaxf(kb(d), kb(p)));
+  }
+}
+// The queries' part, for the keys' in `t`, after a barrier and before one.
+template <int D, class QBound>
+__device__ __forceinline__ void query_scales(ScaleTable& t, int half, QBound qb) {
   const int lane = threadIdx.x & 63;
-  int ek[D / 64], emax = -1000;
+  if (threadIdx.x >= 64) return;
+  int emax = -1000;
 #pragma unroll
   for (int i = 0; i < D / 64; ++i) {
     const int d = lane + 64 * i, p = d < half ? d + half : d < 2 * half ? d - half : d;
-    ek[i] = bound_exp(fmaxf(kb(d), kb(p)));
-    const int e = bound_exp(fmaxf(qb(d), qb(p))) + ek[i];
+    const int e = bound_exp(fmaxf(qb(d), qb(p))) - t.k[d];
     emax = e > emax ? e : emax;
   }
 #pragma unroll
@@ -122,15 +131,9 @@ __device__ __forceinline__ void scale_table(ScaleTable& t, int half, KBound kb, 
     const int other = __shfl_xor(emax, off, kWave);
     emax = other > emax ? other : emax;
   }
-  if (threadIdx.x < 64) {
 #pragma unroll
-    for (int i = 0; i < D / 64; ++i) {
-      t.k[lane + 64 * i] = -ek[i];
-      t.q[lane + 64 * i] = ek[i] - emax;
-    }
-    if (lane == 0) t.logit = emax;
-  }
-  __syncthreads();
+  for (int i = 0; i < D / 64; ++i) t.q[lane + 64 * i] = -t.k[lane + 64 * i] - emax;
+  if (lane == 0) t.logit = emax;
 }
 // After RMSNorm |x_d| <= sqrt(D) |w_d|; |DyT(x)_d| <= |gamma_d| + |beta_d| (`dyt` = [alpha, gamma, beta]).
 template <int D>
@@ -523,7 +526,8 @@ __device__ __forceinline__ void store_diff_f32(uint16_t* __restrict__ stages, co
 // has found each tile's largest magnitude (`stats`, a barrier), by the tile's own power of two, so that the largest lies in
 // [2^11, 2^12) whatever the norms, the tables and the inputs made of it. What a half cannot hold is below 2^-37 of it.
 // The tile's code (its power of two + 128) lies in bit 14 of the first 8 lo values of key kCodeKey, which is free there
-// as in a split V tile.
+// as in a split V tile. So do the powers of two of the dims (128 - k), for the calls that attend to keys which another
+// call prepared: bit r of dim d's in key r < 8 of the first tile of k (`scales` not null).
 template <int D, int ROWS>
 struct KeyRows {
   using T = SplitTile<D>;
@@ -556,7 +560,7 @@ struct KeyRows {
   }
   // `planes(tensor, tile)`: the hi plane of a tile.
   template <class Planes>
-  __device__ __forceinline__ void store(const Stats& st, Planes planes) const {
+  __device__ __forceinline__ void store(const Stats& st, const ScaleTable* scales, Planes planes) const {
     if (ROWS * PAIRS < 256 && threadIdx.x >= ROWS * PAIRS) return;
 #pragma unroll
     for (int i = 0; i < TASKS; ++i) {
@@ -568,12 +572,23 @@ struct KeyRows {
         for (int w = 0; w < PER_TILE; ++w) amax = MaxU32()(amax, st.part[tsr][PER_TILE * tile + w]);
         const int up = 11 - lead_exp(amax);
         uint16_t* hi = planes(tsr, tile);
+        const bool dims = scales && tsr == 0 && row < 8;
         st_split(hi + T::k_at(r, m1), T::PLANE, y[i][tsr][0], up, [&](u32x4& l) {
           if (r == kCodeKey && m1 == 0) add_code(l, 128 - up);
+          if (dims) add_code(l, scale_bits(*scales, m1, row));
         });
-        st_split(hi + T::k_at(r, m2), T::PLANE, y[i][tsr][1], up);
+        st_split(hi + T::k_at(r, m2), T::PLANE, y[i][tsr][1], up, [&](u32x4& l) {
+          if (dims) add_code(l, scale_bits(*scales, m2, row));
+        });
       }
     }
+  }
+  // Bit r of the codes of group g's dims.
+  __device__ static __forceinline__ int scale_bits(const ScaleTable& scales, int g, int r) {
+    int bits = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) bits |= (((128 - scales.k[8 * g + j]) >> r) & 1) << j;
+    return bits;
   }
   // Puts a code into 8 split values. Only the lo halves of infinities and NaNs may have the bit set; they may lose it.
   __device__ static __forceinline__ void add_code(u32x4& l, int code) {
@@ -585,9 +600,9 @@ struct KeyRows {
 // The workspace's K, K_diff and V^T tiles of the 64 keys from l0, by the whole workgroup; V^T through LDS, so that the
 // stores are whole lines. `ws`: the first of the 64 rows in the K region.
 template <int D>
-__device__ __forceinline__ void store_tiles(const KeyRows<D, 64>& keys, const float* __restrict__ V, int64_t pitch, int l0,
-                                            int end, const float* __restrict__ mask, float* __restrict__ ws,
-                                            int64_t region) {
+__device__ __forceinline__ void store_tiles(const KeyRows<D, 64>& keys, const ScaleTable* scales,
+                                            const float* __restrict__ V, int64_t pitch, int l0, int end,
+                                            const float* __restrict__ mask, float* __restrict__ ws, int64_t region) {
   using T = SplitTile<D>;
   constexpr int NT = 64 / T::KT;
   __shared__ __attribute__((aligned(16))) uint16_t image[NT * T::TENSOR];
@@ -595,7 +610,7 @@ __device__ __forceinline__ void store_tiles(const KeyRows<D, 64>& keys, const fl
   __shared__ typename KeyRows<D, 64>::Stats kst;
   keys.stats(kst);
   __syncthreads();
-  keys.store(kst, [&](int tsr, int tile) {
+  keys.store(kst, scales, [&](int tsr, int tile) {
     return reinterpret_cast<uint16_t*>(ws + tsr * region) + tile * T::TENSOR;
   });
   VTile<D> v[NT];
@@ -737,19 +752,21 @@ __global__ __launch_bounds__(256) void dense_prep_f32(const float* __restrict__ 
   const int64_t HD = static_cast<int64_t>(H) * D, bh = static_cast<int64_t>(b) * H + h;
   const float* xb = qkv + static_cast<int64_t>(b) * L * rs + h * D;
   float* block = ws + (bh * Lp + l0) * D;
-  scale_table<D>(scale, half, rms_bound<D>(kw), [](int) { return 1.f; });  // only the key's part is used here
+  key_scales<D>(scale, half, rms_bound<D>(kw));
+  __syncthreads();
   KeyRows<D, 64> keys;
   rms_rows_f32<D, 64>(xb, rs, sk * HD, skd * HD, l0, L, half, kw, eps, cosT, sinT,
                       [&](int tsr, int i, int, int g1, const float (&x1)[8], int g2, const float (&x2)[8]) {
                         keys.take(scale, tsr, i, g1, x1, g2, x2);
                       });
-  store_tiles<D>(keys, xb + sv * HD, rs, l0, L, vmask ? vmask + static_cast<int64_t>(b) * L : nullptr, block, region);
+  store_tiles<D>(keys, l0 == 0 ? &scale : nullptr, xb + sv * HD, rs, l0, L,
+                 vmask ? vmask + static_cast<int64_t>(b) * L : nullptr, block, region);
 }
 
-// The key tiles [t_lo, t_hi) through the stages: `attend(stage, t)` for each.
-template <int D, class Attend>
+// The key tiles [t_lo, t_hi) through the stages: `attend(stage, t)` for each, after `first(stage)` for the first one.
+template <int D, class First, class Attend>
 __device__ __forceinline__ void stream_tiles(const SplitCopy<D>& copy, int t_lo, int t_hi,
-                                             uint16_t* __restrict__ smem, Attend attend) {
+                                             uint16_t* __restrict__ smem, First first, Attend attend) {
   using T = SplitTile<D>;
   const uint32_t ldsA = lds_addr(smem);
   if constexpr (T::STAGES == 2) {
@@ -759,6 +776,7 @@ __device__ __forceinline__ void stream_tiles(const SplitCopy<D>& copy, int t_lo,
     copy(t_lo, ldsA);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
+    first(smem);
     for (int t = t_lo; t < t_hi; t += 2) {
       if (t + 1 < t_hi) copy(t + 1, ldsB);
       attend(smem, t);
@@ -775,6 +793,7 @@ __device__ __forceinline__ void stream_tiles(const SplitCopy<D>& copy, int t_lo,
       copy(t, ldsA);
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
+      if (t == t_lo) first(smem);
       attend(smem, t);
       __syncthreads();
     }
@@ -783,7 +802,7 @@ __device__ __forceinline__ void stream_tiles(const SplitCopy<D>& copy, int t_lo,
 
 template <int D>
 __global__ __launch_bounds__(256, SplitTile<D>::OCC) void dense_attend_f32(
-    const float* __restrict__ qkv, int64_t rs, int sqd, const float* __restrict__ qw, const float* __restrict__ kw,
+    const float* __restrict__ qkv, int64_t rs, int sqd, const float* __restrict__ qw,
     const float* __restrict__ cosT, const float* __restrict__ sinT, int half, float eps, const float* __restrict__ ws,
     int64_t region, int B, int L, int Lk, int Lkp, int H, const float* __restrict__ lam, float* __restrict__ out) {
   using T = SplitTile<D>;
@@ -793,7 +812,17 @@ __global__ __launch_bounds__(256, SplitTile<D>::OCC) void dense_attend_f32(
   const int tile = xcd_remap(blockIdx.x, B * H * nqb);
   const int qb = tile % nqb, bh = tile / nqb, h = bh % H, b = bh / H;
   const int wave = wave_id(), br = wave >> 1, q = qb * 64 + (wave & 1) * 32 + (threadIdx.x & 31);
-  scale_table<D>(scale, half, rms_bound<D>(kw), rms_bound<D>(qw));
+  // The powers of two that the preparation gave the keys' dims, from its own k_weight (KeyRows).
+  for (int d = threadIdx.x; d < D; d += 256) {
+    const uint16_t* lo = reinterpret_cast<const uint16_t*>(ws + static_cast<int64_t>(bh) * Lkp * D) + T::PLANE;
+    int code = 0;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) code |= ((lo[T::k_at(r, d / 8) + d % 8] >> 14) & 1) << r;
+    scale.k[d] = 128 - code;
+  }
+  __syncthreads();
+  query_scales<D>(scale, half, rms_bound<D>(qw));
+  __syncthreads();
 
   u32x4 qf[2][D / 16];
   const float* xb = qkv + static_cast<int64_t>(b) * L * rs + h * D;
@@ -804,7 +833,13 @@ __global__ __launch_bounds__(256, SplitTile<D>::OCC) void dense_attend_f32(
   Branch<D> state;
   // Keys past Lk are zeros in the workspace (Lkp is a multiple of 128).
   const SplitCopy<D> copy(ws, region, static_cast<int64_t>(bh) * Lkp);
-  stream_tiles<D>(copy, 0, (Lk + T::KT - 1) / T::KT, smem, [&](const uint16_t* s, int t) {
+  auto clear = [&](uint16_t* s) {  // the dims' powers of two leave the first tile
+    const int d = 4 * (threadIdx.x % (D / 4)), step = 256 / (D / 4);
+    for (int r = threadIdx.x / (D / 4); r < 8; r += step)
+      *reinterpret_cast<u32x2*>(s + T::PLANE + T::k_at(r, d / 8) + d % 8) &= ~kCodeBits;
+    __syncthreads();
+  };
+  stream_tiles<D>(copy, 0, (Lk + T::KT - 1) / T::KT, smem, clear, [&](const uint16_t* s, int t) {
     attend_tile_f32<D>(s + br * T::TENSOR, s + 2 * T::TENSOR, qf, state, n, (t + 1) * T::KT > Lk,
                        [&](int k) { return t * T::KT + k < Lk; });
   });
@@ -931,13 +966,14 @@ __global__ __launch_bounds__(256) void band_keys_f32(const float* __restrict__ q
   const int64_t HD = static_cast<int64_t>(H) * D, bh = static_cast<int64_t>(b) * H + h;
   const float* xb = qkv + static_cast<int64_t>(b) * S * rs + h * D;
   float* block = ws + (bh * Sp + 64 * t) * D;
-  scale_table<D>(scale, half, dyt_bound<D>(kdyt), [](int) { return 1.f; });  // only the key's part is used here
+  key_scales<D>(scale, half, dyt_bound<D>(kdyt));
+  __syncthreads();
   KeyRows<D, 64> keys;
   band_rows_f32<D, 64>(xb, rs, HD, 4 * HD, 64 * t, S, half, DytPair<D>(kdyt, half), cosT, sinT,
                        [&](int tsr, int i, int, int g1, const float (&x1)[8], int g2, const float (&x2)[8]) {
                          keys.take(scale, tsr, i, g1, x1, g2, x2);
                        });
-  store_tiles<D>(keys, xb + 2 * HD, rs, 64 * t, S, nullptr, block, region);
+  store_tiles<D>(keys, nullptr, xb + 2 * HD, rs, 64 * t, S, nullptr, block, region);
 }
 
 // WS: the key tiles that meet the block's band come from the workspace of band_keys_f32; otherwise each query block
@@ -958,7 +994,10 @@ __global__ __launch_bounds__(256, WS ? SplitTile<D>::OCC : SplitTile<D>::OCC - 1
   const int64_t HD = static_cast<int64_t>(H) * D;
   const float* xb = qkv + static_cast<int64_t>(b) * S * rs + h * D;
 
-  scale_table<D>(scale, half, dyt_bound<D>(kdyt), dyt_bound<D>(qdyt));
+  key_scales<D>(scale, half, dyt_bound<D>(kdyt));
+  __syncthreads();
+  query_scales<D>(scale, half, dyt_bound<D>(qdyt));
+  __syncthreads();
   u32x4 qf[2][D / 16];
   int n;
   {
@@ -983,7 +1022,7 @@ __global__ __launch_bounds__(256, WS ? SplitTile<D>::OCC : SplitTile<D>::OCC - 1
   };
   if constexpr (WS) {  // every tile's rows lie below Sp: Sp is a multiple of 128 and k0 < S
     const SplitCopy<D> copy(ws, region, static_cast<int64_t>(bh) * Sp);
-    stream_tiles<D>(copy, t_lo, t_hi, smem, attend);
+    stream_tiles<D>(copy, t_lo, t_hi, smem, [](uint16_t*) {}, attend);
   } else {
     __shared__ VStats<D> st;
     __shared__ typename KeyRows<D, T::KT>::Stats kst;
@@ -999,7 +1038,7 @@ __global__ __launch_bounds__(256, WS ? SplitTile<D>::OCC : SplitTile<D>::OCC - 1
                               });
       keys.stats(kst);
       __syncthreads();
-      keys.store(kst, [&](int tsr, int) { return smem + tsr * T::TENSOR; });
+      keys.store(kst, nullptr, [&](int tsr, int) { return smem + tsr * T::TENSOR; });
       v.store(smem + 2 * T::TENSOR, VTile<D>::code(st, S - t * T::KT));
       __syncthreads();
       attend(smem, t);
@@ -1032,7 +1071,7 @@ int launch_dense_prep_f32(hipStream_t stream, const void* qkv, int64_t rs, int s
   return launched("dense_prep_f32");
 }
 
-int launch_dense_attend_f32(hipStream_t stream, const void* qkv, int64_t rs, int sqd, const float* qw, const float* kw,
+int launch_dense_attend_f32(hipStream_t stream, const void* qkv, int64_t rs, int sqd, const float* qw,
                             const float* cosT, const float* sinT, int half, float eps, const void* ws, const float* lam,
                             void* out, int B, int L, int Lk, int H, int D, const DenseLayout& lay) {
   const int nblocks = B * H * ((L + 63) / 64);
@@ -1041,7 +1080,7 @@ int launch_dense_attend_f32(hipStream_t stream, const void* qkv, int64_t rs, int
   float* o = static_cast<float*>(out);
   const int Lkp = static_cast<int>(lay.Lp);
   auto attend = D == 64 ? dense_attend_f32<64> : dense_attend_f32<128>;
-  hipLaunchKernelGGL(attend, dim3(nblocks), dim3(256), 0, stream, x, rs, sqd, qw, kw, cosT, sinT, half, eps, w,
+  hipLaunchKernelGGL(attend, dim3(nblocks), dim3(256), 0, stream, x, rs, sqd, qw, cosT, sinT, half, eps, w,
                      lay.region_elems, B, L, Lk, Lkp, H, lam, o);
   return launched("dense_attend_f32");
 }

@@ -127,7 +127,8 @@ int hb_dense_prep(hipStream_t stream, const void* qkv, int dtype, int64_t row_st
                   const float* vmask, int B, int L, int H, int D, float eps, void* workspace,
                   size_t workspace_bytes);
 /* Stage 2: RMSNorm + RoPE of q and q_diff (read from the same qkv), both softmax attentions and the
- * subtraction, against a workspace that hb_dense_prep filled from this qkv. Arguments as hb_dense_diffattn. */
+ * subtraction, against a workspace that hb_dense_prep filled from this qkv. Arguments as hb_dense_diffattn; k_weight
+ * bounds the logits for 16-bit inputs and is not read for HB_F32. */
 int hb_dense_attend(hipStream_t stream, const void* qkv, int dtype, int64_t row_stride,
                     const float* q_weight, const float* k_weight, const float* cos, const float* sin, int half,
                     const float* lam, void* out, int B, int L, int H, int D, float eps,
@@ -219,7 +220,9 @@ int hb_band_diffattn(hipStream_t stream, const void* qkv, int dtype, int64_t row
  *   workspace : >= hb_cross_workspace_size(dtype, B, Nk, H, D) bytes, 256-byte aligned.
  * hb_cross_prep writes the prepared k, k_diff and v of the context into the workspace; hb_cross_attend reads
  * them, for as many query sets as the caller has (the reference computes them once per clip and reuses them in
- * every sampler step). k_weight is passed to hb_cross_attend too: it bounds the logits for the softmax. */
+ * every sampler step). k_weight is passed to hb_cross_attend too: with 16-bit inputs its largest magnitude bounds the
+ * logits for the softmax (any vector with at least that of the one that prepared the keys will do); HB_F32 does not read
+ * it. */
 size_t hb_cross_workspace_size(int dtype, int B, int Nk, int H, int D);
 int hb_cross_validate(int dtype, int64_t q_row_stride, int64_t kv_row_stride, int B, int L, int Nk, int H, int D,
                       float eps);

@@ -2,11 +2,15 @@
 holds, against the oracle at the fp32 contract taken dim by dim and row by row (not relative to the largest output)."""
 from __future__ import annotations
 
+import dataclasses
+
 import numpy as np
 import pytest
 import torch
 
+from hummingbird_amd import _lib
 from hummingbird_amd import band_attention as ba
+from hummingbird_amd import cross_attention as xattn
 from hummingbird_amd import dense_attention as da
 from hummingbird_amd import workloads
 from tests import test_band_gpu as band
@@ -154,6 +158,50 @@ def test_band_dyt_far_below_its_bound(power, workspace):
     finally:
         ba.FP32_WORKSPACE_CAP = cap
     check_rows(got[0], ref[0], set(), f"power {power}")
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1, 2, 64), (2, 100, 77, 2, 64), (1, 70, 128, 2, 128)],
+                         ids=lambda s: "B%dL%dNk%dH%dD%d" % s)
+@pytest.mark.parametrize("other", ["larger", "uneven"])
+def test_cross_attend_reads_the_scales_that_the_preparation_used(shape, other):
+    """The k_weight that hb_cross_attend gets only bounds the logits: another one, or the same storage edited after the
+    preparation, does not change the fp32 results."""
+    print(f"\n[case] fp32 cross other k_weight {shape} {other}", flush=True)
+    b, length, nk, h, d = shape
+    inp = workloads.cross_inputs(b, length, nk, h, d, seed=20, dtype="fp32")
+    q, kv = (torch.from_numpy(inp[n]).to("cuda") for n in ("q", "kv"))
+    qw, kw = (torch.from_numpy(inp[n]).to("cuda") for n in ("q_weight", "k_weight"))
+    lam = torch.from_numpy(inp["lam"]).to("cuda")
+    context = xattn.prepare_cross_kv(kv, kw, h, d, inp["eps"])
+    ref = xattn.cross_attention(q, context, qw, inp["eps"], lam=lam)
+    assert_fp32_parity(ref.cpu().numpy(), cross.oracle(inp, "fp32"), f"cross {shape}")
+    factor = 8.0 if other == "larger" else 2.0 ** torch.arange(d, device="cuda").remainder(7)
+    bound = dataclasses.replace(context, k_weight=kw * factor)
+    assert torch.equal(xattn.cross_attention(q, bound, qw, inp["eps"], lam=lam), ref)
+    kw *= factor
+    assert torch.equal(xattn.cross_attention(q, context, qw, inp["eps"], lam=lam), ref)
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+def test_dense_stages_share_no_k_weight(dim):
+    """hb_dense_attend with another k_weight than hb_dense_prep: the keys are those that were prepared."""
+    print(f"\n[case] fp32 dense stages D{dim}", flush=True)
+    h, length, half = 2, 150, dim // 4
+    inp = workloads.dense_inputs(1, length, h, dim, seed=21, dtype="fp32", half=half)
+    dev = {n: torch.from_numpy(inp[n]).to("cuda") for n in ("qkv", "q_weight", "k_weight", "inv_freq", "valid", "lam")}
+    cos, sin, mask = da.tables(length, dev["inv_freq"], dev["valid"], dim, torch.float32)
+    workspace = torch.empty(da.workspace_bytes(torch.float32, 1, length, h, dim), dtype=torch.uint8, device="cuda")
+    out = torch.empty((1, length, h * dim), device="cuda")
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+
+    def args(k_weight):
+        return (stream, dev["qkv"].data_ptr(), _lib.HB_F32, 5 * h * dim, dev["q_weight"].data_ptr(), k_weight.data_ptr(),
+                cos.data_ptr(), sin.data_ptr(), half)
+    shape = (1, length, h, dim, inp["eps"], workspace.data_ptr(), workspace.numel())
+    _lib.check(lib.hb_dense_prep(*args(dev["k_weight"]), mask.data_ptr(), *shape), "prep")
+    for weight in (dev["k_weight"], dev["k_weight"] * 2.0 ** torch.arange(dim, device="cuda").remainder(5)):
+        _lib.check(lib.hb_dense_attend(*args(weight), dev["lam"].data_ptr(), out.data_ptr(), *shape), "attend")
+        assert_fp32_parity(out.cpu().numpy(), dense.oracle(inp, "xla", compute="fp32"), f"stages D{dim}")
 
 
 def test_identical_branches_cancel_in_split_and_wide_tiles():
