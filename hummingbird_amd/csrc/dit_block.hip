@@ -71,32 +71,90 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
-// A row per workgroup, one 16-byte chunk per lane (rows of up to kRowLanes chunks; longer ones take more turns), for
-// the norms. A DiT evaluation has one to a few thousand rows, so one wave per row left a SIMD with one or two waves
-// and a serial walk over three chunks: latency, not bytes, was the time. residual_rms on 1422 rows of 1536 bf16
-// values, in the denoiser: 10.5 -> 8.7 us (17.5 MB; 3.7 us at a large copy's rate).
+// One wave per row: the mean of squares over the row (fp32), then the normalised row scaled by `w` (fp32), cast,
+// and with `scale` the modulation by the row's batch entry of `scale` / `shift` (`mod_stride` elements apart per
+// batch, `L` rows per batch). The row is read twice; the second read hits the cache. A row per workgroup, as in
+// residual_rms_kernel, is slower here from a few thousand rows on (1536 bf16 values: 8.8 against 9.6 us at 4096 rows,
+// 23.4 against 26.7 at 16384) and 0.7 us faster at 1422.
+template <typename T>
+__global__ __launch_bounds__(256) void rms_modulate_kernel(const T* __restrict__ x, int64_t xs,
+                                                           const float* __restrict__ w, float eps,
+                                                           const T* __restrict__ scale, const T* __restrict__ shift,
+                                                           int64_t mod_stride, int L, T* __restrict__ out, int64_t os,
+                                                           int64_t N, int C) {
+  constexpr int V = Vec<T>::N;
+  const int lane = threadIdx.x & 63;
+  const int64_t n = static_cast<int64_t>(blockIdx.x) * 4 + wave_id();
+  if (n >= N) return;  // wave-uniform
+  const T* row = x + n * xs;
+  float ss = 0.f;
+  for (int c0 = lane * V; c0 < C; c0 += 64 * V) {
+    float v[V];
+    Vec<T>::load(row + c0, v);
+#pragma unroll
+    for (int j = 0; j < V; ++j) ss = ss + v[j] * v[j];
+  }
+  const float inv = rsqrtf(wave_sum(ss) * (1.f / static_cast<float>(C)) + eps);
+  const int64_t b = n / L;
+  const T* sc = scale ? scale + b * mod_stride : nullptr;
+  const T* sh = shift ? shift + b * mod_stride : nullptr;
+  T* orow = out + n * os;
+  for (int c0 = lane * V; c0 < C; c0 += 64 * V) {
+    float v[V];
+    Vec<T>::load(row + c0, v);
+#pragma unroll
+    for (int j = 0; j < V; ++j) v[j] = Vec<T>::round((v[j] * inv) * w[c0 + j]);
+    if (sc) {
+      float s[V], t[V];
+      Vec<T>::load(sc + c0, s);
+      Vec<T>::load(sh + c0, t);
+#pragma unroll
+      for (int j = 0; j < V; ++j) v[j] = Vec<T>::round(Vec<T>::round(v[j] * Vec<T>::round(1.f + s[j])) + t[j]);
+    }
+    Vec<T>::store(orow + c0, v);
+  }
+}
+
+// residual_rms: a row per workgroup, one 16-byte chunk per lane (rows of up to kRowLanes chunks). A DiT evaluation has
+// one to a few thousand rows, so one wave per row left a SIMD with one or two waves and a serial walk over the chunks:
+// latency, not bytes, was the time. 1536 bf16 values: 7.0 -> 6.6 us at 1422 rows (17.5 MB; 3.7 us at a large copy's rate),
+// 39.1 -> 33.6 at 16384.
 template <typename T>
 constexpr int kRowLanes = 2048 / Vec<T>::N;
 constexpr int kMaxRowBlocks = 1 << 20;  // workgroups of a launch; further rows are taken in turns
 
-// Adds the squares of up to kRowLanes chunks of a row, one in each lane's `v` (zeros past the row), to `ss`: lane l of
-// every wave adds chunks l, l + 64, l + 128, ... in that order, and wave_sum of `ss` is then the row's sum, the same in
-// all waves. That is the order of one wave walking the row, so that a seed renders the same bits as with such waves;
-// adding the waves' own sums rounds otherwise in one of some thousand rows, which the 24 blocks of a denoiser grow to 2e-2.
-// `row` holds a chunk per lane and must be free of reads (a barrier lies between two calls).
+// rsqrt(mean of the row's squares + eps), the same in every lane; `v` is this lane's chunk (zeros past the row). The
+// first wave adds the squares, lane l those of chunks l, l + 64, l + 128, ... in that order, and then the lanes: the order
+// of a wave that walks the row, so that a row gives the bits of rms_modulate and a seed renders the same ones whatever the
+// layout. Adding the waves' own sums rounds otherwise in one of some thousand rows, which the 24 blocks of a denoiser
+// grow to 2e-2 (and takes 6.3 us at 1422 rows, 31.1 at 16384). `row` and `result` must be free of reads.
 template <typename T>
-__device__ __forceinline__ void add_squares(const float (&v)[Vec<T>::N], T* row, float& ss) {
+__device__ __forceinline__ float row_inv_rms(const float (&v)[Vec<T>::N], int C, float eps, T* row, float* result) {
   constexpr int V = Vec<T>::N;
-  Vec<T>::store(row + threadIdx.x * V, v);
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < kRowLanes<T> / 64; ++k) {
-    if (64 * k >= static_cast<int>(blockDim.x)) break;
-    float u[V];
-    Vec<T>::load(row + (64 * k + (threadIdx.x & 63)) * V, u);
-#pragma unroll
-    for (int j = 0; j < V; ++j) ss = ss + u[j] * u[j];
+  const bool one = blockDim.x == 64;  // the row is one wave's: no exchange
+  if (!one) {
+    Vec<T>::store(row + threadIdx.x * V, v);
+    __syncthreads();
   }
+  float inv = 0.f;
+  if (threadIdx.x < 64) {
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < V; ++j) ss = ss + v[j] * v[j];
+#pragma unroll
+    for (int k = 1; k < kRowLanes<T> / 64; ++k) {
+      if (64 * k >= static_cast<int>(blockDim.x)) break;
+      float u[V];
+      Vec<T>::load(row + (64 * k + threadIdx.x) * V, u);
+#pragma unroll
+      for (int j = 0; j < V; ++j) ss = ss + u[j] * u[j];
+    }
+    inv = rsqrtf(wave_sum(ss) * (1.f / static_cast<float>(C)) + eps);
+    if (threadIdx.x == 0) *result = inv;
+  }
+  if (one) return inv;
+  __syncthreads();
+  return *result;
 }
 
 template <typename T>
@@ -117,56 +175,6 @@ __device__ __forceinline__ void norm_chunk(float (&v)[Vec<T>::N], float inv, con
   for (int j = 0; j < Vec<T>::N; ++j) {
     v[j] = Vec<T>::round((v[j] * inv) * w[j]);
     if (mod) v[j] = Vec<T>::round(Vec<T>::round(v[j] * Vec<T>::round(1.f + s[j])) + t[j]);
-  }
-}
-
-// The mean of squares over the row (fp32), then the normalised row scaled by `w` (fp32), cast, and with `scale` the
-// modulation by the row's batch entry of `scale` / `shift` (`mod_stride` elements apart per batch, `L` rows per
-// batch). A lane's first chunk stays in its registers; the others of a long row are read again (from the cache).
-template <typename T>
-__global__ __launch_bounds__(kRowLanes<T>) void rms_modulate_kernel(
-    const T* __restrict__ x, int64_t xs, const float* __restrict__ w, float eps, const T* __restrict__ scale,
-    const T* __restrict__ shift, int64_t mod_stride, int L, T* __restrict__ out, int64_t os, int64_t N, int C) {
-  constexpr int V = Vec<T>::N;
-  __shared__ __attribute__((aligned(16))) T squares[kRowLanes<T> * V];
-  const int first = threadIdx.x * V, step = blockDim.x * V;
-  for (int64_t n = blockIdx.x; n < N; n += gridDim.x) {
-    const int64_t b = static_cast<unsigned>(n) / static_cast<unsigned>(L);  // N <= 2^31
-    const T* row = x + n * xs;
-    T* orow = out + n * os;
-    float v[V] = {}, wv[V] = {}, s[V] = {}, t[V] = {};
-    if (first < C) {  // every load before the first use
-      Vec<T>::load(row + first, v);
-      load_weight<T>(w + first, wv);
-      if (scale) {
-        Vec<T>::load(scale + b * mod_stride + first, s);
-        Vec<T>::load(shift + b * mod_stride + first, t);
-      }
-    }
-    float ss = 0.f;
-    add_squares<T>(v, squares, ss);
-    for (int turn = step; turn < C; turn += step) {  // uniform: every lane joins every turn
-      float u[V] = {};
-      if (first + turn < C) Vec<T>::load(row + first + turn, u);
-      __syncthreads();
-      add_squares<T>(u, squares, ss);
-    }
-    const float inv = rsqrtf(wave_sum(ss) * (1.f / static_cast<float>(C)) + eps);
-    if (first < C) {
-      norm_chunk<T>(v, inv, wv, scale != nullptr, s, t);
-      Vec<T>::store(orow + first, v);
-    }
-    for (int c0 = first + step; c0 < C; c0 += step) {
-      Vec<T>::load(row + c0, v);
-      load_weight<T>(w + c0, wv);
-      if (scale) {
-        Vec<T>::load(scale + b * mod_stride + c0, s);
-        Vec<T>::load(shift + b * mod_stride + c0, t);
-      }
-      norm_chunk<T>(v, inv, wv, scale != nullptr, s, t);
-      Vec<T>::store(orow + c0, v);
-    }
-    if (n + gridDim.x < N) __syncthreads();  // `squares` is free again
   }
 }
 
@@ -226,6 +234,7 @@ __global__ __launch_bounds__(kRowLanes<T>) void residual_rms_kernel(
     int64_t mod_stride, int L, T* __restrict__ out_h, T* __restrict__ out_y, int64_t os, int64_t N, int C) {
   constexpr int V = Vec<T>::N;
   __shared__ __attribute__((aligned(16))) T squares[kRowLanes<T> * V];
+  __shared__ float result;
   const int c0 = threadIdx.x * V;
   for (int64_t n = blockIdx.x; n < N; n += gridDim.x) {
     const int64_t b = static_cast<unsigned>(n) / static_cast<unsigned>(L);  // N <= 2^31
@@ -263,14 +272,12 @@ __global__ __launch_bounds__(kRowLanes<T>) void residual_rms_kernel(
       }
       Vec<T>::store(out_h + n * os + c0, r);
     }
-    float ss = 0.f;
-    add_squares<T>(r, squares, ss);
-    const float inv = rsqrtf(wave_sum(ss) * (1.f / static_cast<float>(C)) + eps);
+    const float inv = row_inv_rms<T>(r, C, eps, squares, &result);
     if (c0 < C) {
       norm_chunk<T>(r, inv, wv, scale != nullptr, s, t);
       Vec<T>::store(out_y + n * os + c0, r);
     }
-    if (n + gridDim.x < N) __syncthreads();  // `squares` is free again
+    if (n + gridDim.x < N) __syncthreads();  // `squares` and `result` are free again
   }
 }
 
@@ -339,7 +346,8 @@ unsigned row_blocks(int64_t N) { return static_cast<unsigned>(N < blk::kMaxRowBl
 template <typename T>
 void launch_rms(hipStream_t s, const void* x, int64_t xs, const float* w, float eps, const void* scale,
                 const void* shift, int64_t ms, int L, void* out, int64_t os, int64_t N, int C) {
-  hipLaunchKernelGGL(blk::rms_modulate_kernel<T>, dim3(row_blocks(N)), dim3(row_lanes<T>(C)), 0, s, static_cast<const T*>(x), xs, w, eps,
+  const dim3 grid(static_cast<unsigned>((N + 3) / 4));
+  hipLaunchKernelGGL(blk::rms_modulate_kernel<T>, grid, dim3(256), 0, s, static_cast<const T*>(x), xs, w, eps,
                      static_cast<const T*>(scale), static_cast<const T*>(shift), ms, L, static_cast<T*>(out), os, N,
                      C);
 }
