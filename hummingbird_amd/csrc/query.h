@@ -38,38 +38,51 @@ struct RmsQuery {
   // 1 / rms of every row, in both lane halves. A row's squares are added in the order of its dims, as by a lane that
   // holds the whole row, so that a seed renders the same bits as with such lanes: the sum of the two halves' own sums
   // rounds otherwise, which moves 2e-4 of an attention's results by one bf16 step and, over the 24 blocks of a denoiser,
-  // its output by 2e-2. Two rows go together, one per lane half (one chain of D additions for both); a single row is
-  // added in both halves. Against the halves' own sums: 102.3 -> 102.9 us at B = 2, L = 1292, 12 x 128 (fp16).
+  // its output by 2e-2. Two rows are added by one lane half each, which gets the other's chunks (one chain of D additions
+  // for both); for a single row the sum goes from half to half. Against
+  // the halves' own sums: cross-attention B = 2, L = 2584 x 257, 24 x 64 33.4 -> 33.5 us, L = 8192 x 33 26.4 -> 27.5, 12 x
+  // 128 37.1 -> 37.7; self-attention B = 2, L = 1292, 12 x 128 97.6 -> 98.3, 24 x 64 unchanged.
   template <int NCT>
   __device__ __forceinline__ void stats(const u32x4 (&raw)[NCT][1][D / 16], float (&st)[NCT][1]) const {
     static_assert(NCT == 1 || NCT == 2, "one row, or one per lane half");
     float ss = 0.f;
+    auto add = [&](u32x4 chunk) {
+      float x[8];
+      IO::unpack8(chunk, x);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ss = __fmaf_rn(x[j], x[j], ss);
+    };
+    auto halves = [](float v, float (&h)[2]) {  // lanes 0-31's value and lanes 32-63's, each in both
+      const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+      h[0] = __uint_as_float(r[0]);
+      h[1] = __uint_as_float(r[1]);
+    };
+    float h[2];
 #pragma unroll
     for (int kk = 0; kk < D / 16; ++kk) {
-      u32x4 c[2];  // chunks 2 kk and 2 kk + 1 of the first row in lanes 0-31, of the last one in lanes 32-63
+      if constexpr (NCT == 1) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const auto r = __builtin_amdgcn_permlane32_swap(raw[0][0][kk][e], raw[NCT - 1][0][kk][e], false, false);
-        c[0][e] = r[0];
-        c[1][e] = r[1];
-      }
+        for (int i = 0; i < 2; ++i) {  // chunk 2 kk + i, this lane's in half i
+          add(raw[0][0][kk]);
+          halves(ss, h);
+          ss = h[i];
+        }
+      } else {
+        u32x4 c[2];  // chunks 2 kk and 2 kk + 1 of the first row in lanes 0-31, of the second in lanes 32-63
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        float x[8];
-        IO::unpack8(c[i], x);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) ss = __fmaf_rn(x[j], x[j], ss);
+        for (int e = 0; e < 4; ++e) {
+          const auto r = __builtin_amdgcn_permlane32_swap(raw[0][0][kk][e], raw[1][0][kk][e], false, false);
+          c[0][e] = r[0];
+          c[1][e] = r[1];
+        }
+        add(c[0]);
+        add(c[1]);
       }
     }
     const float inv = rsqrtf(ss / static_cast<float>(D) + eps);
-    if constexpr (NCT == 1) {
-      st[0][0] = inv;
-    } else {
-      const uint32_t u = __float_as_uint(inv);
-      const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-      st[0][0] = __uint_as_float(r[0]);
-      st[1][0] = __uint_as_float(r[1]);
-    }
+    halves(inv, h);
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct) st[ct][0] = h[ct];
   }
   __device__ __forceinline__ void apply(u32x4 raw, const Par& p, float inv, float (&y)[8]) const {
     IO::unpack8(raw, y);
