@@ -248,8 +248,8 @@ __device__ __forceinline__ void dense_attend_loop(
   }
 }
 
-// `qkv` rows hold q at section 0 and q_diff at section `sqd` (units of H * D); the L queries are padded to Lp (a
-// multiple of 128), the Lk keys of the workspace to Lkp. Self-attention has Lk = L. QB: queries per workgroup;
+// `qkv` rows hold q at section 0 and q_diff at section `sqd` (units of H * D); the last workgroup of a (batch, head) may
+// hold fewer than QB of the L queries; the Lk keys of the workspace are padded to Lkp. Self-attention has Lk = L. QB: queries per workgroup;
 // the 64-query form runs three workgroups per CU.
 // ROPE: false for half = 0 (the cross-attention), whose workgroups are short enough for the rotary forms they would
 // only jump over to show: 29.0 -> 28.2 us at B = 2, L = 2584, 257 keys, 24 heads of 64 (28.8 before query.h).
@@ -257,7 +257,7 @@ template <class IO, int D, int QB, int NW, bool ROPE>
 __global__ __launch_bounds__(64 * NW, D == 64 ? (QB == 64 ? 3 : 2) : 1) void dense_attend(
     const uint16_t* __restrict__ qkv, int64_t rs, int sqd, const float* __restrict__ cosT,
     const float* __restrict__ sinT, int half, float eps, const uint16_t* __restrict__ ws, int64_t region, int B,
-    int L, int Lp, int Lk, int Lkp, int H, const float* __restrict__ qw, const float* __restrict__ kw,
+    int L, int Lk, int Lkp, int H, const float* __restrict__ qw, const float* __restrict__ kw,
     const float* __restrict__ lam, uint16_t* __restrict__ out) {
   using T = DenseTile<D, QB, NW>;
   constexpr int NB = T::NB, NCT = T::NCT;
@@ -402,27 +402,28 @@ int launch_dense_attend_16bit(hipStream_t stream, int dtype, const void* q, int6
                               const float* kw, const float* cos, const float* sin, int half, float eps,
                               const float* lam, void* out, int B, int L, int Lk, int H, int D, const DenseLayout& lay,
                               const void* workspace) {
-  const int Lp = (L + 127) / 128 * 128;
   const uint16_t* x = static_cast<const uint16_t*>(q);
   const uint16_t* ws = static_cast<const uint16_t*>(workspace);
   uint16_t* o = static_cast<uint16_t*>(out);
   const int Lkp = static_cast<int>(lay.Lp);
   const bool f16 = dtype == HB_F16;
-  // head_dim 64: 128-query workgroups run two per CU. With between one and one and a half of them per CU, some CUs would
-  // run two while most run one; 64-query workgroups (three per CU) spread the same work more evenly (3 to 9 % faster
-  // over that range, 4 % slower at exactly one per CU, 7 to 13 % between 1.6 and two, where they cost more per query
-  // than they gain in balance). Past two per CU, where the second round of 128-query workgroups is mostly empty, they
-  // win again: 7 % at 2.06, 5 % at 2.25, 4 % at 2.44 per CU; at 2.6 they lose 7 %. And on grids of at most half a
-  // 128-query workgroup per CU they halve the work of each busy CU: 16.2 against 19.6 us at B = 2, L = 512, H = 16.
-  const int64_t blocks128 = static_cast<int64_t>(B) * H * (Lp / 128);
+  // head_dim 64: 128-query workgroups run two per CU, 64-query ones three, which spread the same work more evenly but
+  // cost more per query. Measured over B = 1, 24 and 16 heads, L = 318 .. 4224: on grids of at most half a 128-query
+  // workgroup per CU they halve the work of each busy CU (24 to 33 % faster); past one per CU, where some CUs would run
+  // two and most one, they are 11 % faster, 6 to 8 % still at one and a half (three 64-query ones), and 8 to 11 % slower
+  // from there to two, where the 128-query ones fill both places; past two, where the second round of those is mostly
+  // empty, 8 % faster at 2.06, 6 % at 2.3, 3 to 5 % at 2.45, as long as the 64-query ones are at most five per CU (24 heads, L
+  // = 3390: 154.8 against 159.9 us; L = 3456, 1296 of them on 256 CUs: 175.1 against 161.7). Between a half and one they
+  // are within 6 % faster (0.56) and 1 % slower (1.0) and the 128-query form runs.
+  const int64_t blocks128 = static_cast<int64_t>(B) * H * ((L + 127) / 128);
+  const int64_t blocks64 = static_cast<int64_t>(B) * H * ((L + 63) / 64);
   const int64_t ncu = device_cus();
   const bool spread = 2 * blocks128 <= ncu || (blocks128 > ncu && 2 * blocks128 <= 3 * ncu) ||
-                      (blocks128 > 2 * ncu && 5 * blocks128 <= 12 * ncu);
+                      (blocks128 > 2 * ncu && blocks64 <= 5 * ncu);
   if (D == 64 && spread) {
-    const int nblocks = B * H * ((L + 63) / 64);
     auto kernel = f16 ? attend_kernel<F16Io, 64, 64, 4>(half) : attend_kernel<Bf16Io, 64, 64, 4>(half);
-    hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(DenseTile<64, 64>::NT), 0, stream, x, rs, sqd, cos, sin, half, eps,
-                       ws, lay.region_elems, B, L, Lp, Lk, Lkp, H, qw, kw, lam, o);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks64)), dim3(DenseTile<64, 64>::NT), 0, stream, x, rs,
+                       sqd, cos, sin, half, eps, ws, lay.region_elems, B, L, Lk, Lkp, H, qw, kw, lam, o);
   } else {
     // head_dim 128: 8 waves of one branch each, two per SIMD. With the queries of query.h they are faster on every grid
     // than 4 waves holding both branches (12 heads, half 32: 29.0 against 32.7 us at B = 1, L = 512, 49.6 against 57.5
@@ -430,7 +431,7 @@ int launch_dense_attend_16bit(hipStream_t stream, int dtype, const void* q, int6
     auto kernel = D == 64 ? (f16 ? attend_kernel<F16Io, 64, 128, 4>(half) : attend_kernel<Bf16Io, 64, 128, 4>(half))
                           : (f16 ? attend_kernel<F16Io, 128, 128, 8>(half) : attend_kernel<Bf16Io, 128, 128, 8>(half));
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks128)), dim3(D == 64 ? 256 : 512), 0, stream, x, rs, sqd,
-                       cos, sin, half, eps, ws, lay.region_elems, B, L, Lp, Lk, Lkp, H, qw, kw, lam, o);
+                       cos, sin, half, eps, ws, lay.region_elems, B, L, Lk, Lkp, H, qw, kw, lam, o);
   }
   return launch_status("dense_attend");
 }

@@ -1,6 +1,6 @@
 // Key tiles of the flash-style attention kernels (dense, and band with a wide window): the prepared-tile
-// layout in the workspace and in LDS, the global -> LDS copier, and the differential epilogue of a 4-wave
-// workgroup. Shared by dense.hip and band_tiled.hip.
+// layout in the workspace and in LDS, the global -> LDS copier, and the differential epilogue of a workgroup
+// (4 or 8 waves). Shared by dense.hip and band_tiled.hip; fp32.hip takes the DMA copy, the swizzle and the key order.
 #pragma once
 
 #include <type_traits>
@@ -41,8 +41,8 @@ __device__ __forceinline__ int swz(int row, int chunk) {
 
 // Attention tiling: a workgroup of NW waves attends QB queries.
 //   - Split layouts (D = 64 with 4 waves; D = 128 with 8 waves): each wave owns one differential branch of
-//     32 * NCT queries; the first NW / 2 waves run branch 1 (q, k), the others branch 2 (q_diff, k_diff), and each
-//     branch-2 wave hands its normalised result to the branch-1 wave of the same queries through LDS at the end.
+//     32 * NCT queries; the first NW / 2 waves run branch 1 (q, k), the others branch 2 (q_diff, k_diff), and the two
+//     waves of the same queries each finish half of their output tiles at the end (store_diff_split).
 //     D = 64: QB = 128 (two MFMA column tiles per wave, so every K fragment read from LDS feeds two MFMAs while a
 //     wave's registers still fit two waves per SIMD) or 64 for grids too small to fill the GPU. D = 128: QB = 128
 //     over 8 waves, one column tile each, so two waves share each SIMD in the one workgroup per CU that the 96 KB
@@ -60,7 +60,7 @@ struct DenseTile {
   static constexpr int STAGE = 3 * K_ELEMS;  // K, K_diff, V^T of one 64-key tile, swizzled rows
   static constexpr int BPT = 64 * D * 2 / 1024;  // 1 KB blocks per tensor of a 64-key tile
   static constexpr int NBLK = 3 * BPT;            // blocks per tile (a multiple of the waves)
-  // the split epilogue's hand-over (fp32 accumulators of every branch-2 wave), and the LDS a workgroup declares
+  // the split epilogue's exchange (half of every wave's fp32 accumulators), and the LDS a workgroup declares
   static constexpr int XBUF_BYTES = SPLIT ? (NW / 2) * NCT * (D / 32) * 16 * 64 * 4 : 0;
   static constexpr int SMEM_ELEMS = 2 * STAGE > XBUF_BYTES / 2 ? 2 * STAGE : XBUF_BYTES / 2;
 };

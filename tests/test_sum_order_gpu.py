@@ -12,6 +12,7 @@ import pytest
 import torch
 
 from hummingbird_amd import cross_attention as xattn
+from hummingbird_amd import dense_attention as da
 from hummingbird_amd import elementwise
 
 pytestmark = pytest.mark.gpu
@@ -62,3 +63,22 @@ def test_queries_add_their_squares_in_order(length, heads, dim):
     context = xattn.prepare_cross_kv(kv, torch.ones(dim, device=DEV), heads, dim, 1e-6)
     got = xattn.cross_attention(q, context, weight, 0.0)
     assert torch.equal(got, xattn.cross_attention(zeros, context, weight, 0.0))
+
+
+@pytest.mark.parametrize("length", [1350, 3390, 3456])
+def test_workgroup_sizes_give_the_same_bits(length):
+    """24 heads at lengths on both sides of the lines between 64- and 128-query workgroups (256 CUs: 24 x 22 64-query ones,
+    24 x 53, and 24 x 27 128-query ones) against the same heads one by one, which run 64-query ones at every length."""
+    print(f"\n[case] workgroup sizes L{length}", flush=True)
+    heads, dim, half = 24, 64, 16
+    gen = torch.Generator(device=DEV).manual_seed(2)
+    qkv = torch.randn((1, length, 5, heads, dim), generator=gen, device=DEV).to(torch.bfloat16)
+    weight = 1 + 0.02 * torch.randn(dim, generator=gen, device=DEV)
+    cos, sin = da.rope_tables(length, 10000.0 ** (-torch.arange(half, device=DEV) / half))
+
+    def run(x):
+        return da.dense_attention(x.reshape(1, length, -1).contiguous(), weight, weight, cos, sin, None, x.shape[3], dim,
+                                  half, 1e-6)
+    whole = run(qkv).reshape(length, heads, dim)
+    for head in (0, heads - 1):
+        assert torch.equal(run(qkv[:, :, :, head:head + 1]).reshape(length, dim), whole[:, head])
