@@ -848,7 +848,7 @@ __global__ __launch_bounds__(256, SplitTile<D>::OCC) void dense_attend_f32(
 }
 
 // tanh in fp32. Below 0.625: y + y^3 Q(y^2), Q a degree-5 least-maximum fit of (tanh(y)/y - 1)/y^2 (made for this
-// kernel; 2^-32 relative to tanh before rounding). Above: 1 - 2 / (1 + 2^(2 log2(e) |y|)) with the rounding error of
+// kernel; its fp32 coefficients are within 2^-28.5 of tanh before rounding). Above: 1 - 2 / (1 + 2^(2 log2(e) |y|)) with the rounding error of
 // the exponent carried into the exponential and one Newton step on the reciprocal; 2 / (1 + e) is below 0.45 there,
 // so the hardware exponential's error is at least halved. Both sides are computed and one is selected: 22
 // instructions without a branch, where the library's tanhf branches per element (both sides run in most waves).

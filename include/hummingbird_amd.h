@@ -68,7 +68,9 @@ enum hb_status {
  * operands (K, q * scale, P, V) are rounded to bf16 as in the reference's fused kernels
  * (sa3jax/dense_attention.py:75-77, 83, 90; sa3jax/band_attention.py:85, 94, 101), while the RMSNorm and RoPE
  * outputs round to the compute dtype (sa3jax/dense_attention.py:66, 69) and the output is written in it. HB_F32
- * is the FP32_PARITY preset: fp32 throughout (the XLA chain's arithmetic). */
+ * is the FP32_PARITY preset, at fp32 accuracy: norms, RoPE, softmax, sums and the subtraction are fp32 (as in the XLA
+ * chain), and the two matrix products run on half matrix cores from operands split into two halves each, with fp32
+ * accumulation, or on the fp32 matrix cores where V has a range that a split does not hold. */
 enum hb_dtype { HB_BF16 = 0, HB_F32 = 1, HB_F16 = 2 };
 
 /* Message for the last failing call on this thread ("" if none). */

@@ -66,8 +66,8 @@ def test_dense_fp32_gains_over_many_magnitudes(half):
 
 @pytest.mark.parametrize("scale", [1e-30, 1e-6, 1.0, 1e6, 1e30])
 def test_dense_fp32_values_over_many_magnitudes(scale):
-    """V of any magnitude, and growing by 1e12 from the first key tile to the last (the accumulators follow the largest
-    tile so far), with a tile of zeros among them."""
+    """V of any magnitude, and growing by 1e12 from the first key tile to the last, with a tile of zeros among them: the
+    result as a whole, and each dim by itself."""
     print(f"\n[case] fp32 dense V {scale}", flush=True)
     h, d, length = 2, 64, 200
     inp = workloads.dense_inputs(1, length, h, d, seed=8, dtype="fp32")
@@ -76,6 +76,8 @@ def test_dense_fp32_values_over_many_magnitudes(scale):
     inp["qkv"][0, :, 2 * h * d:3 * h * d] *= grow[:, None]
     got, ref = dense_both(inp)
     assert_fp32_parity(got, ref, f"V {scale}")
+    for dim in range(h * d):
+        assert_fp32_parity(got[0, :, dim], ref[0, :, dim], f"V {scale} dim {dim}")
 
 
 @pytest.mark.parametrize("window,dim", [(0, 64), (31, 64), (32, 64), (33, 128), (95, 64), (200, 128)])
