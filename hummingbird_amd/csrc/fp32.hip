@@ -106,24 +106,28 @@ __device__ __forceinline__ int bound_exp(float b) {
 struct ScaleTable {
   int k[128], q[128], logit;
 };
+// Exponent of the key bound of dim d.
+template <class KBound>
+__device__ __forceinline__ int key_exp(int d, int half, KBound kb) {
+  const int p = d < half ? d + half : d < 2 * half ? d - half : d;
+  return bound_exp(fmaxf(kb(d), kb(p)));
+}
 // The keys' part, before a barrier.
 template <int D, class KBound>
 __device__ __forceinline__ void key_scales(ScaleTable& t, int half, KBound kb) {
-  for (int d = threadIdx.x; d < D; d += 256) {
-    const int p = d < half ? d + half : d < 2 * half ? d - half : d;
-    t.k[d] = -bound_exp(fmaxf(kb(d), kb(p)));
-  }
+  for (int d = threadIdx.x; d < D; d += 256) t.k[d] = -key_exp(d, half, kb);
 }
-// The queries' part, for the keys' in `t`, after a barrier and before one.
-template <int D, class QBound>
-__device__ __forceinline__ void query_scales(ScaleTable& t, int half, QBound qb) {
+// The queries' part, by the first wave, before a barrier: `ek(d)` is -k[d], the exponent of the key bound of dim d.
+template <int D, class KExp, class QBound>
+__device__ __forceinline__ void query_scales(ScaleTable& t, int half, KExp ek, QBound qb) {
   const int lane = threadIdx.x & 63;
   if (threadIdx.x >= 64) return;
-  int emax = -1000;
+  int k[D / 64], emax = -1000;
 #pragma unroll
   for (int i = 0; i < D / 64; ++i) {
     const int d = lane + 64 * i, p = d < half ? d + half : d < 2 * half ? d - half : d;
-    const int e = bound_exp(fmaxf(qb(d), qb(p))) - t.k[d];
+    k[i] = ek(d);
+    const int e = bound_exp(fmaxf(qb(d), qb(p))) + k[i];
     emax = e > emax ? e : emax;
   }
 #pragma unroll
@@ -132,7 +136,7 @@ __device__ __forceinline__ void query_scales(ScaleTable& t, int half, QBound qb)
     emax = other > emax ? other : emax;
   }
 #pragma unroll
-  for (int i = 0; i < D / 64; ++i) t.q[lane + 64 * i] = -t.k[lane + 64 * i] - emax;
+  for (int i = 0; i < D / 64; ++i) t.q[lane + 64 * i] = k[i] - emax;
   if (lane == 0) t.logit = emax;
 }
 // After RMSNorm |x_d| <= sqrt(D) |w_d|; |DyT(x)_d| <= |gamma_d| + |beta_d| (`dyt` = [alpha, gamma, beta]).
@@ -813,15 +817,13 @@ __global__ __launch_bounds__(256, SplitTile<D>::OCC) void dense_attend_f32(
   const int qb = tile % nqb, bh = tile / nqb, h = bh % H, b = bh / H;
   const int wave = wave_id(), br = wave >> 1, q = qb * 64 + (wave & 1) * 32 + (threadIdx.x & 31);
   // The powers of two that the preparation gave the keys' dims, from its own k_weight (KeyRows).
-  for (int d = threadIdx.x; d < D; d += 256) {
-    const uint16_t* lo = reinterpret_cast<const uint16_t*>(ws + static_cast<int64_t>(bh) * Lkp * D) + T::PLANE;
+  const uint16_t* lo = reinterpret_cast<const uint16_t*>(ws + static_cast<int64_t>(bh) * Lkp * D) + T::PLANE;
+  query_scales<D>(scale, half, [&](int d) {
     int code = 0;
 #pragma unroll
     for (int r = 0; r < 8; ++r) code |= ((lo[T::k_at(r, d / 8) + d % 8] >> 14) & 1) << r;
-    scale.k[d] = 128 - code;
-  }
-  __syncthreads();
-  query_scales<D>(scale, half, rms_bound<D>(qw));
+    return code - 128;
+  }, rms_bound<D>(qw));
   __syncthreads();
 
   u32x4 qf[2][D / 16];
@@ -994,9 +996,8 @@ __global__ __launch_bounds__(256, WS ? SplitTile<D>::OCC : SplitTile<D>::OCC - 1
   const int64_t HD = static_cast<int64_t>(H) * D;
   const float* xb = qkv + static_cast<int64_t>(b) * S * rs + h * D;
 
-  key_scales<D>(scale, half, dyt_bound<D>(kdyt));
-  __syncthreads();
-  query_scales<D>(scale, half, dyt_bound<D>(qdyt));
+  if constexpr (!WS) key_scales<D>(scale, half, dyt_bound<D>(kdyt));
+  query_scales<D>(scale, half, [&](int d) { return key_exp(d, half, dyt_bound<D>(kdyt)); }, dyt_bound<D>(qdyt));
   __syncthreads();
   u32x4 qf[2][D / 16];
   int n;
