@@ -11,11 +11,11 @@
 //                workspace of three (B, H, Sp, D) regions; V is stored transposed per 64-key tile in the order
 //                the PV MFMA consumes it. Keys at or past S are zero.
 //   band_attend  one workgroup of 4 waves per (batch, head, 128-query block): the lanes prepare the query
-//                rows (query.h: DyT, RoPE and the softmax scale, one rounding), then the 64-key tiles of the block's window
-//                [q0 - w, q0 + 128 + w) stream through LDS (global_load_lds, double-buffered). Each wave skips
-//                the tiles outside its band, runs the tiles inside |k - q| <= w for all of its queries unmasked
-//                and masks the others per score (band_attention.py:108-110); the branches are subtracted in fp32
-//                with one cast (same_l.py:168-169).
+//                rows (query.h: DyT, RoPE and the softmax scale, one rounding), then the 64-key tiles of the block's
+//                window [q0 - w, q0 + 128 + w) stream through LDS (global_load_lds, double-buffered). Each wave skips
+//                the tiles outside its band, runs the tiles inside |k - q| <= w for all of its queries unmasked and
+//                masks the others per score (band_attention.py:108-110); the branches are subtracted in fp32 with one
+//                cast (same_l.py:168-169).
 //
 // Every key is prepared once per call and read back from L2 by the blocks whose window covers it.
 #include "api.h"

@@ -248,11 +248,11 @@ __device__ __forceinline__ void dense_attend_loop(
   }
 }
 
-// `qkv` rows hold q at section 0 and q_diff at section `sqd` (units of H * D); the last workgroup of a (batch, head) may
-// hold fewer than QB of the L queries; the Lk keys of the workspace are padded to Lkp. Self-attention has Lk = L. QB: queries per workgroup;
-// the 64-query form runs three workgroups per CU.
-// ROPE: false for half = 0 (the cross-attention), whose workgroups are short enough for the rotary forms they would
-// only jump over to show: 29.0 -> 28.2 us at B = 2, L = 2584, 257 keys, 24 heads of 64 (28.8 before query.h).
+// `qkv` rows hold q at section 0 and q_diff at section `sqd` (units of H * D); the last workgroup of a (batch, head)
+// may hold fewer than QB of the L queries; the Lk keys of the workspace are padded to Lkp. Self-attention has Lk = L.
+// QB: queries per workgroup; the 64-query form runs three workgroups per CU. ROPE: false for half = 0 (the
+// cross-attention), whose workgroups are short enough for the rotary forms they would only jump over to show: 29.0 ->
+// 28.2 us at B = 2, L = 2584, 257 keys, 24 heads of 64 (28.8 before query.h).
 template <class IO, int D, int QB, int NW, bool ROPE>
 __global__ __launch_bounds__(64 * NW, D == 64 ? (QB == 64 ? 3 : 2) : 1) void dense_attend(
     const uint16_t* __restrict__ qkv, int64_t rs, int sqd, const float* __restrict__ cosT,
@@ -410,11 +410,11 @@ int launch_dense_attend_16bit(hipStream_t stream, int dtype, const void* q, int6
   // head_dim 64: 128-query workgroups run two per CU, 64-query ones three, which spread the same work more evenly but
   // cost more per query. Measured over B = 1, 24 and 16 heads, L = 318 .. 4224: on grids of at most half a 128-query
   // workgroup per CU they halve the work of each busy CU (24 to 33 % faster); past one per CU, where some CUs would run
-  // two and most one, they are 11 % faster, 6 to 8 % still at one and a half (three 64-query ones), and 8 to 11 % slower
-  // from there to two, where the 128-query ones fill both places; past two, where the second round of those is mostly
-  // empty, 8 % faster at 2.06, 6 % at 2.3, 3 to 5 % at 2.45, as long as the 64-query ones are at most five per CU (24 heads, L
-  // = 3390: 154.8 against 159.9 us; L = 3456, 1296 of them on 256 CUs: 175.1 against 161.7). Between a half and one they
-  // are within 6 % faster (0.56) and 1 % slower (1.0) and the 128-query form runs.
+  // two and most one, they are 11 % faster, 6 to 8 % still at one and a half (three 64-query ones), and 8 to 11 %
+  // slower from there to two, where the 128-query ones fill both places; past two, where the second round of those is
+  // mostly empty, 8 % faster at 2.06, 6 % at 2.3, 3 to 5 % at 2.45, as long as the 64-query ones are at most five per
+  // CU (24 heads, L = 3390: 154.8 against 159.9 us; L = 3456, 1296 of them on 256 CUs: 175.1 against 161.7). Between a
+  // half and one they are within 6 % faster (0.56) and 1 % slower (1.0) and the 128-query form runs.
   const int64_t blocks128 = static_cast<int64_t>(B) * H * ((L + 127) / 128);
   const int64_t blocks64 = static_cast<int64_t>(B) * H * ((L + 63) / 64);
   const int64_t ncu = device_cus();

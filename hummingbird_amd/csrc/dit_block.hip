@@ -117,17 +117,17 @@ __global__ __launch_bounds__(256) void rms_modulate_kernel(const T* __restrict__
 
 // residual_rms: a row per workgroup, one 16-byte chunk per lane (rows of up to kRowLanes chunks). A DiT evaluation has
 // one to a few thousand rows, so one wave per row left a SIMD with one or two waves and a serial walk over the chunks:
-// latency, not bytes, was the time. 1536 bf16 values: 7.0 -> 6.6 us at 1422 rows (17.5 MB; 3.7 us at a large copy's rate),
-// 39.1 -> 33.6 at 16384.
+// latency, not bytes, was the time. 1536 bf16 values: 7.0 -> 6.6 us at 1422 rows (17.5 MB; 3.7 us at a large copy's
+// rate), 39.1 -> 33.6 at 16384.
 template <typename T>
 constexpr int kRowLanes = 2048 / Vec<T>::N;
 constexpr int kMaxRowBlocks = 1 << 20;  // workgroups of a launch; further rows are taken in turns
 
 // rsqrt(mean of the row's squares + eps), the same in every lane; `v` is this lane's chunk (zeros past the row). The
-// first wave adds the squares, lane l those of chunks l, l + 64, l + 128, ... in that order, and then the lanes: the order
-// of a wave that walks the row, so that a row gives the bits of rms_modulate and a seed renders the same ones whatever the
-// layout. Adding the waves' own sums rounds otherwise in one of some thousand rows, which the 24 blocks of a denoiser
-// grow to 2e-2 (and takes 6.3 us at 1422 rows, 31.1 at 16384). `row` and `result` must be free of reads.
+// first wave adds the squares, lane l those of chunks l, l + 64, l + 128, ... in that order, and then the lanes: the
+// order of a wave that walks the row, so that a row gives the bits of rms_modulate and a seed renders the same ones
+// whatever the layout. Adding the waves' own sums rounds otherwise in one of some thousand rows, which the 24 blocks of
+// a denoiser grow to 2e-2 (and takes 6.3 us at 1422 rows, 31.1 at 16384). `row` and `result` must be free of reads.
 template <typename T>
 __device__ __forceinline__ float row_inv_rms(const float (&v)[Vec<T>::N], int C, float eps, T* row, float* result) {
   constexpr int V = Vec<T>::N;

@@ -9,27 +9,28 @@
 // lo hi + hi lo + hi hi (the lo lo one left out is below 2^-22 of the product at its largest, 2^-25 rms) accumulated in
 // fp32. An fp32 MFMA chain rounds its accumulator once per two dims and key tile after key tile; these round it three
 // times per sixteen, and a tile's P V is added up apart, so the results are nearer to the 64-bit ones than the fp32
-// chain's were: relative error (2-norm) 3.3e-7 against 9.1e-7 on dense B = 2, L = 1292, 2.7e-7 against 5.4e-7 on the band
-// at S = 16384, w = 128. Times, whole calls against the fp32 matrix cores fed through registers: dense (2, 1292, 24
-// heads) 530 -> 188 us, L = 2584 1570 -> 599, head_dim 128 (2, 1292, 12 heads) 683 -> 171, cross (2, 2584 x 257) 204 ->
-// 74, band S = 16384, w = 128 468 -> 140. Three bf16 terms and six products, which need no scaling, were measured too:
-// 290 us for the first of these. The matrix cores slow down on such operands (about 27 ns per 32x32x16 product and SIMD),
-// so the number of products sets the time.
+// chain's were: relative error (2-norm) 3.4e-7 against 8.9e-7 on dense B = 2, L = 1292, 2.8e-7 against 6.9e-7 on the
+// band at S = 16384, w = 128. Times, whole calls against the fp32 matrix cores fed through registers: dense (2, 1292,
+// 24 heads) 529 -> 186 us, L = 2584 1570 -> 594, head_dim 128 (2, 1292, 12 heads) 684 -> 166, cross (2, 2584 x 257) 204
+// -> 75, band S = 16384, w = 128 467 -> 141. Three bf16 terms and six products, which need no scaling, were measured
+// too: 290 us for the first of these. The matrix cores slow down on such operands (about 27 ns per 32x32x16 product and
+// SIMD), so the number of products sets the time.
 //
 //   S^T[key][query] = K Q^T   A = K rows from LDS, B = q in registers
-//   P = exp2(S^T c - m)       m the max of the tile's S^T c, one FMA per score; masked scores are -inf and give exactly 0
+//   P = exp2(S^T c - m)       m the max of the tile's S^T c, one FMA per score; masked scores are -inf and give 0
 //   acc = V^T P^T             A = V^T rows from LDS, B = P straight from the S^T accumulators
 //   O^T[d][query] += acc      online softmax: one factor per query takes the tile's share to the running max
 //
 // Ranges. A half holds 2^-24 .. 65504, so every operand is scaled by powers of two (exact, undone in c and at the end):
-//   - dim d of the keys by 2^k[d] and of the queries by 2^q[d], from the norm parameters (scale_table), so that gains of
-//     many magnitudes leave no dim out; then each key tile and each query row by a power of two from its own largest
-//     value, so that neither tables that are no rotation nor norms far below their bounds leave the half range. What a half
-//     cannot hold is below 2^-37 of a tile's largest key value and 2^-39 of a row's largest query value, so scaled.
-//   - V by a power of two per key tile, from the tile's largest magnitude and stored with the tile. A tile whose keys or
-//     dims differ too much for that (VTile), or that holds an infinity or NaN, keeps its fp32 bits, and its P V runs on
-//     the fp32 matrix cores: every dim and every query has fp32 accuracy relative to its own size, whatever other values
-//     V holds.
+//   - dim d of the keys by 2^k[d] and of the queries by 2^q[d], from the norm parameters (ScaleTable), so that gains
+//     of many magnitudes leave no dim out; then each key tile and each query row by a power of two from its own largest
+//     value, so that neither tables that are no rotation nor norms far below their bounds leave the half range. What a
+//     half cannot hold is below 2^-37 of a tile's largest key value and 2^-39 of a row's largest query value, so
+//     scaled.
+//   - V by a power of two per key tile, from the tile's largest magnitude and stored with the tile. A tile whose keys
+//     or dims differ too much for that (VTile), or that holds an infinity or NaN, keeps its fp32 bits, and its P V runs
+//     on the fp32 matrix cores: every dim and every query has fp32 accuracy relative to its own size, whatever other
+//     values V holds.
 //   - P by 2^14, relative to the tile's own largest.
 //
 // Work split: a workgroup (4 waves) owns 64 queries of one (batch, head); waves 0-1 run branch 1 on 32 queries
@@ -50,7 +51,7 @@ __device__ __forceinline__ void st4(float* p, f32x4 v) { *reinterpret_cast<f32x4
 // One key tile, the same bytes in LDS and in the workspace: K, K_diff and V, each a hi and a lo plane of KT x D halves.
 // K planes are [key][d], V planes V^T [d][position] in v_tile_key order; the 16-byte chunks of a row are XOR-swizzled,
 // so that the 16 rows that a pass of the operand reads takes fall in distinct banks.
-// D = 64: two stages (48 KB), three workgroups per CU (156 VGPRs). D = 128: one (48 KB), two workgroups per CU by
+// D = 64: two stages (48 KB), three workgroups per CU (161 VGPRs). D = 128: one (48 KB), two workgroups per CU by
 // registers (256 VGPRs).
 template <int D>
 struct SplitTile {
@@ -150,7 +151,8 @@ __device__ __forceinline__ auto dyt_bound(const float* __restrict__ dyt) {
 }
 
 // Exponent of the leading bit of the largest magnitude `amax` (its bits) of operands scaled by a ScaleTable, at least
-// -100. An infinite one (gains or tables) must not cost the finite ones beside it their place: they are about 1 or less.
+// -100. An infinite one (gains or tables) must not cost the finite ones beside it their place: they are about 1 or
+// less.
 __device__ __forceinline__ int lead_exp(uint32_t amax) {
   const int e = static_cast<int>(amax >> 23) - 127;
   return e < -100 ? -100 : e > 127 ? 1 : e;
@@ -162,7 +164,8 @@ __device__ __forceinline__ uint32_t amax8(const float (&x)[8]) {
   return __float_as_uint(a);
 }
 
-// 8 values times 2^up, split, into a hi chunk and the lo chunk `plane` halves on; `edit(l)` may change the lo ones first.
+// 8 values times 2^up, split, into a hi chunk and the lo chunk `plane` halves on; `edit(l)` may change the lo ones
+// first.
 template <class Edit>
 __device__ __forceinline__ void st_split(uint16_t* __restrict__ hi, int plane, const float (&x)[8], int up, Edit edit) {
   float y[8];
@@ -201,8 +204,8 @@ struct MinU32 {
   __device__ uint32_t operator()(uint32_t a, uint32_t b) const { return a < b ? a : b; }
 };
 
-// The largest and smallest magnitudes of a V tile, as the bits of non-negative floats (which order as the floats do, with
-// infinities and then NaN last), collected in LDS by VTile::stats: of every key's row (over D / 64 waves), and the
+// The largest and smallest magnitudes of a V tile, as the bits of non-negative floats (which order as the floats do,
+// with infinities and then NaN last), collected in LDS by VTile::stats: of every key's row (over D / 64 waves), and the
 // smallest nonzero one of the 8-key pieces of dims.
 template <int D>
 struct VStats {
@@ -211,16 +214,16 @@ struct VStats {
 };
 
 // V of one key tile in registers: a lane per dim, so that a wave's loads are whole rows and the transpose costs no
-// shuffle. A tile is stored in one of two forms, told apart by the 8-bit code in it (v_code):
+// shuffle. A tile is stored in one of two forms, told apart by the 8-bit code in it (read_code):
 //   - split: v 2^-e as hi + lo halves, the largest in [2^11, 2^12); code e + 128. What a half cannot hold costs up to
 //     2^-37 of the tile's largest value, so a tile takes this form only if every key and every 8-key piece of a dim has
 //     a value of at least 2^-12 of it (keys past the sequence aside, which no query weighs, and zero pieces): the error
 //     is then at most 2^-25 of any key's and any dim's own largest. A tile of zeros is exact.
-//   - wide: the fp32 bits, upper and lower halves in the two planes, for the fp32 matrix cores; code 0. Tiles with a key
-//     of zeros among others are wide too: a query may give that key nearly all of its weight, and then needs its small
-//     probabilities to fp32 accuracy, which P's halves have only near the tile's largest.
-// The code lies in the first 8 lo values (dim 0, positions 0-7), at bit 14 of each: a lo half is at most 1 there (half a
-// unit of a hi below 2^12), so that bit is free in a split tile; in a wide one it changes places with bit 0, which is
+//   - wide: the fp32 bits, upper and lower halves in the two planes, for the fp32 matrix cores; code 0. Tiles with a
+//     key of zeros among others are wide too: a query may give that key nearly all of its weight, and then needs its
+//     small probabilities to fp32 accuracy, which P's halves have only near the tile's largest.
+// The code lies in the first 8 lo values (dim 0, positions 0-7), at bit 14 of each: a lo half is at most 1 there (half
+// a unit of a hi below 2^12), so that bit is free in a split tile; in a wide one it changes places with bit 0, which is
 // lost (those 8 values keep 23 bits).
 constexpr float kWideRange = 0x1p-12f;
 constexpr uint32_t kCodeBits = 0x40004000u;
@@ -380,10 +383,10 @@ struct Branch {
 // takes part for this lane's query.
 // The tile's probabilities are relative to its own largest logit (at most 1, and 1 somewhere), its products go into
 // accumulators of their own, and one factor per query then takes both to the state: so neither the halves of P nor the
-// power of two of V depends on what other tiles hold. That costs 16 FMAs per 32 dims: dense (2, 1292, 24 heads) 175 -> 187
-// us against products straight into O, and halves the error (6.2e-7 -> 3.3e-7); adding straight into O while a tile's
-// maximum and power of two are near the state's is 3 % faster and has neither that accuracy nor one path. The state is
-// rescaled only when some lane's maximum moves (it would multiply by exactly 1).
+// power of two of V depends on what other tiles hold. That costs 16 FMAs per 32 dims: dense (2, 1292, 24 heads) 175 ->
+// 187 us against products straight into O, and halves the error (6.2e-7 -> 3.3e-7); adding straight into O while a
+// tile's maximum and power of two are near the state's is 3 % faster and has neither that accuracy nor one path. The
+// state is rescaled only when some lane's maximum moves (it would multiply by exactly 1).
 template <int D, class Valid>
 __device__ __forceinline__ void attend_tile_f32(const uint16_t* __restrict__ sK, const uint16_t* __restrict__ sV,
                                                 const u32x4 (&q)[2][D / 16], Branch<D>& b, int n, bool masked,
@@ -526,12 +529,12 @@ __device__ __forceinline__ void store_diff_f32(uint16_t* __restrict__ stages, co
 }
 
 // The split forms of k and k_diff of ROWS keys (32-key tiles), a (row, RoPE group pair) per thread and pass as
-// rms_rows_f32 and band_rows_f32 hand them out: scaled by the ScaleTable as they come (`take`), then, when the workgroup
-// has found each tile's largest magnitude (`stats`, a barrier), by the tile's own power of two, so that the largest lies in
-// [2^11, 2^12) whatever the norms, the tables and the inputs made of it. What a half cannot hold is below 2^-37 of it.
-// The tile's code (its power of two + 128) lies in bit 14 of the first 8 lo values of key kCodeKey, which is free there
-// as in a split V tile. So do the powers of two of the dims (128 - k), for the calls that attend to keys which another
-// call prepared: bit r of dim d's in key r < 8 of the first tile of k (`scales` not null).
+// rms_rows_f32 and band_rows_f32 hand them out: scaled by the ScaleTable as they come (`take`), then, when the
+// workgroup has found each tile's largest magnitude (`stats`, a barrier), by the tile's own power of two, so that the
+// largest lies in [2^11, 2^12) whatever the norms, the tables and the inputs made of it. What a half cannot hold is
+// below 2^-37 of it. The tile's code (its power of two + 128) lies in bit 14 of the first 8 lo values of key kCodeKey,
+// which is free there as in a split V tile. So do the powers of two of the dims (128 - k), for the calls that attend to
+// keys which another call prepared: bit r of dim d's in key r < 8 of the first tile of k (`scales` not null).
 template <int D, int ROWS>
 struct KeyRows {
   using T = SplitTile<D>;
@@ -635,9 +638,9 @@ __device__ __forceinline__ void store_tiles(const KeyRows<D, 64>& keys, const Sc
 
 // RMSNorm (dit.py:45-57) and rotate-half RoPE (dit.py:90-98) in fp32 of two tensors (row offsets offA, offB) for the
 // ROWS positions from pos0 (of the batch whose rows start at `xb`): `sink(tensor, pass, row, group, values, group,
-// values)` takes the two 8-dim groups; positions at or past L give zeros. One (row, RoPE group pair) per thread and pass:
-// the rotation partner of every dim is in the thread's own registers; the mean of squares is reduced over the D / 16 lanes
-// of a row, neighbours in one wave.
+// values)` takes the two 8-dim groups; positions at or past L give zeros. One (row, RoPE group pair) per thread and
+// pass: the rotation partner of every dim is in the thread's own registers; the mean of squares is reduced over the D /
+// 16 lanes of a row, neighbours in one wave.
 template <int D, int ROWS, class Sink>
 __device__ __forceinline__ void rms_rows_f32(const float* __restrict__ xb, int64_t rs, int64_t offA, int64_t offB,
                                              int pos0, int L, int half, const float* __restrict__ w, float eps,
@@ -699,9 +702,9 @@ __device__ __forceinline__ void rms_rows_f32(const float* __restrict__ xb, int64
 }
 
 // The split q and q_diff of the workgroup's 64 queries, through LDS in passes of 64 rows (32 at head_dim 128):
-// `rows(r0, sink)` prepares the pass that starts at row r0. Besides the ScaleTable's, each row of each branch has a power
-// of two of its own, from its largest magnitude (then in [2^13, 2^14)). Returns the power of two of this lane's logits
-// but for the key tile's. Ends with a barrier, the stages free.
+// `rows(r0, sink)` prepares the pass that starts at row r0. Besides the ScaleTable's, each row of each branch has a
+// power of two of its own, from its largest magnitude (then in [2^13, 2^14)). Returns the power of two of this lane's
+// logits but for the key tile's. Ends with a barrier, the stages free.
 template <int D>
 constexpr int kQueryRows = 4096 / D;
 template <int D, class Rows>
@@ -850,10 +853,11 @@ __global__ __launch_bounds__(256, SplitTile<D>::OCC) void dense_attend_f32(
 }
 
 // tanh in fp32. Below 0.625: y + y^3 Q(y^2), Q a degree-5 least-maximum fit of (tanh(y)/y - 1)/y^2 (made for this
-// kernel; its fp32 coefficients are within 2^-28.5 of tanh before rounding). Above: 1 - 2 / (1 + 2^(2 log2(e) |y|)) with the rounding error of
-// the exponent carried into the exponential and one Newton step on the reciprocal; 2 / (1 + e) is below 0.45 there,
-// so the hardware exponential's error is at least halved. Both sides are computed and one is selected: 22
-// instructions without a branch, where the library's tanhf branches per element (both sides run in most waves).
+// kernel; its fp32 coefficients are within 2^-28.5 of tanh before rounding). Above: 1 - 2 / (1 + 2^(2 log2(e) |y|))
+// with the rounding error of the exponent carried into the exponential and one Newton step on the reciprocal; 2 / (1 +
+// e) is below 0.45 there, so the hardware exponential's error is at least halved. Both sides are computed and one is
+// selected: 22 instructions without a branch, where the library's tanhf branches per element (both sides run in most
+// waves).
 __device__ __forceinline__ float tanh_f32(float y) {
   const float z = __fmul_rn(y, y);
   float q = 0.0021429606713354588f;
@@ -900,10 +904,10 @@ struct DytPair {
 };
 
 // DyT (same_l.py:58-69) and RoPE (same_l.py:92-100) in fp32 of two tensors (row offsets offA, offB) for the ROWS
-// positions from pos0: `sink` as in rms_rows_f32; positions outside [0, S) give zeros. One (row, RoPE group pair) per thread and pass: the rotation partner of every dim is in the thread's own registers,
-// and the pass's 16-byte loads are all issued before its arithmetic. Measured at S = 16384, 8 heads of 64: the key
-// kernel 199.6 -> 42.0 us (201 MB at the rate of a large copy) against the library tanhf with the parameters read per
-// element.
+// positions from pos0: `sink` as in rms_rows_f32; positions outside [0, S) give zeros. One (row, RoPE group pair) per
+// thread and pass: the rotation partner of every dim is in the thread's own registers, and the pass's 16-byte loads are
+// all issued before its arithmetic. Measured at S = 16384, 8 heads of 64: the key kernel 199.6 -> 42.0 us (201 MB at
+// the rate of a large copy) against the library tanhf with the parameters read per element.
 template <int D, int ROWS, class Sink>
 __device__ __forceinline__ void band_rows_f32(const float* __restrict__ xb, int64_t rs, int64_t offA, int64_t offB,
                                               int pos0, int S, int half, const DytPair<D>& dp,
@@ -979,8 +983,9 @@ __global__ __launch_bounds__(256) void band_keys_f32(const float* __restrict__ q
 }
 
 // WS: the key tiles that meet the block's band come from the workspace of band_keys_f32; otherwise each query block
-// prepares its own from qkv, with one workgroup less per CU: the preparation's registers would spill (S = 16384, w = 128,
-// 8 x 64: 317 -> 286 us; 4 x 128, w = 300: 614 us spilling, 627 not).
+// prepares its own from qkv, with one workgroup less per CU, for the registers of the preparation: three at head_dim 64
+// spill 110 and take 322 us where two take 286 (S = 16384, w = 128, 8 x 64); two at 128 spill 223 and take 614 where one
+// takes 627 without (4 x 128, w = 300). With each key tile's own power of two found there: 314 and 676.
 template <int D, bool WS>
 __global__ __launch_bounds__(256, WS ? SplitTile<D>::OCC : SplitTile<D>::OCC - 1) void band_attend_f32(
     const float* __restrict__ qkv, int64_t rs, int B, int S, int Sp, int H, int w, const float* __restrict__ qdyt,

@@ -5,8 +5,8 @@
 // tile, which is what the B operand of S^T = K Q^T wants: lanes exchange only what the row's sum of squares needs,
 // and with one column tile per wave no row is prepared twice. A rotary pair (chunks c and c + half / 8) lies in one
 // lane whenever half is a multiple of 16; otherwise the partner chunk belongs to the other lane half and each lane
-// loads and normalises it a second time (B = 2, L = 2584, 4 x 64, one workgroup per CU: 52.1 us at half 24 against 48.5 at
-// 16; 49.6 at 24 when a lane held the whole row).
+// loads and normalises it a second time (B = 2, L = 2584, 4 x 64, one workgroup per CU: 52.1 us at half 24 against 48.5
+// at 16; 49.6 at 24 when a lane held the whole row).
 //
 // The prologue is bound by latency (nothing else runs on the SIMD yet), so every load of it is issued before the
 // first use. Before, each lane prepared a whole row and v_permlane32_swap redistributed it; with one column tile the
@@ -38,11 +38,11 @@ struct RmsQuery {
   }
   // 1 / rms of every row, in both lane halves. A row's squares are added in the order of its dims, as by a lane that
   // holds the whole row, so that a seed renders the same bits as with such lanes: the sum of the two halves' own sums
-  // rounds otherwise, which moves 2e-4 of an attention's results by one bf16 step and, over the 24 blocks of a denoiser,
-  // its output by 2e-2. Two rows are added by one lane half each, which gets the other's chunks (one chain of D additions
-  // for both); for a single row the sum goes from half to half. Against
-  // the halves' own sums: cross-attention B = 2, L = 2584 x 257, 24 x 64 33.4 -> 33.5 us, L = 8192 x 33 26.4 -> 27.5, 12 x
-  // 128 37.1 -> 37.7; self-attention B = 2, L = 1292, 12 x 128 97.6 -> 98.3, 24 x 64 unchanged.
+  // rounds otherwise, which moves 2e-4 of an attention's results by one bf16 step and, over the 24 blocks of a
+  // denoiser, its output by 2e-2. Two rows are added by one lane half each, which gets the other's chunks (one chain of
+  // D additions for both); for a single row the sum goes from half to half. Against the halves' own sums:
+  // cross-attention B = 2, L = 2584 x 257, 24 x 64 33.4 -> 33.5 us, L = 8192 x 33 26.4 -> 27.5, 12 x 128 37.1 -> 37.7;
+  // self-attention B = 2, L = 1292, 12 x 128 97.6 -> 98.3, 24 x 64 unchanged.
   template <int NCT>
   __device__ __forceinline__ void stats(const u32x4 (&raw)[NCT][1][D / 16], float (&st)[NCT][1]) const {
     static_assert(NCT == 1 || NCT == 2, "one row, or one per lane half");

@@ -17,11 +17,11 @@ namespace hb {
 __device__ __forceinline__ int v_tile_key(int pos) { return (pos & ~12) | ((pos & 4) << 1) | ((pos & 8) >> 1); }
 
 // Asynchronous 16-byte copy global -> LDS for a whole wave: lane i's 16 bytes at `sbase` + `voff` bytes
-// (`sbase` wave-uniform) land at byte 16 i of the 1 KB LDS block at byte address `lds` (wave-uniform). Issued as inline assembly
-// so that the compiler does not serialise it against the LDS reads of the other stage; the caller waits for it
-// (s_waitcnt vmcnt(0)) before the barrier that publishes the stage. The assembly writes M0 (the LDS address of
-// the copy); nothing else in these kernels reads M0, so the compiler's note that a reserved register in a
-// clobber list may not be preserved has no consumer here.
+// (`sbase` wave-uniform) land at byte 16 i of the 1 KB LDS block at byte address `lds` (wave-uniform). Issued as inline
+// assembly so that the compiler does not serialise it against the LDS reads of the other stage; the caller waits for it
+// (s_waitcnt vmcnt(0)) before the barrier that publishes the stage. The assembly writes M0 (the LDS address of the
+// copy); nothing else in these kernels reads M0, so the compiler's note that a reserved register in a clobber list may
+// not be preserved has no consumer here.
 __device__ __forceinline__ void lds_dma16(const void* sbase, uint32_t voff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(sbase) : "m0");
 }
@@ -107,7 +107,8 @@ struct TileCopy {
 // normalised other half (rounded per element) through LDS (`xbuf_mem`, free of tile reads: the caller has passed a
 // barrier after its last tile), 16 bytes per lane and access, and subtracts, in the same order in both, what it gets
 // back. Handing everything to the branch-1 waves left the others idle: the call at B = 1, L = 1422, 24 x 64
-// 46.1 -> 45.5 us, tiled band S = 16384, w = 256 104.3 -> 103.9. Other layouts: each wave holds both branches. Every lane of the workgroup must call it.
+// 46.1 -> 45.5 us, tiled band S = 16384, w = 256 104.3 -> 103.9. Other layouts: each wave holds both branches. Every
+// lane of the workgroup must call it.
 template <int D, int QB = 128, class IO = Bf16Io, int NW = 4>
 __device__ __forceinline__ void store_diff_split(
     uint16_t* __restrict__ out, int64_t b, int N, int H, int h, int q0w, int br0, float lamh,
