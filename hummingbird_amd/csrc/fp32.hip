@@ -221,7 +221,9 @@ struct VStats {
 //     is then at most 2^-25 of any key's and any dim's own largest. A tile of zeros is exact.
 //   - wide: the fp32 bits, upper and lower halves in the two planes, for the fp32 matrix cores; code 0. Tiles with a
 //     key of zeros among others are wide too: a query may give that key nearly all of its weight, and then needs its
-//     small probabilities to fp32 accuracy, which P's halves have only near the tile's largest.
+//     small probabilities to fp32 accuracy, which P's halves have only near the tile's largest. A call of wide tiles
+//     only (dense (2, 1292, 24 heads), every tenth key masked) takes 291 us against 180, and 527 with both products on
+//     the fp32 matrix cores.
 // The code lies in the first 8 lo values (dim 0, positions 0-7), at bit 14 of each: a lo half is at most 1 there (half
 // a unit of a hi below 2^12), so that bit is free in a split tile; in a wide one it changes places with bit 0, which is
 // lost (those 8 values keep 23 bits).
